@@ -51,6 +51,10 @@ struct orda_ctx {
     int64_t bytes = 0;
   };
   std::map<std::string, Buf> bufs;
+  bool planes_live = false;   // the three-plane buffers are in use by this call
+  // Fewest plane bytes a call ran out of memory with (0: none since the limit
+  // was set or the workspace trimmed): calls of as many do not try again.
+  int64_t planes_refused = 0;
   // Pinned host staging for small device-to-host reads (the labels, which
   // the host validates and counts): a copy into pageable memory costs
   // several times as long.
@@ -164,6 +168,20 @@ DType to_dtype(int32_t d, const char* what) {
 }
 
 // ------------------------------------------------------------ workspace
+void ws_release(orda_ctx* c, const std::string& name);
+
+// The buffers of the three-plane form (use_planes3): a call that runs short of
+// memory does without them, so they are given up before any other.
+void release_planes3(orda_ctx* c) {
+  for (const char* n : {"p3.w", "p3.tw", "p3.hs", "p3.th", "p3.grad"}) ws_release(c, n);
+}
+bool reclaim_planes3(orda_ctx* c) {
+  const int64_t before = c->held;
+  if (c->planes_live) return false;
+  release_planes3(c);
+  return c->held < before;
+}
+
 void* ws(orda_ctx* c, const std::string& name, int64_t bytes) {
   orda_ctx::Buf& b = c->bufs[name];
   if (bytes <= 0) return b.p;
@@ -174,11 +192,15 @@ void* ws(orda_ctx* c, const std::string& name, int64_t bytes) {
     b = orda_ctx::Buf{};
   }
   const int64_t rounded = (bytes + 255) / 256 * 256;
-  if (c->mem_limit > 0 && c->held + rounded > c->mem_limit)
+  if (c->mem_limit > 0 && c->held + rounded > c->mem_limit && !(reclaim_planes3(c) && c->held + rounded <= c->mem_limit))
     fail(ORDA_ERR_OOM, "workspace '%s' (%lld bytes) exceeds the context memory limit",
          name.c_str(), static_cast<long long>(rounded));
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, rounded);
+  if (e == hipErrorOutOfMemory && reclaim_planes3(c)) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, rounded);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
     if (e == hipErrorOutOfMemory)
@@ -450,6 +472,7 @@ struct LossPlan {
   DType dt;
   bool quant, stochastic;
   uint64_t seed;
+  bool planes3;             // fp32 products over three-plane operands (use_planes3)
   bool fast_math;           // approximate per-row logs and divisions
   bool online;              // one-pass row statistics (KernelConfig::online_softmax)
 };
@@ -523,6 +546,47 @@ bool teacher_logits_direct(const LossPlan& P, const Inputs& in) {
           in.tl.ld % 8 == 0 && in.tl.cols % 8 == 0 && reinterpret_cast<uintptr_t>(in.tl.p) % 16 == 0);
 }
 
+// Whether an fp32 call runs its products over three-plane operands
+// (GemmArgs::plane_a) instead of the fp32 MFMA: six bf16 products take the
+// place of one fp32 product, at 240 against 133 TFLOP/s of fp32 work, and the
+// gradients come out nearer to a float64 result (2.2e-6 against 3.2e-6 for
+// the hidden rows, 6.1e-7 against 9.8e-7 for the weights at BT=2048, H=4096,
+// V=32000). The planes are made by a pass over the weights and one over the
+// hidden rows, and K is padded to 64, so that calls of few operations do not
+// gain. The line lies at 2^34 operations: with planes for every product,
+// fp32 MFMA / planes in us per call, 3.2e9 operations (Tied 128 x 512 x 4096)
+// 155 / 183, 1.3e10 (Tied 256 x 512 x 8192) 223 / 226, 2.5e10 (Precomputed
+// 64 x 2048 x 32000) 740 / 614; as the products now go, 2.6e10 (Tied 2048 x
+// 256 x 4096) 353 / 316, 2.5e10 (Tied 16 x 4096 x 32000) 1955 / 1935, 3.2e12
+// (Tied 2048 x 4096 x 32000) 24.2 / 18.2 ms, 4.8e12 (Separate 4096 x (2048,
+// 4096) x 32000) 36.3 / 20.4 ms.
+bool use_planes3(const LossPlan& P) {
+  if (P.dt != orda::DType::F32 || P.h < 64 || P.v < 64) return false;
+  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
+  if (t_rows && P.ht < 64) return false;
+  const double width = 3.0 * P.h + (t_rows ? (P.w_t > 0.f ? 3.0 : 1.0) * P.ht : 0.0);
+  return 2.0 * P.bt * P.v * width >= 17179869184.0;
+}
+
+// Whether the logits products take planes too. A Tied teacher's stay on the
+// fp32 MFMA: each logit carries the rounding of its fp32 accumulation (1.5e-6
+// rms at H=4096), which the INT8 scales of grad_W's unlabelled rows show as up
+// to 1.2e-5 relative, and those are held to 1e-5 of an fp32 product's
+// (tests/test_gpu_full_size.py). Accumulated in the same order the two differ
+// by 5e-6; over planes, though nearer to float64, by 1.5e-5.
+bool planes3_logits(const LossPlan& P) {
+  return P.planes3 && !(P.need_teacher && P.mode == ORDA_TEACHER_TIED);
+}
+
+// Device bytes of the three-plane buffers of a call whose groups hold `cap`
+// rows: the weights, and the rows' share (as run_loss sizes them).
+int64_t planes3_bytes(const LossPlan& P, int64_t cap) {
+  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
+  const int64_t ph = round64(P.h), pt = t_rows ? round64(P.ht) : 0, pv = round64(P.v);
+  return 6 * (pv * (ph + (P.mode == ORDA_TEACHER_SEPARATE ? pt : 0)) +
+              cap * ((planes3_logits(P) ? ph + pt : 0) + (P.need_teacher ? 2 : 1) * pv));
+}
+
 // Device bytes the loss stages per chunk row: the buffers run_loss sizes by
 // the group's rows. (The split-K partials of small backward GEMMs are sized
 // by the GEMM, at most 256 MB, and come on top.)
@@ -535,6 +599,10 @@ int64_t staged_bytes_per_row(const LossPlan& P, const Inputs& in) {
   const int64_t ldl = logits_pitch(P.v, lt);
   int64_t b = blocks * ldl *
               (orda::dtype_size(lt) + (lt == P.dt ? 0 : orda::dtype_size(P.dt)));
+  // three-plane gradient rows and hidden rows (6 bytes an element)
+  if (P.planes3)
+    b += 6 * (blocks * round64(P.v) +
+              (planes3_logits(P) ? round64(P.h) + (in.th.p == nullptr ? 0 : round64(P.ht)) : 0));
   // the teacher's fp32 logits, and its bf16 gradient rows with teacher CE
   if (sep_epi) b += ldl * (P.w_t > 0.f ? 6 : 4);
   b += 2 * nst * 16 + 2 * 4;   // statistics, label logits
@@ -547,7 +615,7 @@ int64_t staged_bytes_per_row(const LossPlan& P, const Inputs& in) {
   // teacher and teacher CE; else the student's, then the Separate teacher's).
   b += (P.mode == ORDA_TEACHER_TIED && P.w_t > 0.f ? 2 * P.h
                                                    : std::max(P.h, P.has_gwt ? P.ht : int64_t{0})) *
-       orda::dtype_size(P.dt);
+       (P.planes3 ? 6 : orda::dtype_size(P.dt));
   return b;
 }
 
@@ -593,7 +661,27 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
   void* L = ws(c, "logits", blocks * cap * ldl * dtype_size(lt));
   void* TL = sep_epi ? ws(c, "tlogits", cap * ldl * 4) : nullptr;
   void* TG = sep_epi && P.w_t > 0.f ? ws(c, "tgrad", cap * ldl * es) : nullptr;
-  void* Gb = dt == lt ? L : ws(c, "dlogits", blocks * cap * ldl * es);
+  struct Live {
+    orda_ctx* c;
+    ~Live() { c->planes_live = false; }
+  } live{c};
+  c->planes_live = P.planes3;
+  // Three-plane operands: the weights once, the hidden rows and the gradient
+  // rows of a group; K (hidden width, V, rows) padded to whole 64s with zeros.
+  const bool p3 = P.planes3, p3_logits = planes3_logits(P);
+  const bool sep = P.mode == ORDA_TEACHER_SEPARATE;
+  const int64_t ph = round64(std::max<int64_t>(h, 1)), pt = sep ? round64(std::max<int64_t>(P.ht, 1)) : ph;
+  const int64_t pv = round64(v), vr = round64(v);
+  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
+  void* W3 = p3 ? ws(c, "p3.w", vr * 6 * ph) : nullptr;
+  void* TW3 = p3 && t_rows && sep ? ws(c, "p3.tw", vr * 6 * pt) : W3;
+  void* HS3 = p3_logits ? ws(c, "p3.hs", cap * 6 * ph) : nullptr;
+  void* TH3 = p3_logits && t_rows ? ws(c, "p3.th", cap * 6 * pt) : nullptr;
+  // gradient rows: the student's, then the teacher's (a Tied teacher's follow
+  // at once: one K of 2·rows for grad_W), each block padded to 64 rows
+  const int64_t g3rows = tied_tce ? round64(2 * cap) : blocks * round64(cap);
+  void* Gb = p3 ? ws(c, "p3.grad", g3rows * 6 * pv)
+                : dt == lt ? L : ws(c, "dlogits", blocks * cap * ldl * es);
   // Statistics and label logits of a whole group: student rows, then teacher
   // rows (the logits GEMM of problem p writes row p*M + r).
   float4* stats = static_cast<float4*>(ws(c, "stats", 2 * cap * nst * 16));
@@ -606,7 +694,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
   // The hidden rows of a group transposed ([width][rows], pitch ldh_cat):
   // the K-major A operand of grad_Wᵀ.
   const int64_t ldh_cat = round64(tied_tce ? 2 * cap : cap);   // rows on 128-byte lines
-  void* hcat = ws(c, "hcat", std::max(h, P.has_gwt ? P.ht : int64_t{0}) * ldh_cat * es);
+  void* hcat = ws(c, "hcat", std::max(h, P.has_gwt ? P.ht : int64_t{0}) * ldh_cat * (p3 ? 6 : es));
   float2* cross = paired || t_epi ? static_cast<float2*>(ws(c, "cross", cap * nst * 8)) : nullptr;
   // bf16 logits are stored relative to their half-tile maxima: per row
   // pair and 128-column half, the student's and the teacher's maximum side
@@ -638,6 +726,22 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
     if (P.has_ght) zero_out(in.ght, P.ht);
     hip_check(hipMemsetAsync(row3_out, 0, 3 * bt * 4, c->stream), "hipMemsetAsync");
   }
+  if (p3) {
+    timed(c, ORDA_KERNEL_OTHER, [&] {
+      const hipError_t e = launch_split3_rows(static_cast<const float*>(in.W.p), in.W.ld, v, h, W3, vr, ph, c->stream);
+      if (e != hipSuccess || TW3 == W3) return e;
+      return launch_split3_rows(static_cast<const float*>(in.tw.p), in.tw.ld, v, P.ht, TW3, vr, pt, c->stream);
+    });
+  }
+  // Operands of a product in three-plane form: A and B with their planes.
+  auto planes = [](GemmArgs& g, int64_t pa, int64_t pb, int64_t k) {
+    g.in_type = DType::BF16;
+    g.plane_a = pa;
+    g.plane_b = pb;
+    g.lda = 3 * pa;
+    g.ldb = 3 * pb;
+    g.K = round64(k);
+  };
   for (int64_t g0 = 0; v > 0 && g0 < nc; g0 += G) {
     const int64_t g1 = std::min(nc, g0 + G);
     const int64_t gs = g0 * cs;
@@ -647,7 +751,9 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
     void* Ls = L;
     void* Lt = sep_epi ? TL : at(L, btg * ldl, lt);
     void* Gs = Gb;
-    void* Gt = sep_epi ? TG : at(Gb, btg * ldl, dt);
+    void* Gt = sep_epi ? TG
+               : p3    ? at(Gb, (tied_tce ? btg : round64(btg)) * 3 * pv, DType::BF16)
+                       : at(Gb, btg * ldl, dt);
     const bool first = g0 == 0;
     const bool last = ge >= bt;
 
@@ -702,6 +808,18 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       f.lg.cross = cross;
     }
     f.group_m = 8;
+    if (p3_logits) {
+      timed(c, ORDA_KERNEL_OTHER, [&] {
+        const hipError_t e = launch_split3_rows(reinterpret_cast<const float*>(at(in.hs.p, gs * in.hs.ld, dt)),
+                                                in.hs.ld, btg, h, HS3, btg, ph, c->stream);
+        if (e != hipSuccess || !t_rows) return e;
+        return launch_split3_rows(reinterpret_cast<const float*>(at(in.th.p, gs * in.th.ld, dt)), in.th.ld,
+                                  btg, in.th.cols, TH3, btg, pt, c->stream);
+      });
+      planes(f, ph, ph, kh);
+      f.prob[0].a = HS3;
+      f.prob[0].b = W3;
+    }
     // fp32 logits of fp32 inputs, for a product with fewer output tiles than
     // CUs (small BT·V): stored plainly, on 128 x 128 tiles where the product
     // has at most 64 of 256 x 256 and/or with K split over the CUs
@@ -713,7 +831,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       GemmArgs sg = g;
       sg.epi = GemmEpilogue::StoreF32;
       sg.lg = LogitStatsArgs{};
-      if (lt != DType::F32 || g.in_type != DType::F32 || paired ||
+      if (lt != DType::F32 || dt != DType::F32 || paired ||
           (gemm_split_bytes(sg) <= 0 && !gemm_small_tiles(sg))) {
         timed(c, ORDA_KERNEL_GEMM_LOGITS, [&] { return launch_gemm(g, c->stream); });
         return false;
@@ -786,11 +904,15 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
     auto teacher_gemm = [&] {
       GemmArgs t = f;
       t.nprob = 1;
-      const bool sep = P.mode == ORDA_TEACHER_SEPARATE;
       t.K = sep ? std::max<int64_t>(P.ht, 1) : kh;
       t.lda = in.th.ld;
       t.ldb = sep ? in.tw.ld : in.W.ld;
       t.prob[0] = {at(in.th.p, gs * in.th.ld, dt), sep ? in.tw.p : in.W.p, Lt};
+      if (p3_logits) {
+        planes(t, pt, pt, t.K);
+        t.prob[0].a = TH3;
+        t.prob[0].b = TW3;
+      }
       t.lg.stats = stats + btg * nst;
       t.lg.xy = xy + btg;
       t.lg.hmax = hmax ? hmax + 1 : nullptr;   // the teacher side
@@ -838,8 +960,9 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       r.student = Ls;
       r.teacher = !P.need_teacher ? nullptr : tl_direct ? at(in.tl.p, gs * in.tl.ld, in.tl.t) : Lt;
       r.ld_t = tl_direct ? in.tl.ld : sep_epi ? ldl : 0;
-      r.grad_s = dt == lt ? nullptr : Gs;
-      r.grad_t = sep_epi || dt != lt ? Gt : nullptr;
+      r.grad_s = dt == lt && !p3 ? nullptr : Gs;
+      r.grad_t = sep_epi || dt != lt || p3 ? Gt : nullptr;
+      r.grad_plane = p3 ? pv : 0;
       r.gtype = dt;
       r.ld = ldl;
       r.n_rows = btg;
@@ -886,6 +1009,17 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       timed(c, ORDA_KERNEL_ROW_PASS, [&] { return launch_row_pass(r, c->stream); });
     }
 
+    if (p3) {
+      // rows up to grad_W's K: any finite values (the hidden planes are zero there)
+      auto pad_rows = [&](void* rows3, int64_t n) {
+        if (n % 64 != 0)
+          hip_check(hipMemsetAsync(at(rows3, n * 3 * pv, DType::BF16), 0, (round64(n) - n) * 6 * pv, c->stream),
+                    "hipMemsetAsync");
+      };
+      pad_rows(Gs, tied_tce ? 2 * btg : btg);
+      if (P.has_gwt) pad_rows(Gt, btg);
+    }
+
     // ---- grad_hidden = dlogits · W, scaled by the deferred mean (api.rs:347-366, 381-388)
     {
       GemmArgs d{};
@@ -910,16 +1044,23 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         d.nprob = 2;
         d.prob[1] = {Gt, in.W.p, in.ght.p + gs * in.ght.ld};
       }
+      if (p3) {
+        planes(d, pv, ph, v);
+        d.prob[0].b = d.prob[1].b = W3;
+      }
       attach_split_ws(c, d);
       timed(c, ORDA_KERNEL_GEMM_GRAD_HIDDEN, [&] { return launch_gemm(d, c->stream); });
       if (P.has_ght && !fuse) {
         GemmArgs t = d;
         t.nprob = 1;
-        const bool sep = P.mode == ORDA_TEACHER_SEPARATE;
         t.N = sep ? P.ht : h;
         t.ldb = sep ? in.tw.ld : in.W.ld;
         t.ldc = in.ght.ld;
         t.prob[0] = {Gt, sep ? in.tw.p : in.W.p, in.ght.p + gs * in.ght.ld};
+        if (p3) {
+          planes(t, pv, pt, v);
+          t.prob[0].b = TW3;
+        }
         attach_split_ws(c, t);
         timed(c, ORDA_KERNEL_GEMM_GRAD_HIDDEN, [&] { return launch_gemm(t, c->stream); });
       }
@@ -935,6 +1076,9 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
                            int64_t width, const void* D, float* C, int64_t ldc) {
       const int64_t k = hb != nullptr ? 2 * btg : btg;
       timed(c, ORDA_KERNEL_OTHER, [&] {
+        if (p3)
+          return launch_transpose_split3(static_cast<const float*>(ha), lda_h, static_cast<const float*>(hb),
+                                         ldb_h, btg, width, hcat, round64(k), c->stream);
         return launch_transpose_rows(ha, lda_h, hb, ldb_h, btg, width, hcat, ldh_cat, dt,
                                      c->stream);
       });
@@ -955,6 +1099,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       w.group_m = 8;
       w.nprob = 1;
       w.prob[0] = {hcat, D, C};
+      if (p3) planes(w, round64(k), pv, k);
       attach_split_ws(c, w);
       timed(c, ORDA_KERNEL_GEMM_GRAD_WEIGHT, [&] { return launch_gemm(w, c->stream); });
     };
@@ -1149,8 +1294,17 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
   // ---- chunk plan, staging group, OOM retry (resolver.rs:103-126)
   orda::ChunkPlan plan = plan0;
   const int64_t limit = o->config.has_max_chunks ? o->config.max_chunks : default_max_chunks_limit(bt);
-  const int64_t chunk_bytes = plan.chunk_size * staged_bytes_per_row(P, in);
-  int64_t G = std::max<int64_t>(1, std::min<int64_t>(plan.num_chunks, c->staging_budget / std::max<int64_t>(chunk_bytes, 1)));
+  P.planes3 = use_planes3(P);
+  auto group_of = [&] {
+    const int64_t chunk_bytes = plan.chunk_size * staged_bytes_per_row(P, in);
+    return std::max<int64_t>(1, std::min<int64_t>(plan.num_chunks, c->staging_budget / std::max<int64_t>(chunk_bytes, 1)));
+  };
+  int64_t G = group_of();
+  const int64_t planes_need = P.planes3 ? planes3_bytes(P, std::min(bt, G * plan.chunk_size)) : 0;
+  if (P.planes3 && c->planes_refused > 0 && planes_need >= c->planes_refused) {
+    P.planes3 = false;
+    G = group_of();
+  }
   for (;;) {
     try {
       run_loss(c, P, in, plan, G, row3, scal, &lstat->mean_scale);
@@ -1171,6 +1325,13 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
       ws_release(c, "tlogits");
       ws_release(c, "tgrad");
       ws_release(c, "splitk");
+      if (P.planes3) {   // plain fp32 operands need less: first without the planes
+        release_planes3(c);
+        c->planes_refused = c->planes_refused > 0 ? std::min(c->planes_refused, planes_need) : planes_need;
+        P.planes3 = false;
+        G = group_of();
+        continue;
+      }
       if (G > 1) {
         G /= 2;
         continue;
@@ -1558,6 +1719,7 @@ int32_t orda_ctx_set_stream(orda_ctx* c, void* s) {
 int32_t orda_ctx_set_memory_limit(orda_ctx* c, int64_t bytes) {
   if (!c || bytes < 0) return ORDA_ERR_INVALID;
   c->mem_limit = bytes;
+  c->planes_refused = 0;
   return ORDA_OK;
 }
 
@@ -1578,6 +1740,7 @@ int32_t orda_ctx_trim(orda_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   ws_trim(c);
+  c->planes_refused = 0;
   return ORDA_OK;
 }
 

@@ -57,6 +57,7 @@
 
 #include "kl_sums.h"
 #include "orda_kernels.h"
+#include "split3.h"
 
 namespace orda {
 namespace {
@@ -335,7 +336,6 @@ struct PairLoader {
       goff[t] = static_cast<uint32_t>((rr - b0) * ldb + q * 16);
     }
   }
-  __device__ __forceinline__ const unsigned char* src(int pair) const { return base + pair * step; }
 };
 
 // ---------------------------------------------------------------- fragments
@@ -517,6 +517,29 @@ __device__ __forceinline__ void mfma_step(f32x4 (&acc)[kFrag][kFrag], const u32x
   }
 }
 
+// fp32 products on the bf16 matrix units (GemmArgs::plane_a): each operand is
+// stored as three bf16 planes h + m + l (split3.h), which hold every bit of
+// an fp32 value, and a product of two such operands is the sum of the six
+// plane products hl, hm, hh, mm, mh, lh; the three left out (ml, lm, ll) lie
+// below 2^-26 of |a·b| each, under half an ulp of one fp32 product. The bf16
+// loops walk K in pairs of stages (64 elements): pair p is plane product p % 6
+// of K block p / 6.
+constexpr uint32_t kPlanesA = 0 << 0 | 0 << 2 | 0 << 4 | 1 << 6 | 1 << 8 | 2 << 10;
+constexpr uint32_t kPlanesB = 2 << 0 | 1 << 2 | 0 << 4 | 1 << 6 | 0 << 8 | 0 << 10;
+constexpr int kPlaneProducts = 6;
+
+// Source of stage pair `pair` of an operand whose pairs lie `step` bytes apart:
+// with three planes, plane (planes >> 2q) & 3 (`plane` elements apart) of K
+// block pair / 6, q = pair % 6.
+template <bool P3, uint32_t PLANES>
+__device__ __forceinline__ const unsigned char* pair_src(const unsigned char* base, int pair, int64_t step,
+                                                         int64_t plane) {
+  if constexpr (!P3) return base + pair * step;
+  const uint32_t kb = static_cast<uint32_t>(pair) / kPlaneProducts;
+  const uint32_t q = static_cast<uint32_t>(pair) - kb * kPlaneProducts;
+  return base + kb * step + static_cast<int64_t>((PLANES >> (2 * q)) & 3) * (2 * plane);
+}
+
 struct TileCoord {
   int p, m0, n0, ntile;
 };
@@ -579,8 +602,9 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-template <typename T, bool AK, bool BK, GemmEpilogue EPI, typename LT, bool CT>
+template <typename T, bool AK, bool BK, GemmEpilogue EPI, typename LT, bool CT, bool P3 = false>
 __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
+  static_assert(!P3 || Elem<T>::kSize == 2, "three-plane operands are bf16");
   // The logits epilogues: the product's own rows (Logits), or student rows
   // beside teacher logits read from memory (LogitsTeacher: fp32,
   // LogitsTeacher16: bf16).
@@ -713,7 +737,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       else
         pa.init(pr.a, g.lda, g.M, tc.m0, wave, lane);
       pb.init(pr.b, g.ldb, g.N, tc.n0, wave, lane);
-      const int np = nkf / 2;
+      const int np = P3 ? static_cast<int>(Kl / 64) * kPlaneProducts : nkf / 2;
+      auto src_a = [&](int pair) { return pair_src<P3, kPlanesA>(pa.base, pair, pa.step, g.plane_a); };
+      auto src_b = [&](int pair) { return pair_src<P3, kPlanesB>(pb.base, pair, pb.step, g.plane_b); };
       // Transfer x (0-7 A, 8-15 B) of a pair's DMA into double slot D, from
       // the pair's sources sa, sb.
       auto dma_op = [&](auto d_c, int x, uint64_t sa, uint64_t sb) {
@@ -740,12 +766,12 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       };
       if (np > 0) {
         {
-          const uint64_t sa = uniform64(pa.src(0)), sb = uniform64(pb.src(0));
+          const uint64_t sa = uniform64(src_a(0)), sb = uniform64(src_b(0));
   #pragma unroll
           for (int x = 0; x < 16; ++x) dma_op(SlotC<0>{}, x, sa, sb);
         }
         if (np > 1) {
-          const uint64_t sa = uniform64(pa.src(1)), sb = uniform64(pb.src(1));
+          const uint64_t sa = uniform64(src_a(1)), sb = uniform64(src_b(1));
   #pragma unroll
           for (int x = 0; x < 16; ++x) dma_op(SlotC<1>{}, x, sa, sb);
           __builtin_amdgcn_s_waitcnt(vm_wait(16));   // pair 0 landed
@@ -791,8 +817,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
             // overlaps MFMAs.
             const int p = (st >> 1) + 2;
             const int nxt = p < np ? p : np - 1;
-            sa = uniform64(pa.src(nxt));
-            sb = uniform64(pb.src(nxt));
+            sa = uniform64(src_a(nxt));
+            sb = uniform64(src_b(nxt));
           }
           if (!kOdd && pr == kMid) {
             __builtin_amdgcn_sched_barrier(0);
@@ -852,12 +878,20 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       // followed by exactly 16 (s even) or 4 (s odd) younger ones. Past the
       // last pair the DMAs re-read stage 0 (B) or the last pair (A) into
       // slots nobody reads again.
-      const int np = nkf / 2;
+      const int np = P3 ? static_cast<int>(Kl / 64) * kPlaneProducts : nkf / 2;
       const int ns = 2 * np;
       PairLoader<AK> pa;
       pa.init(pr.a, g.lda, g.M, tc.m0, wave, lane);
       LoaderB lb;
       init_b(lb);
+      auto src_a = [&](int pair) { return pair_src<P3, kPlanesA>(pa.base, pair, pa.step, g.plane_a); };
+      // B stage st: half st % 2 of pair st / 2's 64 K rows
+      auto src_b = [&](int st) {
+        if constexpr (!P3) return lb.stage_src(st);
+        else
+          return pair_src<true, kPlanesB>(lb.base, st >> 1, 64 * lb.ld_bytes, g.plane_b) +
+                 (st & 1) * 32 * lb.ld_bytes;
+      };
       // Transfer x (0-7) of an A pair into double slot D.
       auto dma_a = [&](auto d_c, int x, uint64_t sa) {
         constexpr int MA = decltype(d_c)::value * 2 * kOpBytes;
@@ -885,22 +919,22 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       if (np > 0) {
         // A pair 0, B stages 0-3, A pair 1; then stage 0 is followed by 20
         // younger transfers.
-        uint64_t sa = uniform64(pa.src(0));
+        uint64_t sa = uniform64(src_a(0));
 #pragma unroll
         for (int x = 0; x < 8; ++x) dma_a(SlotC<0>{}, x, sa);
-        uint64_t sb = uniform64(lb.stage_src(0));
+        uint64_t sb = uniform64(src_b(0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<0>{}, x, sb);
-        sb = uniform64(lb.stage_src(1 < ns ? 1 : 0));
+        sb = uniform64(src_b(1 < ns ? 1 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<1>{}, x, sb);
-        sb = uniform64(lb.stage_src(2 < ns ? 2 : 0));
+        sb = uniform64(src_b(2 < ns ? 2 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<2>{}, x, sb);
-        sb = uniform64(lb.stage_src(3 < ns ? 3 : 0));
+        sb = uniform64(src_b(3 < ns ? 3 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<3>{}, x, sb);
-        sa = uniform64(pa.src(np > 1 ? 1 : 0));
+        sa = uniform64(src_a(np > 1 ? 1 : 0));
 #pragma unroll
         for (int x = 0; x < 8; ++x) dma_a(SlotC<1>{}, x, sa);
         __builtin_amdgcn_s_waitcnt(vm_wait(20));
@@ -959,10 +993,10 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
             // DMA sources (B stage s+4, A pair s/2 + 2), computed behind the
             // first MFMAs.
             const int nb = st + kRing < ns ? st + kRing : 0;
-            sb = uniform64(lb.stage_src(nb));
+            sb = uniform64(src_b(nb));
             if constexpr (kOdd) {
               const int p = (st >> 1) + 2;
-              sa = uniform64(pa.src(p < np ? p : np - 1));
+              sa = uniform64(src_a(p < np ? p : np - 1));
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -985,6 +1019,14 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
     }
     __builtin_amdgcn_sched_barrier(0);
     mfma_drain();
+    if constexpr (P3) {
+      // With no tail stage after the loop the compiler would copy the store
+      // epilogues' accumulators out at the loop's exit, ahead of the drain.
+#pragma unroll
+      for (int i = 0; i < kFrag; ++i)
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) asm volatile("" : "+a"(acc[i][j]));
+    }
     __builtin_amdgcn_sched_barrier(0);
   } else {
     // fp32: an MFMA stage is long (256 v_mfma_f32_16x16x4_f32), so one
@@ -1016,7 +1058,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
     }
     st_done = nkf;
   }
-  if (static_cast<int64_t>(st_done) * SK < Kl) {
+  // (three-plane operands are padded to whole pairs: nothing left)
+  if (!P3 && static_cast<int64_t>(st_done) * SK < Kl) {
     // Stages the main loop left — after the bf16 pairs an odd full stage,
     // and a partial last stage — one at a time through slot 0 in the
     // single-stage layout: DMA the valid part, zero the rest.
@@ -1635,12 +1678,32 @@ ORDA_GEMM(gemm_kmt_accum_f32, float, true, false, GemmEpilogue::AccumF32, float,
 // statistics then come from a separate pass over the stored logits).
 ORDA_GEMM(gemm_kk_store_f32, float, true, true, GemmEpilogue::StoreF32, float, false)
 #undef ORDA_GEMM
+// The fp32 products over three-plane operands.
+#define ORDA_GEMM3(NAME, BK, EPI, CT) \
+  __global__ __launch_bounds__(kThreads, 1) void NAME(GemmArgs g) { gemm_body<__bf16, true, BK, EPI, float, CT, true>(g); }
+ORDA_GEMM3(gemm_kk_logits_bf16x3_f32, true, GemmEpilogue::Logits, false)
+ORDA_GEMM3(gemm_kk_store_bf16x3, true, GemmEpilogue::StoreF32, false)
+ORDA_GEMM3(gemm_km_store_bf16x3, false, GemmEpilogue::StoreF32, false)
+ORDA_GEMM3(gemm_kmt_store_bf16x3, false, GemmEpilogue::StoreF32, true)
+ORDA_GEMM3(gemm_kmt_accum_bf16x3, false, GemmEpilogue::AccumF32, true)
+#undef ORDA_GEMM3
 
 typedef void (*GemmKernel)(GemmArgs);
 
 GemmKernel select_kernel(const GemmArgs& g) {
   using E = GemmEpilogue;
   const bool bf = g.in_type == DType::BF16;
+  if (g.plane_a > 0) {
+    if (!bf || !g.a_kmajor) return nullptr;
+    if (g.epi == E::Logits)
+      return g.b_kmajor && !g.c_trans && g.logits_type == DType::F32 && g.lg.pair_rows == 0 &&
+                     g.lg.teacher_logits == nullptr
+                 ? gemm_kk_logits_bf16x3_f32
+                 : nullptr;
+    if (g.b_kmajor) return g.epi == E::StoreF32 && !g.c_trans ? gemm_kk_store_bf16x3 : nullptr;
+    if (g.c_trans) return g.epi == E::StoreF32 ? gemm_kmt_store_bf16x3 : gemm_kmt_accum_bf16x3;
+    return g.epi == E::StoreF32 ? gemm_km_store_bf16x3 : nullptr;
+  }
   if (g.epi == E::Logits) {
     if (!g.a_kmajor || !g.b_kmajor || g.c_trans) return nullptr;
     if (g.lg.teacher_logits != nullptr) {
@@ -1758,6 +1821,55 @@ __global__ __launch_bounds__(256) void transpose_rows_kernel(const E* a, int64_t
   }
 }
 
+// fp32 rows transposed into three-plane rows (launch_transpose_split3), the
+// same 64 x 64 blocks through LDS; a thread writes 8 consecutive r of one
+// column as one 16-byte segment of each plane.
+template <bool VEC>
+__global__ __launch_bounds__(256) void transpose_split3_kernel(const float* a, int64_t lda,
+                                                               const float* b, int64_t ldb,
+                                                               int64_t rows, int64_t cols,
+                                                               __bf16* dst, int64_t plane) {
+  constexpr int kT = 64;
+  __shared__ float tile[kT][kT + 1];   // the 8 rows x 8 columns a wave reads: 64 banks
+  const int64_t krows = b != nullptr ? 2 * rows : rows;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kT;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kT;
+  const int tid = threadIdx.x;
+  for (int q = tid; q < kT * kT / 4; q += 256) {
+    const int rl = q / (kT / 4), cl = q % (kT / 4) * 4;
+    const int64_t r = r0 + rl, c = c0 + cl;
+    const float* src = nullptr;
+    if (r < krows) src = (r < rows ? a + r * lda : b + (r - rows) * ldb) + c;
+    f32x4 w = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+      if (src != nullptr && c < cols) w = *reinterpret_cast<const f32x4*>(src);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (src != nullptr && c + k < cols) w[k] = src[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tile[rl][cl + k] = w[k];
+  }
+  __syncthreads();
+  for (int q = tid; q < kT * (kT / 8); q += 256) {
+    const int cl = q / (kT / 8), sg = q % (kT / 8);
+    const int64_t c = c0 + cl;
+    if (c >= cols) continue;
+    u32x4 w[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t p[3];
+      split3_pack(tile[sg * 8 + 2 * i][cl], tile[sg * 8 + 2 * i + 1][cl], p);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) w[k][i] = p[k];
+    }
+    __bf16* d = dst + 3 * c * plane + r0 + sg * 8;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(d + k * plane) = w[k];
+  }
+}
+
 struct SplitPlan {
   int splits;
   int64_t len, ldp, stride, bytes;
@@ -1819,7 +1931,7 @@ void set_band_blocks(GemmArgs& g) {
   if (g.sh_a > 0 || g.epi != GemmEpilogue::Logits || g.in_type != DType::BF16) return;
   const int64_t Mv = ((g.M + kTile - 1) / kTile) * g.nprob;
   const int64_t Nt = (g.N + kTile - 1) / kTile;
-  const int64_t strip = int64_t{kTile} * g.K * 2;
+  const int64_t strip = int64_t{kTile} * g.K * (g.plane_a > 0 ? 6 : 2);
   const int64_t gm = g.group_m > 0 ? g.group_m : 1;
   const int64_t live = (Mv < 8 * gm ? Mv : 8 * gm) * strip;
   if (live <= kBandLive || 32 * strip > kBandMax || Mv < 32) return;
@@ -2192,6 +2304,25 @@ hipError_t launch_transpose_rows(const void* a, int64_t lda, const void* b, int6
   return hipGetLastError();
 }
 
+hipError_t launch_transpose_split3(const float* a, int64_t lda, const float* b, int64_t ldb,
+                                   int64_t rows, int64_t cols, void* dst, int64_t plane,
+                                   hipStream_t stream) {
+  const int64_t krows = b != nullptr ? 2 * rows : rows;
+  if (rows < 0 || cols < 0 || plane < krows || plane % 64 || reinterpret_cast<uintptr_t>(dst) % 16)
+    return hipErrorInvalidValue;
+  if (rows == 0 || cols == 0) return hipSuccess;
+  const dim3 grid(static_cast<unsigned>(plane / 64), static_cast<unsigned>((cols + 63) / 64));
+  const bool vec = lda % 4 == 0 && (b == nullptr || ldb % 4 == 0) && cols % 4 == 0 &&
+                   reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+  if (vec)
+    hipLaunchKernelGGL(transpose_split3_kernel<true>, grid, dim3(256), 0, stream, a, lda, b, ldb,
+                       rows, cols, static_cast<__bf16*>(dst), plane);
+  else
+    hipLaunchKernelGGL(transpose_split3_kernel<false>, grid, dim3(256), 0, stream, a, lda, b, ldb,
+                       rows, cols, static_cast<__bf16*>(dst), plane);
+  return hipGetLastError();
+}
+
 namespace {
 
 // The part of g over columns [c0, c1) and rows [r0, r1) of C (operands and
@@ -2298,6 +2429,9 @@ hipError_t launch_gemm_impl(const GemmArgs& g, hipStream_t stream, bool whole) {
     return hipErrorInvalidValue;
   if (g.epi == GemmEpilogue::Logits && g.logits_type == DType::BF16 &&
       (g.lg.hmax == nullptr || g.lg.hmax_ld % 2 || g.lg.hmax_ld < 4 * ((g.N + kTile - 1) / kTile)))
+    return hipErrorInvalidValue;
+  if ((g.plane_a > 0) != (g.plane_b > 0) ||
+      (g.plane_a > 0 && (g.K % 64 || g.plane_a % 8 || g.plane_b % 8)))
     return hipErrorInvalidValue;
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
   if (whole && small_f32(g)) return launch_small(g, stream);

@@ -104,6 +104,11 @@ struct GemmArgs {
   // Set by launch_gemm when share_rounds applies: each XCD takes an
   // sh_a (M) x sh_b (N) block of a round, sh_xn XCDs side by side in N.
   int sh_a, sh_b, sh_xn;
+  // Three-plane operands (fp32 values as bf16 planes h + m + l, split3.h):
+  // in_type BF16, the planes of A plane_a elements apart and those of B
+  // plane_b apart, inside the pitches lda / ldb; K a multiple of 64, both
+  // operands zero from the true K on. 0: plain operands.
+  int64_t plane_a, plane_b;
   // Store/Accum only: C is stored transposed, element (m, n) of the
   // product at C[n*ldc + m] (C is [N][ldc]).
   bool c_trans;
@@ -140,6 +145,12 @@ GemmSplit gemm_split_plan(const GemmArgs& g);
 hipError_t launch_transpose_rows(const void* a, int64_t lda, const void* b, int64_t ldb,
                                  int64_t rows, int64_t cols, void* dst, int64_t ldd, DType t,
                                  hipStream_t stream);
+// The same for fp32 rows into three-plane rows (GemmArgs::plane_a): column c
+// of the sources becomes row c, its planes of plane elements at
+// dst + c*3*plane; plane >= rows (2*rows), a multiple of 64, zeros past them.
+hipError_t launch_transpose_split3(const float* a, int64_t lda, const float* b, int64_t ldb,
+                                   int64_t rows, int64_t cols, void* dst, int64_t plane,
+                                   hipStream_t stream);
 // Workspace bytes launch_gemm uses to split K for this GEMM (0: no split).
 int64_t gemm_split_bytes(const GemmArgs& g);
 // Whether launch_gemm runs this Store/Accum GEMM on 128 x 128 tiles (fp32
@@ -202,6 +213,10 @@ struct RowPassArgs {
   void* grad_s;
   void* grad_t;
   DType gtype;
+  // > 0: fp32 gradients as three-plane rows (GemmArgs::plane_a), row r's
+  // planes of grad_plane elements (>= v, a multiple of 64, at most the
+  // student pitch ld) at grad_s/grad_t + r*3*grad_plane, zeros past v.
+  int64_t grad_plane;
   // Split mode (chunk-launcher entry point): gradients go to separate
   // buffers instead of overwriting the logits, and are not merged.
   bool split;
@@ -323,5 +338,11 @@ hipError_t launch_mark_targets(const int64_t* labels, int64_t n, int64_t ignore_
 hipError_t launch_convert_rows(DType src_t, const void* src, int64_t lds, DType dst_t,
                                void* dst, int64_t ldd, int64_t rows, int64_t cols,
                                hipStream_t stream);
+
+// fp32 rows as three-plane rows (GemmArgs::plane_a): row r's planes of
+// `plane` elements at dst + r*3*plane, zeros from column cols and, up to
+// rows_pad, from row rows on.
+hipError_t launch_split3_rows(const float* src, int64_t lds, int64_t rows, int64_t cols, void* dst,
+                              int64_t rows_pad, int64_t plane, hipStream_t stream);
 
 }  // namespace orda

@@ -14,6 +14,7 @@
 #include <math.h>
 
 #include "orda_kernels.h"
+#include "split3.h"
 
 namespace orda {
 namespace {
@@ -280,6 +281,45 @@ __global__ __launch_bounds__(256) void convert_rows_kernel(const S* src, int64_t
   }
 }
 
+// fp32 rows as three bf16 planes (split3.h): row r's planes at dst + r*3*plane,
+// each plane elements long, zeros from column `cols` and from row `rows` on.
+// One workgroup per (row, 2048 columns), eight columns a thread: two 16-byte
+// loads (single elements where the row does not allow them or ends), three
+// 16-byte stores. Bound by HBM.
+__global__ __launch_bounds__(256) void split3_rows_kernel(const float* src, int64_t lds, __bf16* dst,
+                                                          int64_t plane, int64_t rows, int64_t cols,
+                                                          int64_t cpr) {
+  const int64_t r = blockIdx.x / cpr;
+  const int64_t c0 = (blockIdx.x - r * cpr) * kConvCols + threadIdx.x * 8;
+  if (c0 >= plane) return;
+  const float* s = src + r * lds + c0;
+  float x[8];
+  if (r < rows && c0 + 8 <= cols && reinterpret_cast<uintptr_t>(s) % 16 == 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 w = reinterpret_cast<const f32x4*>(s)[h];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[4 * h + i] = w[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = r < rows && c0 + i < cols ? s[i] : 0.f;
+  }
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  u4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t p[3];
+    split3_pack(x[2 * i], x[2 * i + 1], p);
+    w[0][i] = p[0];
+    w[1][i] = p[1];
+    w[2][i] = p[2];
+  }
+  __bf16* d = dst + 3 * r * plane + c0;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<u4*>(d + q * plane) = w[q];
+}
+
 unsigned grid_for(int64_t total) {
   int64_t b = (total + 255) / 256;
   if (b > 65536) b = 65536;
@@ -348,6 +388,18 @@ hipError_t launch_convert_rows(DType st, const void* src, int64_t lds, DType dt,
   else
     hipLaunchKernelGGL((convert_rows_kernel<__bf16, __bf16>), g, b, 0, s,
                        static_cast<const __bf16*>(src), lds, static_cast<__bf16*>(dst), ldd, cols, cpr);
+  return hipGetLastError();
+}
+
+hipError_t launch_split3_rows(const float* src, int64_t lds, int64_t rows, int64_t cols, void* dst,
+                              int64_t rows_pad, int64_t plane, hipStream_t s) {
+  if (rows_pad <= 0 || plane <= 0) return hipSuccess;
+  if (rows > rows_pad || cols > plane || plane % 8 != 0 || reinterpret_cast<uintptr_t>(dst) % 16 != 0)
+    return hipErrorInvalidValue;
+  const int64_t cpr = (plane + kConvCols - 1) / kConvCols;
+  if (rows_pad * cpr > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(split3_rows_kernel, dim3(static_cast<unsigned>(rows_pad * cpr)), dim3(256), 0, s,
+                     src, lds, static_cast<__bf16*>(dst), plane, rows, cols, cpr);
   return hipGetLastError();
 }
 

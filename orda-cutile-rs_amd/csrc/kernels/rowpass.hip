@@ -28,8 +28,11 @@
 // folded into one FMA per element.
 #include <math.h>
 
+#include <type_traits>
+
 #include "kl_sums.h"
 #include "orda_kernels.h"
+#include "split3.h"
 
 namespace orda {
 namespace {
@@ -378,8 +381,7 @@ __global__ __launch_bounds__(TPB) void row_pass_kernel(RowPassArgs a) {
   }
 }
 
-// Eight consecutive logits (16-byte aligned) as fp32, and eight gradients
-// back in the storage type.
+// Eight consecutive logits (16-byte aligned) as fp32.
 template <typename T>
 __device__ __forceinline__ void load8(const T* p, float (&x)[8]);
 template <>
@@ -395,22 +397,92 @@ template <>
 __device__ __forceinline__ void load8(const __bf16* p, float (&x)[8]) {
   Vec<__bf16>::unpack(*reinterpret_cast<const u32x4*>(p), x);
 }
-template <typename T>
-__device__ __forceinline__ void store8(T* p, const float (&g)[8]);
-template <>
-__device__ __forceinline__ void store8(float* p, const float (&g)[8]) {
-  reinterpret_cast<u32x4*>(p)[0] = u32x4{__float_as_uint(g[0]), __float_as_uint(g[1]),
-                                         __float_as_uint(g[2]), __float_as_uint(g[3])};
-  reinterpret_cast<u32x4*>(p)[1] = u32x4{__float_as_uint(g[4]), __float_as_uint(g[5]),
-                                         __float_as_uint(g[6]), __float_as_uint(g[7])};
-}
-template <>
-__device__ __forceinline__ void store8(__bf16* p, const float (&g)[8]) {
-  *reinterpret_cast<u32x4*>(p) = Vec<__bf16>::pack(g);
-}
 // Streaming forms for data touched once (non-temporal hint on the access).
 __device__ __forceinline__ void store8_nt(__bf16* p, const float (&g)[8]) {
   __builtin_nontemporal_store(Vec<__bf16>::pack(g), reinterpret_cast<u32x4*>(p));
+}
+
+// N gradient values to p (aligned to their size), as fp32 or packed bf16.
+template <bool NT, int N>
+__device__ __forceinline__ void store_vec(float* p, const float (&g)[N]) {
+#pragma unroll
+  for (int h = 0; h < N / 4; ++h) {
+    const u32x4 w = u32x4{__float_as_uint(g[4 * h]), __float_as_uint(g[4 * h + 1]),
+                          __float_as_uint(g[4 * h + 2]), __float_as_uint(g[4 * h + 3])};
+    if (NT) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p) + h);
+    else reinterpret_cast<u32x4*>(p)[h] = w;
+  }
+}
+template <bool NT, int N>
+__device__ __forceinline__ void store_vec(__bf16* p, const float (&g)[N]) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  uint32_t w[N / 2];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i)
+    w[i] = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(g[2 * i]),
+                                               static_cast<__bf16>(g[2 * i + 1])});
+  if constexpr (N == 8) {
+    const u32x4 v = u32x4{w[0], w[1], w[2], w[3]};
+    if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+    else *reinterpret_cast<u32x4*>(p) = v;
+  } else {
+    static_assert(N == 4, "4 or 8 values");
+    const u32x2 v = u32x2{w[0], w[1]};
+    if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(p));
+    else *reinterpret_cast<u32x2*>(p) = v;
+  }
+}
+// A gradient row: N values at column j (whole vectors), or one value. GT
+// float or __bf16: a plain row; Planes3: an fp32 row as three bf16 planes
+// (RowPassArgs::grad_plane), which the GEMMs over three-plane operands read.
+struct Planes3 {};
+template <typename GT>
+struct GradRow {
+  GT* p;
+  __device__ GradRow(const RowPassArgs& a, void* base, int64_t r) : p(static_cast<GT*>(base) + r * a.ld) {}
+  template <bool NT, int N>
+  __device__ __forceinline__ void store(int64_t j, const float (&g)[N]) const;
+  __device__ __forceinline__ void set(int64_t j, float g) const { p[j] = static_cast<GT>(g); }
+};
+template <>
+struct GradRow<Planes3> {
+  __bf16* p;
+  int64_t plane;
+  __device__ GradRow(const RowPassArgs& a, void* base, int64_t r)
+      : p(static_cast<__bf16*>(base) + 3 * r * a.grad_plane), plane(a.grad_plane) {}
+  template <bool NT, int N>
+  __device__ __forceinline__ void store(int64_t j, const float (&g)[N]) const;
+  __device__ __forceinline__ void set(int64_t j, float g) const {
+    float h, m, l;
+    split3(g, h, m, l);
+    p[j] = static_cast<__bf16>(h);
+    p[plane + j] = static_cast<__bf16>(m);
+    p[2 * plane + j] = static_cast<__bf16>(l);
+  }
+};
+
+template <typename GT>
+template <bool NT, int N>
+__device__ __forceinline__ void GradRow<GT>::store(int64_t j, const float (&g)[N]) const {
+  store_vec<NT>(p + j, g);
+}
+template <bool NT, int N>
+__device__ __forceinline__ void GradRow<Planes3>::store(int64_t j, const float (&g)[N]) const {
+  typedef uint32_t uv __attribute__((ext_vector_type(N / 2)));
+  uv w[3];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    uint32_t q[3];
+    split3_pack(g[2 * i], g[2 * i + 1], q);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) w[k][i] = q[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    uv* d = reinterpret_cast<uv*>(p + k * plane + j);
+    if (NT) __builtin_nontemporal_store(w[k], d);
+    else *d = w[k];
+  }
 }
 
 // The half-tile maxima of one row pair (RowPassArgs::hmax_s / hmax_t), or
@@ -458,16 +530,23 @@ __global__ __launch_bounds__(kThreads) void row_pass_fused_kernel(RowPassArgs a)
   const int nfull = static_cast<int>(v / NV);
   const LT* srow = static_cast<const LT*>(a.student) + r * a.ld;
   const LT* trow = HT ? static_cast<const LT*>(a.teacher) + r * (a.ld_t ? a.ld_t : a.ld) : nullptr;
-  GT* gsrow = static_cast<GT*>(a.grad_s ? a.grad_s : a.student) + r * a.ld;
-  GT* gtrow = TG ? static_cast<GT*>(a.grad_s ? a.grad_t : a.teacher) + r * a.ld : nullptr;
+  const GradRow<GT> gsrow(a, a.grad_s ? a.grad_s : a.student, r);
+  const GradRow<GT> gtrow(a, a.grad_s ? a.grad_t : a.teacher, r);   // TG only
+  if constexpr (std::is_same<GT, Planes3>::value) {   // zeros past the row's last vector
+    const float z[NV] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int64_t j = static_cast<int64_t>(nvec + tid) * NV; j < a.grad_plane; j += kThreads * NV) {
+      gsrow.template store<false>(j, z);
+      if (TG) gtrow.template store<false>(j, z);
+    }
+  }
 
   // cross_entropy.rs:59, kl.rs:92: zero gradient and losses (also for a
   // label outside [0, V), which the host reports as an error).
   if (y == a.ignore_index || y < 0 || y >= v) {
     const float z[NV] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int vi = tid; vi < nvec; vi += kThreads) {
-      store8(gsrow + static_cast<int64_t>(vi) * NV, z);
-      if (TG) store8(gtrow + static_cast<int64_t>(vi) * NV, z);
+      gsrow.template store<false>(static_cast<int64_t>(vi) * NV, z);
+      if (TG) gtrow.template store<false>(static_cast<int64_t>(vi) * NV, z);
     }
     if (tid == 0) {
       a.row_nll_s[r] = 0.f;
@@ -561,8 +640,8 @@ __global__ __launch_bounds__(kThreads) void row_pass_fused_kernel(RowPassArgs a)
       g[i] = valid ? gi : 0.f;
       gt[i] = valid ? ti : 0.f;
     }
-    store8(gsrow + j0, g);
-    if (TG) store8(gtrow + j0, gt);
+    gsrow.template store<false>(j0, g);
+    if (TG) gtrow.template store<false>(j0, gt);
   };
   // The label column's logits, read by its owner before the row is
   // overwritten (the gradient may go in place).
@@ -626,8 +705,8 @@ __global__ __launch_bounds__(kThreads) void row_pass_fused_kernel(RowPassArgs a)
   if (owner) {
     float gy = 0.f, ty = 0.f, cx = 0.f, c = 0.f, d = 0.f;
     elem(xs_y, xt_y, offs(hr.s(y), hr.t(y)), gy, ty, cx, c, d);
-    gsrow[y] = static_cast<GT>(gy - ky);
-    if (TG) gtrow[y] = static_cast<GT>(ty - kyt);
+    gsrow.set(y, gy - ky);
+    if (TG) gtrow.set(y, ty - kyt);
   }
 
   if (KL && a.cross == nullptr) {
@@ -966,36 +1045,6 @@ constexpr int kF32Vec = 1;                                 // NV-element vectors
 constexpr int kF32NV = 4;
 constexpr bool kF32Nt = true;
 constexpr int kF32Chunk = kF32Threads * kF32NV * kF32Vec;  // columns per workgroup
-// N gradient values to p (aligned to their size), as fp32 or packed bf16.
-template <bool NT, int N>
-__device__ __forceinline__ void store_vec(float* p, const float (&g)[N]) {
-#pragma unroll
-  for (int h = 0; h < N / 4; ++h) {
-    const u32x4 w = u32x4{__float_as_uint(g[4 * h]), __float_as_uint(g[4 * h + 1]),
-                          __float_as_uint(g[4 * h + 2]), __float_as_uint(g[4 * h + 3])};
-    if (NT) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p) + h);
-    else reinterpret_cast<u32x4*>(p)[h] = w;
-  }
-}
-template <bool NT, int N>
-__device__ __forceinline__ void store_vec(__bf16* p, const float (&g)[N]) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  uint32_t w[N / 2];
-#pragma unroll
-  for (int i = 0; i < N / 2; ++i)
-    w[i] = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(g[2 * i]),
-                                               static_cast<__bf16>(g[2 * i + 1])});
-  if constexpr (N == 8) {
-    const u32x4 v = u32x4{w[0], w[1], w[2], w[3]};
-    if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = v;
-  } else {
-    static_assert(N == 4, "4 or 8 values");
-    const u32x2 v = u32x2{w[0], w[1]};
-    if (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(p));
-    else *reinterpret_cast<u32x2*>(p) = v;
-  }
-}
 template <bool NT>
 __device__ __forceinline__ u32x4 load_vec(const float* p) {
   if (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
@@ -1015,8 +1064,10 @@ __global__ __launch_bounds__(kF32Threads) void row_grad_f32_kernel(RowPassArgs a
   const float* srow = static_cast<const float*>(a.student) + r * a.ld;
   const float* trow =
       (KL || TG) ? static_cast<const float*>(a.teacher) + r * (a.ld_t ? a.ld_t : a.ld) : nullptr;
-  GT* gsrow = static_cast<GT*>(a.grad_s ? a.grad_s : a.student) + r * a.ld;
-  GT* gtrow = TG ? static_cast<GT*>(a.grad_s ? a.grad_t : a.teacher) + r * a.ld : nullptr;
+  const GradRow<GT> gsrow(a, a.grad_s ? a.grad_s : a.student, r);
+  const GradRow<GT> gtrow(a, a.grad_s ? a.grad_t : a.teacher, r);   // TG only
+  // columns written: three-plane rows get zeros up to their planes' end
+  const int64_t jend = std::is_same<GT, Planes3>::value ? a.grad_plane : v;
   auto col = [&](int q) { return c0 + (static_cast<int64_t>(q) * kF32Threads + tid) * NV; };
   if (y == a.ignore_index || y < 0 || y >= v) {   // zero gradient rows, no KL
     float z[NV];
@@ -1025,9 +1076,9 @@ __global__ __launch_bounds__(kF32Threads) void row_grad_f32_kernel(RowPassArgs a
 #pragma unroll
     for (int q = 0; q < kF32Vec; ++q) {
       const int64_t j = col(q);
-      if (j < v) {
-        store_vec<kF32Nt>(gsrow + j, z);
-        if (TG) store_vec<kF32Nt>(gtrow + j, z);
+      if (j < jend) {
+        gsrow.template store<kF32Nt>(j, z);
+        if (TG) gtrow.template store<kF32Nt>(j, z);
       }
     }
     if (KL && tid == 0) a.kl_part[r * chunks + ci] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1058,7 +1109,7 @@ __global__ __launch_bounds__(kF32Threads) void row_grad_f32_kernel(RowPassArgs a
     xs_y = srow[y];
     if (KL || TG) xt_y = trow[y];
   }
-  u32x4 rs[kF32Vec][NH], rt[kF32Vec][NH];
+  u32x4 rs[kF32Vec][NH] = {}, rt[kF32Vec][NH] = {};
 #pragma unroll
   for (int q = 0; q < kF32Vec; ++q) {
     const int64_t j = col(q);
@@ -1074,7 +1125,7 @@ __global__ __launch_bounds__(kF32Threads) void row_grad_f32_kernel(RowPassArgs a
 #pragma unroll
   for (int q = 0; q < kF32Vec; ++q) {
     const int64_t j = col(q);
-    if (j >= v) continue;
+    if (j >= jend) continue;
     float g[NV], gt[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -1091,14 +1142,14 @@ __global__ __launch_bounds__(kF32Threads) void row_grad_f32_kernel(RowPassArgs a
       g[i] = valid ? gi : 0.f;
       gt[i] = valid ? ti : 0.f;
     }
-    store_vec<kF32Nt>(gsrow + j, g);
-    if (TG) store_vec<kF32Nt>(gtrow + j, gt);
+    gsrow.template store<kF32Nt>(j, g);
+    if (TG) gtrow.template store<kF32Nt>(j, gt);
   }
   if (owner) {   // the label term, after this thread's own store of that column
     float gy = 0.f, ty = 0.f, c = 0.f, d = 0.f;
     elem(xs_y, xt_y, gy, ty, c, d);
-    gsrow[y] = static_cast<GT>(gy - a.w_s * one_m_a);
-    if (TG) gtrow[y] = static_cast<GT>(ty - a.w_t * one_m_a);
+    gsrow.set(y, gy - a.w_s * one_m_a);
+    if (TG) gtrow.set(y, ty - a.w_t * one_m_a);
   }
   if (KL) {
 #pragma unroll
@@ -1469,6 +1520,9 @@ hipError_t launch_row_pass(const RowPassArgs& a, hipStream_t s) {
     return hipGetLastError();
   }
   if (a.ld % 8) return hipErrorInvalidValue;
+  if (a.grad_plane > 0 && (a.ltype != DType::F32 || a.grad_s == nullptr || a.grad_plane % 64 ||
+                           a.grad_plane < a.v || a.grad_plane > a.ld))
+    return hipErrorInvalidValue;
   const bool has_t = a.teacher != nullptr;
   const bool kl = a.kl && has_t;
   const bool tg = a.teacher_grad && has_t;
@@ -1577,7 +1631,9 @@ hipError_t launch_row_pass(const RowPassArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((row_consts_kernel<false, false>), cgrid, dim3(kThreads), 0, s, a);            \
     hipLaunchKernelGGL((row_grad_f32_kernel<GT, false, false>), bgrid, dim3(kF32Threads), 0, s, a, chunks); \
   }
-    if (gt == DType::F32) {
+    if (a.grad_plane > 0) {
+      ORDA_ROWGRAD_F32(Planes3)
+    } else if (gt == DType::F32) {
       ORDA_ROWGRAD_F32(float)
     } else {
       ORDA_ROWGRAD_F32(__bf16)
@@ -1591,7 +1647,9 @@ hipError_t launch_row_pass(const RowPassArgs& a, hipStream_t s) {
   else if (kl) hipLaunchKernelGGL((row_pass_fused_kernel<LT, GT, true, false>), grid, dim3(kThreads), 0, s, a);  \
   else if (tg) hipLaunchKernelGGL((row_pass_fused_kernel<LT, GT, false, true>), grid, dim3(kThreads), 0, s, a);  \
   else hipLaunchKernelGGL((row_pass_fused_kernel<LT, GT, false, false>), grid, dim3(kThreads), 0, s, a);
-  if (a.ltype == DType::F32 && gt == DType::BF16) {
+  if (a.grad_plane > 0) {
+    ORDA_ROWPASS(float, Planes3)
+  } else if (a.ltype == DType::F32 && gt == DType::BF16) {
     ORDA_ROWPASS(float, __bf16)
   } else if (a.ltype == DType::F32 && gt == DType::F32) {
     ORDA_ROWPASS(float, float)
