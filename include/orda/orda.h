@@ -262,7 +262,7 @@ int32_t orda_kl_ce_on_logits_chunk(orda_ctx *ctx, const orda_tensor *logits_chun
  * For callers that cannot allocate during the call (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). ctx is
  * required; every tensor and the targets must be on the device; n_rows is at
- * most 32768 (ORDA_ERR_INVALID beyond). The per-row scratch is one 1.75 MiB
+ * most 32768 (ORDA_ERR_INVALID beyond). The scratch is one 1.75 MiB
  * array per GPU held until the process ends and shared by every call on that
  * GPU: calls that overlap on one GPU race. On a stream under HIP graph
  * capture (the context's stream, orda_ctx_set_stream) the call records its

@@ -867,7 +867,6 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         r.label_rows = g.M;
         r.ignore_index = g.lg.ignore_index;
         r.inv_t = g.lg.inv_t;
-        r.segmented = true;
         timed(c, ORDA_KERNEL_GEMM_LOGITS, [&] { return launch_row_stats(r, c->stream); });
         return true;
       }
@@ -891,7 +890,6 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         r.label_rows = g.M;
         r.ignore_index = g.lg.ignore_index;
         r.inv_t = g.lg.inv_t;
-        r.segmented = true;
         // timed with the logits GEMM, as the fused epilogue's statistics are
         timed(c, ORDA_KERNEL_GEMM_LOGITS, [&] { return launch_row_stats(r, c->stream); });
       }
@@ -946,7 +944,6 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         r.ignore_index = P.ignore;
         r.inv_t = inv_t;
         r.online = P.online;
-        r.segmented = true;
         timed(c, ORDA_KERNEL_OTHER, [&] { return launch_row_stats(r, c->stream); });
       } else {
         seg_t = teacher_gemm();
@@ -1004,7 +1001,6 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       r.row_nll_s = rnll_s + gs;
       r.row_nll_t = rnll_t + gs;
       r.row_kl = rkl + gs;
-      r.split = false;
       r.fast_math = P.fast_math;
       timed(c, ORDA_KERNEL_ROW_PASS, [&] { return launch_row_pass(r, c->stream); });
     }
@@ -1464,11 +1460,10 @@ namespace orda {
 
 int32_t ctx_device(const orda_ctx* c) { return c->device; }
 
-// kl_ce_on_logits_chunk (src/cuda/launch.rs:51-158): row statistics of both
-// halves of the chunk, then the split row pass. Device logits are read in
-// place at any pitch; host tensors are staged. With `sc`, every tensor must
-// be on the device and the per-row scratch comes from sc instead of the
-// context's workspace (nothing is allocated).
+// kl_ce_on_logits_chunk (src/cuda/launch.rs:51-158): launch_slot over bands of
+// rows. Device logits are read in place at any pitch; host tensors are staged.
+// With `sc`, every tensor must be on the device and the scratch comes from sc
+// instead of the context's workspace (nothing is allocated).
 void kl_ce_slot(orda_ctx* c, const orda_tensor* logits_chunk, const int32_t* targets,
                 int32_t targets_location, int64_t n_rows, float inv_t, float kl_grad_scale,
                 float t_sq, float student_ce_weight, float teacher_ce_weight,
@@ -1528,85 +1523,47 @@ void kl_ce_slot(orda_ctx* c, const orda_tensor* logits_chunk, const int32_t* tar
   OutMat kr = out_mat(c, *kl_per_row, n_rows, 1, "slot.klr", "kl_per_row");
   OutMat cl = out_mat(c, *ce_loss, grid_rows, 1, "slot.cel", "ce_loss");
   if (gk.ld != v || gc.ld != v) fail(ORDA_ERR_INVALID, "gradient outputs must be dense");
-  const int64_t n2 = std::max<int64_t>(1, 2 * n_rows);
-  int64_t* lab;
-  float4* stats;
-  float* xy;
-  float* nll_unused;
+  // Targets on the host are uploaded.
+  const int32_t* tg = targets;
+  if (targets_location != ORDA_DEVICE && n_rows > 0) {
+    void* d = ws(c, "slot.targets", n_rows * 4);
+    hip_check(hipMemcpyAsync(d, targets, n_rows * 4, hipMemcpyHostToDevice, c->stream), "upload targets");
+    tg = static_cast<const int32_t*>(d);
+  }
+  int64_t band = slot_band_rows(L.t, std::max<int64_t>(1, n_rows), v);
+  void* scratch;
   if (sc) {
-    lab = sc->labels;
-    stats = sc->stats;
-    xy = sc->xy;
-    nll_unused = sc->nll;
+    band = std::min(band, sc->bytes / slot_scratch_bytes(1, v));
+    if (band < 1) fail(ORDA_ERR_INVALID, "V=%lld exceeds the no-allocation scratch", static_cast<long long>(v));
+    scratch = sc->p;
   } else {
-    lab = static_cast<int64_t*>(ws(c, "slot.labels", std::max<int64_t>(1, n_rows) * 8));
-    stats = static_cast<float4*>(ws(c, "slot.stats", n2 * 16));
-    xy = static_cast<float*>(ws(c, "slot.xy", n2 * 4));
-    nll_unused = static_cast<float*>(ws(c, "slot.unused", n2 * 4));
+    scratch = ws(c, "slot.scratch", slot_scratch_bytes(band, v));
   }
-  // Targets widened to the kernels' int64 labels on the stream (device
-  // targets), or on the host and uploaded; the label logits start at zero.
-  std::vector<int64_t> hl;   // lives until the stream is synchronized below
-  if (targets_location == ORDA_DEVICE) {
-    hip_check(launch_widen_targets(targets, n_rows, lab, xy, 2 * n_rows, c->stream), "targets");
-  } else {
-    hl.resize(static_cast<size_t>(n_rows));
-    for (int64_t i = 0; i < n_rows; ++i) hl[i] = targets[i];
-    if (n_rows > 0)
-      hip_check(hipMemcpyAsync(lab, hl.data(), n_rows * 8, hipMemcpyHostToDevice, c->stream),
-                "upload targets");
-    hip_check(launch_widen_targets(nullptr, 0, nullptr, xy, 2 * n_rows, c->stream), "targets");
-  }
-  for (int half = 0; half < 2; ++half) {
-    RowStatsArgs r{};
-    r.src_type = L.t;
-    r.src = at(L.p, half * n_rows * L.ld, L.t);
-    r.lds = L.ld;
-    r.dst = nullptr;
-    r.n_rows = n_rows;
-    r.v = v;
-    r.stats = stats + half * n_rows;
-    r.stats_ld = 1;
-    r.xy = xy + half * n_rows;
-    r.labels = lab;
-    r.ignore_index = ignore_index;
-    r.inv_t = inv_t;
-    launch(ORDA_KERNEL_OTHER, [&] { return launch_row_stats(r, c->stream); });
-  }
-  RowPassArgs a{};
+  auto on_line = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 128 == 0; };
+  SlotArgs a{};
   a.ltype = L.t;
-  a.student = const_cast<void*>(L.p);
-  a.teacher = at(L.p, n_rows * L.ld, L.t);
   a.ld = L.ld;
-  a.n_rows = n_rows;
   a.v = v;
-  a.stats_s = stats;
-  a.stats_t = stats + n_rows;
-  a.stats_ld = 1;
-  a.stats_tiles = 1;
-  a.stats_tiles_t = 1;
-  a.xy_s = xy;
-  a.xy_t = xy + n_rows;
-  a.labels = lab;
   a.ignore_index = ignore_index;
   a.w_s = student_ce_weight;
   a.w_t = teacher_ce_weight;
-  a.kd = 0.f;
-  a.temperature = 1.f / inv_t;
   a.label_smoothing = label_smoothing;
-  a.kl = compute_kl != 0;
-  a.row_nll_s = nll_unused;
-  a.row_nll_t = nll_unused + n_rows;
-  a.row_kl = kr.p;
-  a.split = true;
-  a.grad_kl = gk.p;
-  a.grad_ce = gc.p;
-  a.ce_loss = cl.p;
   a.kl_grad_scale = kl_grad_scale;
   a.t_sq = t_sq;
   a.inv_t = inv_t;
-  a.student_only = student_only != 0;
-  launch(ORDA_KERNEL_ROW_PASS, [&] { return launch_row_pass(a, c->stream); });
+  a.kl = compute_kl != 0;
+  a.teacher_ce = student_only == 0;
+  a.n_rows = n_rows;
+  a.out_lines = v % 32 == 0 && on_line(gk.p) && on_line(gc.p);
+  a.scratch = scratch;
+  a.student = L.p;
+  a.teacher = at(L.p, n_rows * L.ld, L.t);
+  a.targets = tg;
+  a.grad_kl = gk.p;
+  a.kl_row = kr.p;
+  a.grad_ce = gc.p;
+  a.ce_loss = cl.p;
+  launch(ORDA_KERNEL_ROW_PASS, [&] { return launch_slot(a, band, c->stream); });
   download(c, gk);
   download(c, gc);
   download(c, kr);

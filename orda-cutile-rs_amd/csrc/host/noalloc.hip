@@ -3,10 +3,10 @@
 // during the call (code under HIP graph capture, tight serving loops,
 // harnesses that forbid hipMalloc).
 //
-// The per-row scratch the kernels need (int64 labels, row statistics of both
-// halves of the chunk, label logits, row losses: 56 bytes per row) lives in
-// one file-scope device array of kMaxRows rows (1.75 MiB), which every GPU
-// the library runs on holds until the process ends. Host code never passes
+// The scratch the kernels need (the statistics of a band of rows' segments)
+// lives in one file-scope device array of 1.75 MiB, which every GPU the
+// library runs on holds until the process ends; the rows of a call go through
+// it in as many bands as that takes. Host code never passes
 // the array's name to a kernel: its device address is looked up once per
 // device with hipGetSymbolAddress (at context creation, with that device
 // current) and only that address is used. Every call on a GPU shares that
@@ -19,9 +19,7 @@
 namespace {
 
 constexpr int64_t kMaxRows = 32768;
-// labels 8 B, stats 2 x 16 B, label logits 2 x 4 B, row losses 2 x 4 B
-constexpr int64_t kBytesPerRow = 8 + 2 * 16 + 2 * 4 + 2 * 4;
-constexpr int64_t kScratchBytes = kMaxRows * kBytesPerRow;
+constexpr int64_t kScratchBytes = kMaxRows * 56;
 constexpr int kMaxDevices = 64;
 
 }  // namespace
@@ -82,10 +80,8 @@ extern "C" int32_t orda_kl_ce_on_logits_chunk_noalloc(
     unsigned char* base = static_cast<unsigned char*>(scratch_of(dev));
     orda::SlotScratch sc;
     sc.max_rows = kMaxRows;
-    sc.labels = reinterpret_cast<int64_t*>(base);
-    sc.stats = reinterpret_cast<float4*>(base + 8 * kMaxRows);
-    sc.xy = reinterpret_cast<float*>(base + 40 * kMaxRows);
-    sc.nll = reinterpret_cast<float*>(base + 48 * kMaxRows);
+    sc.p = base;
+    sc.bytes = kScratchBytes;
     orda::kl_ce_slot(ctx, logits_chunk, targets, targets_location, n_rows, inv_t, kl_grad_scale,
                      t_sq, student_ce_weight, teacher_ce_weight, label_smoothing, ignore_index,
                      student_only, compute_kl, grad_kl_student, kl_per_row, grad_ce, ce_loss, &sc);

@@ -30,15 +30,12 @@ struct Error {
   std::string msg;
 };
 
-// Caller-provided per-row scratch of the chunk-launcher entry point (rows up
-// to max_rows): int64 labels [max_rows], float4 stats [2*max_rows], float
-// label logits [2*max_rows], float row losses [2*max_rows].
+// Caller-provided scratch of the chunk-launcher entry point, for at most
+// max_rows rows a call.
 struct SlotScratch {
   int64_t max_rows;
-  int64_t* labels;
-  float4* stats;
-  float* xy;
-  float* nll;
+  void* p;
+  int64_t bytes;
 };
 
 // kl_ce_on_logits_chunk (src/cuda/launch.rs:51-158) behind both C entry

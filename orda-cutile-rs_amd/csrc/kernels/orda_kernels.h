@@ -161,7 +161,7 @@ int64_t gemm_stat_tiles(int64_t n);   // ceil(n/256)
 
 // ---------------------------------------------------------------- row pass
 // Fused KL + CE + merge over row pairs of a logits chunk, gradient written
-// in place (or to split outputs for the chunk-launcher entry point).
+// in place or to separate rows.
 struct RowPassArgs {
   DType ltype;             // logits storage dtype
   void* student;           // row r of the student block at student + r*ld
@@ -202,9 +202,8 @@ struct RowPassArgs {
   // GEMM (LogitStatsArgs::hmax): half k of row r has its maximum at
   // hmax_s[r*hmax_ld + 2*k] (student) and hmax_t[r*hmax_ld + 2*k]
   // (teacher, hmax_s + 1 for the GEMM's paired layout), or null for rows
-  // stored as they are (Precomputed teacher logits, the chunk-launcher
-  // entry point). The chunked pass over paired bf16 rows runs only with
-  // them, interleaved.
+  // stored as they are (Precomputed teacher logits). The chunked pass over
+  // paired bf16 rows runs only with them, interleaved.
   const float* hmax_s;
   const float* hmax_t;
   int64_t hmax_ld;
@@ -217,16 +216,6 @@ struct RowPassArgs {
   // planes of grad_plane elements (>= v, a multiple of 64, at most the
   // student pitch ld) at grad_s/grad_t + r*3*grad_plane, zeros past v.
   int64_t grad_plane;
-  // Split mode (chunk-launcher entry point): gradients go to separate
-  // buffers instead of overwriting the logits, and are not merged.
-  bool split;
-  float* grad_kl;          // [n_rows][v] (split mode)
-  float* grad_ce;          // [n_rows or 2*n_rows][v] (split mode)
-  float* ce_loss;          // [n_rows or 2*n_rows] (split mode)
-  float kl_grad_scale;     // split mode: KL gradient scale as given
-  float t_sq;              // split mode: T^2 as given
-  float inv_t;             // split mode: 1/T as given
-  bool student_only;       // split mode: CE over student rows only
   bool fast_math;          // per-row logs and divisions by the hardware approximations
   // The teacher rows are logits as they are, fp32 (Precomputed teacher
   // logits, or a Separate teacher's) or bf16 (teacher_bf16: Precomputed
@@ -242,11 +231,13 @@ hipError_t launch_row_pass(const RowPassArgs& a, hipStream_t stream);
 // float4 entries per row of RowPassArgs::kl_part (ceil(v/512)).
 int64_t row_pass_kl_blocks(int64_t v);
 
-// Per-row statistics of rows that were not produced by the GEMM (Precomputed
-// teacher logits, the chunk-launcher entry point). Reads src (fp32 or bf16,
-// any pitch), writes one stats entry per row and the fp32 target logit, and
-// optionally copies the row into dst (logits dtype, pitch ldd, zero padding
-// up to the next multiple of 8).
+// Per-row statistics of rows that were not produced by the GEMM's statistics
+// epilogue (Precomputed teacher logits, fp32 logits of split products). Reads
+// src (fp32 or bf16, any pitch), one workgroup per 8192-column segment of a row,
+// held in registers for both passes (one read); writes segment s's statistics
+// to stats[r * stats_ld + s] (stats_ld >= row_stats_segments(v)) and the fp32
+// target logit, and optionally copies the row into dst (logits dtype, pitch
+// ldd, zero padding up to the next multiple of 8).
 struct RowStatsArgs {
   DType src_type;
   const void* src;
@@ -255,7 +246,7 @@ struct RowStatsArgs {
   void* dst;               // may be null
   int64_t ldd;
   int64_t n_rows, v;
-  float4* stats;           // stats[r * stats_ld]
+  float4* stats;
   int64_t stats_ld;
   float* xy;
   const int64_t* labels;   // may be null (then xy is not written)
@@ -263,11 +254,7 @@ struct RowStatsArgs {
   int64_t ignore_index;
   float inv_t;
   bool online;             // one online pass; else a max pass, then a sum pass
-  // With segmented (and !online): one workgroup per 8192-column segment of a
-  // row, held in registers for both passes (one read), statistics of
-  // segment s at stats[r * stats_ld + s]; stats_ld >= row_stats_segments(v).
-  bool segmented;
-  // segmented fp32 rows only: src holds src_splits split-K partials, split s
+  // fp32 rows, not online: src holds src_splits split-K partials, split s
   // at src + s*src_split_stride; each element is their sum in split order
   // (the reduction launch_gemm would run), written to dst.
   int src_splits;
@@ -275,6 +262,32 @@ struct RowStatsArgs {
 };
 hipError_t launch_row_stats(const RowStatsArgs& a, hipStream_t stream);
 int64_t row_stats_segments(int64_t v);
+
+// ---------------------------------------------------------------- the slot
+// KL and CE of prepared logits to separate outputs (slot.hip); student and
+// teacher rows share one pitch.
+struct SlotArgs {
+  DType ltype;
+  int64_t n_rows;            // row pairs
+  const void* student;
+  const void* teacher;
+  int64_t ld, v;             // any pitch >= v
+  const int32_t* targets;
+  int32_t ignore_index;
+  float w_s, w_t, label_smoothing;
+  float kl_grad_scale, t_sq, inv_t;
+  bool kl, teacher_ce;       // neither: the teacher rows are not read
+  float* grad_kl;            // [rows][v], zeros without kl
+  float* kl_row;
+  float* grad_ce;            // student rows, then (teacher_ce) teacher rows
+  float* ce_loss;            // likewise
+  bool out_lines;            // every output row starts on a 128-byte line
+  void* scratch;             // slot_scratch_bytes(band, v), 16-byte aligned
+};
+// Rows per band for logits of type t, and the scratch of a call in such bands.
+int64_t slot_band_rows(DType t, int64_t n_rows, int64_t v);
+int64_t slot_scratch_bytes(int64_t band, int64_t v);
+hipError_t launch_slot(const SlotArgs& a, int64_t band, hipStream_t stream);
 
 // ---------------------------------------------------------------- reductions
 // Sums per-row losses into the reference's scalars (api.rs:401-405):
@@ -323,11 +336,6 @@ struct LabelStatus {
 };
 hipError_t launch_label_check(const int64_t* labels, int64_t n, int64_t v, int64_t ignore_index,
                               bool mean, LabelStatus* out, hipStream_t stream);
-
-// out64[i] = in32[i] for i < n, and zero[i] = 0 for i < n_zero (the targets of
-// the chunk-launcher entry point widened to the kernels' int64 labels).
-hipError_t launch_widen_targets(const int32_t* in32, int64_t n, int64_t* out64, float* zero,
-                                int64_t n_zero, hipStream_t stream);
 
 // keep[labels[i]] = 1 for every in-range, non-ignored label.
 hipError_t launch_mark_targets(const int64_t* labels, int64_t n, int64_t ignore_index,

@@ -203,16 +203,6 @@ __global__ __launch_bounds__(kCheckThreads) void label_check_kernel(const int64_
   }
 }
 
-__global__ void widen_targets_kernel(const int32_t* in32, int64_t n, int64_t* out64, float* zero,
-                                     int64_t n_zero) {
-  const int64_t total = n > n_zero ? n : n_zero;
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    if (i < n) out64[i] = in32[i];
-    if (i < n_zero) zero[i] = 0.f;
-  }
-}
-
 // Rows of src (any pitch and alignment) into dst rows of pitch ldd, a
 // multiple of 8 elements, zero past `cols`: one workgroup per (row, 2048
 // columns), eight columns a thread, stored as one (bf16) or two (fp32)
@@ -356,15 +346,6 @@ hipError_t launch_label_check(const int64_t* labels, int64_t n, int64_t v, int64
                               bool mean, LabelStatus* out, hipStream_t s) {
   hipLaunchKernelGGL(label_check_kernel, dim3(1), dim3(kCheckThreads), 0, s, labels, n, v,
                      ignore_index, mean, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_widen_targets(const int32_t* in32, int64_t n, int64_t* out64, float* zero,
-                                int64_t n_zero, hipStream_t s) {
-  const int64_t total = n > n_zero ? n : n_zero;
-  if (total <= 0) return hipSuccess;
-  hipLaunchKernelGGL(widen_targets_kernel, dim3(grid_for(total)), dim3(256), 0, s, in32, n, out64,
-                     zero, n_zero);
   return hipGetLastError();
 }
 

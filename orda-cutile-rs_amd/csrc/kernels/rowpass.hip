@@ -30,35 +30,17 @@
 
 #include <type_traits>
 
-#include "kl_sums.h"
 #include "orda_kernels.h"
+#include "row_terms.h"
 #include "split3.h"
 
 namespace orda {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-
-// Per-row constants: precise logf / IEEE division, or with fast_math the
-// hardware approximations (v_log_f32 times ln 2, v_rcp_f32 then a multiply).
-__device__ __forceinline__ float rlog(float x, bool fast) {
-  return fast ? __builtin_amdgcn_logf(x) * kLn2 : logf(x);
-}
-__device__ __forceinline__ float rlog2(float x, bool fast) {
-  return fast ? __builtin_amdgcn_logf(x) : log2f(x);
-}
-__device__ __forceinline__ float rdiv(float a, float b, bool fast) {
-  return fast ? a * __builtin_amdgcn_rcpf(b) : a / b;
-}
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-struct Stat {
-  float m, d1, dT, sx;
-};
 
 __device__ __forceinline__ Stat merge(Stat a, Stat b, float it2) {
   Stat r;
@@ -166,20 +148,6 @@ struct Vec<__bf16> {
   }
 };
 
-// KL_row (without T²) of a row pair from its merged statistics s, t and the
-// paired GEMM's merged KL sums x (kl_sums.h): the mean of the centred
-// difference under p_t^T plus log1p(x.y / t.dT) = lse_s^T - lse_t^T (with
-// the shift between the two maxima taken out of both). Precise log1p and
-// division of the sums in every profile (they carry the small-KL
-// precision; one per row). Should x.y / t.dT not lie in (-1, inf), the two
-// rows' own sums instead.
-__device__ __forceinline__ float kl_paired(float2 x, const Stat& s, const Stat& t, float inv_t,
-                                           bool fast) {
-  const float z = x.y / t.dT;
-  const float lr = isfinite(z) && z > -1.f ? log1pf(z) : rlog(rdiv(s.dT, t.dT, fast), fast);
-  return rdiv(x.x, t.dT, fast) * (kLn2 * inv_t) + lr;
-}
-
 // KL_row (without T²) from the sums of a pass that forms p_s^T and p_t^T
 // itself as 2^(x·log2(e)/T − o) (scaled by the same factor g in both):
 // cross = g·Σ p_t^T (x_t − x_s), sum_t = g·Σ p_t^T, sum_d = g·Σ (p_s^T − p_t^T)
@@ -190,195 +158,6 @@ __device__ __forceinline__ float kl_paired(float2 x, const Stat& s, const Stat& 
 __device__ __forceinline__ float kl_from_sums(float cross, float sum_t, float sum_d, float d_off,
                                               float inv_t, bool fast) {
   return rdiv(cross, sum_t, fast) * inv_t + d_off * kLn2 + log1pf(sum_d / sum_t);
-}
-
-// nll of cross_entropy.rs:46-56 from merged stats, in f64.
-__device__ __forceinline__ double row_nll(const Stat& s, float xy, double alpha, int64_t v) {
-  const double lse = static_cast<double>(s.m) + log(static_cast<double>(s.d1));
-  if (alpha > 0.0)
-    return lse - (1.0 - alpha) * static_cast<double>(xy) -
-           (alpha / static_cast<double>(v)) * static_cast<double>(s.sx);
-  return lse - static_cast<double>(xy);
-}
-
-template <typename LT, bool SPLIT, int TPB>
-__global__ __launch_bounds__(TPB) void row_pass_kernel(RowPassArgs a) {
-  __shared__ Stat sstat[TPB / 64];
-  __shared__ float ssum[TPB / 64];
-  const int64_t r = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int64_t y = a.labels[r];
-  // A label outside [0, V) that is not ignore_index is an error the host
-  // reports; the row is then treated as ignored so no access leaves the row.
-  const bool ignored = y == a.ignore_index || y < 0 || y >= a.v;
-  const bool has_t = a.teacher != nullptr;
-  const float T = a.temperature;
-  const float inv_t = SPLIT ? a.inv_t : 1.0f / T;
-  const float it2 = inv_t * kLog2e;
-
-  const Stat ss = load_row_stats<TPB>(a.stats_s + r * a.stats_ld, a.stats_tiles, it2, sstat);
-  Stat st{-INFINITY, 0.f, 0.f, 0.f};
-  if (has_t) st = load_row_stats<TPB>(a.stats_t + r * a.stats_ld, a.stats_tiles_t, it2, sstat);
-
-  const double alpha = static_cast<double>(a.label_smoothing);
-  // Per-row constants: p = exp2(x*log2e - off).
-  const float lse1_s = ss.m + logf(ss.d1);
-  const float lseT_s = ss.m * inv_t + logf(ss.dT);
-  const float lse1_t = st.m + logf(st.d1);
-  const float lseT_t = st.m * inv_t + logf(st.dT);
-  const float o1s = lse1_s * kLog2e, oTs = lseT_s * kLog2e;
-  const float o1t = lse1_t * kLog2e, oTt = lseT_t * kLog2e;
-
-  const float eps = static_cast<float>(alpha / static_cast<double>(a.v));
-  const float one_m_a = 1.0f - a.label_smoothing;
-  // CE scales (ignored rows -> 0, cross_entropy.rs:59).
-  const float ws = ignored ? 0.f : a.w_s;
-  const float wt = ignored ? 0.f : a.w_t;
-  const bool do_kl = a.kl && has_t;
-  const float gsc = ignored ? 0.f : (SPLIT ? a.kl_grad_scale : a.kd * T);  // kl.rs:85
-  const bool do_tgrad = SPLIT ? (!a.student_only && has_t) : (a.teacher_grad && has_t);
-
-  LT* srow = static_cast<LT*>(a.student) + r * a.ld;
-  LT* trow = has_t ? static_cast<LT*>(a.teacher) + r * a.ld : nullptr;
-  float* gkl = SPLIT ? a.grad_kl + r * a.v : nullptr;
-  float* gce_s = SPLIT ? a.grad_ce + r * a.v : nullptr;
-  float* gce_t = (SPLIT && do_tgrad) ? a.grad_ce + (a.n_rows + r) * a.v : nullptr;
-
-  using VT = Vec<LT>;
-  constexpr int NV = VT::N;
-  float cross = 0.f, sum_pt = 0.f, sum_d = 0.f;
-  const int64_t vpad = (a.v + NV - 1) / NV * NV;
-  // Rows are read where they are, at any pitch: 16-byte vectors where the
-  // row is 16-byte aligned and the vector lies inside the row, single
-  // elements otherwise (nothing past column V is read).
-  const bool vec = (reinterpret_cast<uintptr_t>(srow) & 15) == 0 &&
-                   (!has_t || (reinterpret_cast<uintptr_t>(trow) & 15) == 0);
-  // SPLIT outputs (dense fp32 rows) leave as 16-byte stores where this
-  // row's outputs are 16-byte aligned.
-  const bool ovec = SPLIT && (reinterpret_cast<uintptr_t>(gce_s) & 15) == 0 &&
-                    (!do_kl || (reinterpret_cast<uintptr_t>(gkl) & 15) == 0) &&
-                    (!do_tgrad || (reinterpret_cast<uintptr_t>(gce_t) & 15) == 0);
-  for (int64_t j0 = static_cast<int64_t>(tid) * NV; j0 < vpad; j0 += TPB * NV) {
-    float xs[NV], xt[NV], gs[NV], gt[NV], gk[NV];
-    const bool whole = vec && j0 + NV <= a.v;
-    if (whole) {
-      VT::unpack(*reinterpret_cast<const typename VT::raw*>(srow + j0), xs);
-      if (has_t) VT::unpack(*reinterpret_cast<const typename VT::raw*>(trow + j0), xt);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const bool in = j0 + i < a.v;
-        xs[i] = in ? static_cast<float>(srow[j0 + i]) : 0.f;
-        xt[i] = in && has_t ? static_cast<float>(trow[j0 + i]) : 0.f;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int64_t j = j0 + i;
-      const bool valid = j < a.v;
-      float g = 0.f, gkv = 0.f, gtv = 0.f;
-      if (valid) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(xs[i], kLog2e, -o1s));
-        float prob = p - eps;
-        if (j == y) prob -= one_m_a;
-        g = prob * ws;
-        if (do_kl) {
-          const float ps = __builtin_amdgcn_exp2f(fmaf(xs[i], it2, -oTs));
-          const float pt = __builtin_amdgcn_exp2f(fmaf(xt[i], it2, -oTt));
-          const float d = ps - pt;
-          gkv = gsc * d;
-          cross = fmaf(pt, xt[i] - xs[i], cross);
-          sum_pt += pt;
-          sum_d += d;
-        }
-        if (do_tgrad) {
-          const float q = __builtin_amdgcn_exp2f(fmaf(xt[i], kLog2e, -o1t));
-          float pr = q - eps;
-          if (j == y) pr -= one_m_a;
-          gtv = pr * wt;
-        }
-      }
-      if (SPLIT) {
-        gs[i] = g;
-        gk[i] = gkv;
-        gt[i] = gtv;
-      } else {
-        gs[i] = ignored ? 0.f : g + gkv;
-        gt[i] = gtv;
-      }
-    }
-    if (SPLIT) {
-      if (whole && ovec) {
-        typedef float f4 __attribute__((ext_vector_type(4)));
-        // Non-temporal only where a store instruction covers whole lines
-        // (fp32 logits: 16 bytes a lane, lanes adjacent). With bf16 logits a
-        // lane's 8 outputs are two stores 16 bytes apart, each instruction
-        // covering half of every line: as non-temporal stores the pass took
-        // 0.55 ms at 512 x 131072, as ordinary ones 0.24 ms.
-        auto st4 = [&](float* p, const float* g) {
-          const f4 w = f4{g[0], g[1], g[2], g[3]};
-          if (NV == 4) __builtin_nontemporal_store(w, reinterpret_cast<f4*>(p));
-          else *reinterpret_cast<f4*>(p) = w;
-        };
-#pragma unroll
-        for (int h = 0; h < NV / 4; ++h) {
-          st4(gce_s + j0 + 4 * h, gs + 4 * h);
-          if (do_kl) st4(gkl + j0 + 4 * h, gk + 4 * h);
-          if (do_tgrad) st4(gce_t + j0 + 4 * h, gt + 4 * h);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-          if (j0 + i >= a.v) break;
-          gce_s[j0 + i] = gs[i];
-          if (do_kl) gkl[j0 + i] = gk[i];
-          if (do_tgrad) gce_t[j0 + i] = gt[i];
-        }
-      }
-    } else {
-      if (whole) {
-        *reinterpret_cast<typename VT::raw*>(srow + j0) = VT::pack(gs);
-        if (do_tgrad) *reinterpret_cast<typename VT::raw*>(trow + j0) = VT::pack(gt);
-      } else {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-          if (j0 + i >= a.v) break;
-          srow[j0 + i] = static_cast<LT>(gs[i]);
-          if (do_tgrad) trow[j0 + i] = static_cast<LT>(gt[i]);
-        }
-      }
-    }
-  }
-  if (SPLIT && !do_kl && a.grad_kl) {
-    for (int64_t j = tid; j < a.v; j += TPB) gkl[j] = 0.f;
-  }
-
-  if (do_kl) {
-    cross = block_sum<TPB>(cross, ssum);
-    sum_pt = block_sum<TPB>(sum_pt, ssum);
-    sum_d = block_sum<TPB>(sum_d, ssum);
-  }
-  if (tid == 0) {
-    const float xy_s = ignored ? 0.f : a.xy_s[r];
-    const double nll_s = ignored ? 0.0 : row_nll(ss, xy_s, alpha, a.v);
-    float kl_row = 0.f;
-    if (do_kl && !ignored) {
-      const float t_sq = SPLIT ? a.t_sq : T * T;   // kl.rs:86
-      kl_row = kl_from_sums(cross, sum_pt, sum_d, oTs - oTt, inv_t, false) * t_sq;
-    }
-    double nll_t = 0.0;
-    const bool tce = SPLIT ? (!a.student_only && has_t) : (a.teacher_ce && has_t);
-    if (tce && !ignored) nll_t = row_nll(st, a.xy_t[r], alpha, a.v);
-    if (SPLIT) {
-      a.ce_loss[r] = static_cast<float>(nll_s);
-      if (tce) a.ce_loss[a.n_rows + r] = static_cast<float>(nll_t);
-      if (a.row_kl) a.row_kl[r] = kl_row;
-    } else {
-      a.row_nll_s[r] = static_cast<float>(nll_s);
-      a.row_nll_t[r] = static_cast<float>(nll_t);
-      a.row_kl[r] = kl_row;
-    }
-  }
 }
 
 // Eight consecutive logits (16-byte aligned) as fp32.
@@ -1227,109 +1006,6 @@ __device__ float block_max(float v, float* scratch) {
   return r;
 }
 
-// Per-row statistics {max, Σe^(x-max), Σe^((x-max)/T), Σx} of rows the GEMM
-// did not produce. ONLINE: one read, each element merged into running
-// statistics (two exponentials per statistic); otherwise a max pass, then a
-// pass summing e^(x-max) and e^((x-max)/T) (the second read of a row mostly
-// hits the cache).
-template <typename ST, typename DT, bool ONLINE>
-__global__ __launch_bounds__(kThreads) void row_stats_kernel(RowStatsArgs a) {
-  __shared__ Stat sstat[kThreads / 64];
-  __shared__ float sred[kThreads / 64];
-  const int64_t r = blockIdx.x;
-  const ST* src = static_cast<const ST*>(a.src) + r * a.lds;
-  DT* dst = a.dst ? static_cast<DT*>(a.dst) + r * a.ldd : nullptr;
-  const float it2 = a.inv_t * kLog2e;
-  Stat s{-INFINITY, 0.f, 0.f, 0.f};
-  if constexpr (ONLINE) {
-    for (int64_t j = threadIdx.x; j < a.v; j += kThreads) {
-      const float x = static_cast<float>(src[j]);
-      if (dst) dst[j] = static_cast<DT>(x);
-      s = merge(s, Stat{x, 1.f, 1.f, x}, it2);
-    }
-    s = block_merge(s, it2, sstat);
-  } else {
-    float m = -INFINITY, sx = 0.f;
-    for (int64_t j = threadIdx.x; j < a.v; j += kThreads) {
-      const float x = static_cast<float>(src[j]);
-      if (dst) dst[j] = static_cast<DT>(x);
-      m = fmaxf(m, x);
-      sx += x;
-    }
-    m = block_max(m, sred);
-    const float o1 = -m * kLog2e, oT = -m * it2;
-    float d1 = 0.f, dT = 0.f;
-    for (int64_t j = threadIdx.x; j < a.v; j += kThreads) {
-      const float x = static_cast<float>(src[j]);
-      d1 += __builtin_amdgcn_exp2f(fmaf(x, kLog2e, o1));
-      dT += __builtin_amdgcn_exp2f(fmaf(x, it2, oT));
-    }
-    s.m = m;
-    s.sx = block_sum(sx, sred);
-    s.d1 = block_sum(d1, sred);
-    s.dT = block_sum(dT, sred);
-  }
-  if (dst)
-    for (int64_t j = a.v + threadIdx.x; j < a.ldd; j += kThreads) dst[j] = static_cast<DT>(0.f);
-  if (threadIdx.x == 0) {
-    a.stats[r * a.stats_ld] = make_float4(s.m, s.d1, s.dT, s.sx);
-    if (a.labels) {
-      const int64_t y = a.labels[a.label_rows > 0 ? r % a.label_rows : r];
-      if (y != a.ignore_index && y >= 0 && y < a.v) a.xy[r] = static_cast<float>(src[y]);
-    }
-  }
-}
-
-// The chunk-launcher slot's statistics of whole rows (no converted copy):
-// two passes over the row, max then the exponential sums, by 1024 threads,
-// with 16-byte loads where every row is 16-byte aligned. (With 256 threads
-// and single-element loads the slot ran at 1.0-2.0 TB/s at 512-1024 rows.)
-constexpr int kWideThreads = 1024;
-template <typename ST, bool VEC>
-__global__ __launch_bounds__(kWideThreads) void row_stats_wide_kernel(RowStatsArgs a) {
-  __shared__ float sred[kWideThreads / 64];
-  const int64_t r = blockIdx.x;
-  const ST* src = static_cast<const ST*>(a.src) + r * a.lds;
-  const float it2 = a.inv_t * kLog2e;
-  using VT = Vec<ST>;
-  constexpr int NV = VT::N;
-  const int64_t nfull = VEC ? a.v / NV : 0;
-  auto each = [&](auto&& f) {
-    if constexpr (VEC) {
-      for (int64_t q = threadIdx.x; q < nfull; q += kWideThreads) {
-        float x[NV];
-        VT::unpack(*reinterpret_cast<const typename VT::raw*>(src + q * NV), x);
-#pragma unroll
-        for (int i = 0; i < NV; ++i) f(x[i]);
-      }
-    }
-    for (int64_t j = nfull * NV + threadIdx.x; j < a.v; j += kWideThreads)
-      f(static_cast<float>(src[j]));
-  };
-  float m = -INFINITY, sx = 0.f;
-  each([&](float x) {
-    m = fmaxf(m, x);
-    sx += x;
-  });
-  m = block_max<kWideThreads>(m, sred);
-  const float o1 = -m * kLog2e, oT = -m * it2;
-  float d1 = 0.f, dT = 0.f;
-  each([&](float x) {
-    d1 += __builtin_amdgcn_exp2f(fmaf(x, kLog2e, o1));
-    dT += __builtin_amdgcn_exp2f(fmaf(x, it2, oT));
-  });
-  sx = block_sum<kWideThreads>(sx, sred);
-  d1 = block_sum<kWideThreads>(d1, sred);
-  dT = block_sum<kWideThreads>(dT, sred);
-  if (threadIdx.x == 0) {
-    a.stats[r * a.stats_ld] = make_float4(m, d1, dT, sx);
-    if (a.labels) {
-      const int64_t y = a.labels[a.label_rows > 0 ? r % a.label_rows : r];
-      if (y != a.ignore_index && y >= 0 && y < a.v) a.xy[r] = static_cast<float>(src[y]);
-    }
-  }
-}
-
 // Segmented two-pass statistics: one workgroup per (row, 8192-column
 // segment); each thread holds its 32 columns in registers, so the max pass
 // and the sum pass read HBM once.
@@ -1504,21 +1180,10 @@ hipError_t launch_row_pass(const RowPassArgs& a, hipStream_t s) {
   // Half-tile-relative rows: bf16 logits of the logits GEMM only, and never
   // where the KL cross term is formed from the stored logits.
   if ((a.hmax_s != nullptr || a.hmax_t != nullptr) &&
-      (a.split || a.ltype != DType::BF16 || (a.kl && a.cross == nullptr) ||
+      (a.ltype != DType::BF16 || (a.kl && a.cross == nullptr) ||
        a.hmax_ld < 4 * ((a.v + 255) / 256)))
     return hipErrorInvalidValue;
   dim3 grid(static_cast<unsigned>(a.n_rows));
-  if (a.split) {   // any pitch and alignment
-    // 512 threads a row: at 512 x 131072 and 1024 x 32000 fp32 logits
-    // 0.470 and 0.220 ms per slot call, against 0.50 and 0.220 ms with 256
-    // threads and 0.468 and 0.242 ms with 1024 (bf16 within 3 % of each other).
-    constexpr int kSplitThreads = 512;
-    if (a.ltype == DType::BF16)
-      hipLaunchKernelGGL((row_pass_kernel<__bf16, true, kSplitThreads>), grid, dim3(kSplitThreads), 0, s, a);
-    else
-      hipLaunchKernelGGL((row_pass_kernel<float, true, kSplitThreads>), grid, dim3(kSplitThreads), 0, s, a);
-    return hipGetLastError();
-  }
   if (a.ld % 8) return hipErrorInvalidValue;
   if (a.grad_plane > 0 && (a.ltype != DType::F32 || a.grad_s == nullptr || a.grad_plane % 64 ||
                            a.grad_plane < a.v || a.grad_plane > a.ld))
@@ -1668,58 +1333,34 @@ int64_t row_pass_kl_blocks(int64_t v) { return (v + kF32Chunk - 1) / kF32Chunk; 
 
 hipError_t launch_row_stats(const RowStatsArgs& a, hipStream_t s) {
   if (a.n_rows <= 0) return hipSuccess;
-  if (a.src_splits > 1 && (!a.segmented || a.online || a.src_type != DType::F32 || a.dst == nullptr))
+  if (a.src_splits > 1 && (a.online || a.src_type != DType::F32 || a.dst == nullptr))
     return hipErrorInvalidValue;
-  dim3 grid(static_cast<unsigned>(a.n_rows));
   const bool sf = a.src_type == DType::F32;
   const bool df = a.dst_type == DType::F32;
-  if (a.segmented) {
-    const int64_t nseg = row_stats_segments(a.v);
-    if (a.stats_ld < nseg) return hipErrorInvalidValue;
-    const int64_t blocks = a.n_rows * nseg;
-    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    const dim3 g(static_cast<unsigned>(blocks));
-    // 16-byte fp32 vectors where the rows allow them (split-K partials
-    // always do; a row of any pitch otherwise goes element by element)
-    const bool vec = sf && a.lds % 4 == 0 && reinterpret_cast<uintptr_t>(a.src) % 16 == 0 &&
-                     a.src_split_stride % 4 == 0 &&
-                     (a.dst == nullptr ||
-                      (df && a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0));
-    if (a.src_splits > 1 && !vec) return hipErrorInvalidValue;
+  const int64_t nseg = row_stats_segments(a.v);
+  if (a.stats_ld < nseg) return hipErrorInvalidValue;
+  const int64_t blocks = a.n_rows * nseg;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  const dim3 g(static_cast<unsigned>(blocks));
+  // 16-byte fp32 vectors where the rows allow them (split-K partials
+  // always do; a row of any pitch otherwise goes element by element)
+  const bool vec = sf && a.lds % 4 == 0 && reinterpret_cast<uintptr_t>(a.src) % 16 == 0 &&
+                   a.src_split_stride % 4 == 0 &&
+                   (a.dst == nullptr ||
+                    (df && a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.dst) % 16 == 0));
+  if (a.src_splits > 1 && !vec) return hipErrorInvalidValue;
 #define ORDA_ROWSTATS_SEG(ON)                                                                            \
   if (vec) hipLaunchKernelGGL((row_stats_seg_kernel<float, float, true, ON>), g, dim3(kThreads), 0, s, a, nseg); \
   else if (sf && df) hipLaunchKernelGGL((row_stats_seg_kernel<float, float, false, ON>), g, dim3(kThreads), 0, s, a, nseg); \
   else if (sf) hipLaunchKernelGGL((row_stats_seg_kernel<float, __bf16, false, ON>), g, dim3(kThreads), 0, s, a, nseg); \
   else if (df) hipLaunchKernelGGL((row_stats_seg_kernel<__bf16, float, false, ON>), g, dim3(kThreads), 0, s, a, nseg); \
   else hipLaunchKernelGGL((row_stats_seg_kernel<__bf16, __bf16, false, ON>), g, dim3(kThreads), 0, s, a, nseg);
-    if (a.online) {
-      ORDA_ROWSTATS_SEG(true)
-    } else {
-      ORDA_ROWSTATS_SEG(false)
-    }
-#undef ORDA_ROWSTATS_SEG
-    return hipGetLastError();
-  }
-  if (!a.online && a.dst == nullptr) {
-    const int es = sf ? 4 : 2;
-    const bool vec = reinterpret_cast<uintptr_t>(a.src) % 16 == 0 && (a.lds * es) % 16 == 0;
-    if (sf && vec) hipLaunchKernelGGL((row_stats_wide_kernel<float, true>), grid, dim3(kWideThreads), 0, s, a);
-    else if (sf) hipLaunchKernelGGL((row_stats_wide_kernel<float, false>), grid, dim3(kWideThreads), 0, s, a);
-    else if (vec) hipLaunchKernelGGL((row_stats_wide_kernel<__bf16, true>), grid, dim3(kWideThreads), 0, s, a);
-    else hipLaunchKernelGGL((row_stats_wide_kernel<__bf16, false>), grid, dim3(kWideThreads), 0, s, a);
-    return hipGetLastError();
-  }
-#define ORDA_ROWSTATS(ONLINE)                                                                        \
-  if (sf && df) hipLaunchKernelGGL((row_stats_kernel<float, float, ONLINE>), grid, dim3(kThreads), 0, s, a);   \
-  else if (sf) hipLaunchKernelGGL((row_stats_kernel<float, __bf16, ONLINE>), grid, dim3(kThreads), 0, s, a);  \
-  else if (df) hipLaunchKernelGGL((row_stats_kernel<__bf16, float, ONLINE>), grid, dim3(kThreads), 0, s, a);  \
-  else hipLaunchKernelGGL((row_stats_kernel<__bf16, __bf16, ONLINE>), grid, dim3(kThreads), 0, s, a);
   if (a.online) {
-    ORDA_ROWSTATS(true)
+    ORDA_ROWSTATS_SEG(true)
   } else {
-    ORDA_ROWSTATS(false)
+    ORDA_ROWSTATS_SEG(false)
   }
-#undef ORDA_ROWSTATS
+#undef ORDA_ROWSTATS_SEG
   return hipGetLastError();
 }
 
