@@ -620,7 +620,7 @@ int64_t staged_bytes_per_row(const LossPlan& P, const Inputs& in) {
 }
 
 // The split-K workspace a backward GEMM asks for, if any (one buffer shared
-// by the GEMMs of a call: they run in order on one stream).
+// by the GEMMs of a call: they run in order on one stream) and if it fits.
 void attach_split_ws(orda_ctx* c, orda::GemmArgs& g) {
   const int64_t b = orda::gemm_split_bytes(g);
   if (b <= 0) return;
@@ -628,8 +628,12 @@ void attach_split_ws(orda_ctx* c, orda::GemmArgs& g) {
   // Growing the buffer frees the old one, which launches already queued on
   // the stream may still use.
   if (cur.p && cur.bytes < b) hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-  g.split_ws = static_cast<float*>(ws(c, "splitk", b));
-  g.split_ws_bytes = b;
+  try {
+    g.split_ws = static_cast<float*>(ws(c, "splitk", b));
+    g.split_ws_bytes = b;
+  } catch (const Error& e) {
+    if (e.status != ORDA_ERR_OOM) throw;   // no room: the product runs unsplit
+  }
 }
 
 // ms_dev: the deferred-mean scale on the device (LabelStatus::mean_scale).

@@ -1875,12 +1875,6 @@ struct SplitPlan {
   int64_t len, ldp, stride, bytes;
 };
 
-// Split K when the tiles cannot fill the CUs: about 256 workgroups in all,
-// each split at least 128 elements of K (a multiple of 64), at most 64
-// splits and 256 MB of partials. (At BT=256, H=512, V=8192 fp32 a 512
-// minimum left grad_hidden on 64 workgroups and grad_W unsplit: 0.152 and
-// 0.141 ms against 0.072 and 0.070 ms with 128, reductions included; 64
-// measured the same as 128.)
 // Shared-round blocks (map_tile) for a product with share_rounds set: xn in
 // {1, 2, 4, 8} dividing the N-tiles, b = Nt/xn, a = 32/b; the most tiles per
 // XCD (at least 24), then the fewest operand strips per stage (a + b), then
@@ -1940,28 +1934,60 @@ void set_band_blocks(GemmArgs& g) {
   g.sh_xn = 1;
 }
 
+// What a product's tiles cost, in us on the 256 CUs (one workgroup each): a
+// round of them takes kRoundUs for filling the ring and storing a tile, and
+// stage_us for every 32 elements of K (measured over bf16 products of 64 to
+// 2000 rows, widths of 256 to 4096 and vocabularies of 8000 to 128256: 0.7 us a
+// stage, 9 % off; six plane products a stage; the fp32 MFMA a sixteenth of the
+// bf16 rate). Split over K, a product also writes and reads its partials
+// (kPartUs a byte, 4 TB/s).
+constexpr double kRoundUs = 8.0, kPartUs = 0.25e-6;
+double stage_us(const GemmArgs& g) { return g.plane_a > 0 ? 4.2 : g.in_type == DType::BF16 ? 0.7 : 7.3; }
+double rounds_us(const GemmArgs& g, int64_t tiles, int64_t len) {
+  return static_cast<double>((tiles + 255) / 256) * (static_cast<double>(len) / 32 * stage_us(g) + kRoundUs);
+}
+int64_t tile_count(const GemmArgs& g) {
+  return ((g.M + kTile - 1) / kTile) * ((g.N + kTile - 1) / kTile) * g.nprob;
+}
+
+// Split K where the tiles leave CUs idle, in one round or in a last one: the
+// split of least cost by the measure above, each part at least 128 elements of
+// K (a multiple of 64), at most ceil(256 / tiles) parts of fewer than 192
+// tiles, at most 8 of more (128 of one or two), and 256 MB of partials. (A fixed
+// ceil(256 / tiles) parts put 12 tiles, as grad_hidden at 300 x 768, on 264
+// workgroups, two rounds: grad_hidden measured 1.3 to 1.65 times slower at
+// such counts: 300 x 768 x 50257 128 us against 91, 2000 x 1536 x 128256 929
+// against 594.)
 SplitPlan plan_split(const GemmArgs& g) {
   SplitPlan sp{1, g.K, 0, 0, 0};
   if (g.epi == GemmEpilogue::Logits || g.M <= 0 || g.N <= 0 || g.K <= 0) return sp;
-  const int64_t tiles = ((g.M + kTile - 1) / kTile) * ((g.N + kTile - 1) / kTile) * g.nprob;
-  if (tiles >= 192) return sp;
-  int64_t s = (256 + tiles - 1) / tiles;
-  const int64_t by_k = g.K / 128;
-  if (s > by_k) s = by_k;
-  if (s > 64) s = 64;
+  const int64_t tiles = tile_count(g);
   const int64_t per_split = g.nprob * (g.c_trans ? g.N * ((g.M + 3) / 4 * 4) : g.M * ((g.N + 3) / 4 * 4)) * 4;
-  if (s > (int64_t{256} << 20) / per_split) s = (int64_t{256} << 20) / per_split;
-  if (s <= 1) return sp;
-  const int64_t len = ((g.K + s - 1) / s + 63) / 64 * 64;
-  s = (g.K + len - 1) / len;
-  if (s <= 1) return sp;
-  sp.splits = static_cast<int>(s);
-  sp.len = len;
+  int64_t most = tiles < 192 ? (256 + tiles - 1) / tiles : 8;
+  const int64_t by_k = g.K / 128, by_ws = (int64_t{256} << 20) / per_split;
+  if (most > by_k) most = by_k;
+  if (most > 128) most = 128;
+  if (most > by_ws) most = by_ws;
+  double best = rounds_us(g, tiles, g.K);
+  for (int64_t i = 2; i <= most; ++i) {
+    const int64_t len = ((g.K + i - 1) / i + 63) / 64 * 64, n = (g.K + len - 1) / len;
+    if (n <= 1) break;
+    const double us = rounds_us(g, tiles * n, len) + 2 * kPartUs * static_cast<double>(n * per_split);
+    if (us < best) {
+      best = us;
+      sp.splits = static_cast<int>(n);
+      sp.len = len;
+    }
+  }
+  if (sp.splits <= 1) return sp;
   // partials in C's orientation: rows x ldp, transposed when C is
   sp.ldp = ((g.c_trans ? g.M : g.N) + 3) / 4 * 4;
   sp.stride = g.nprob * (g.c_trans ? g.N : g.M) * sp.ldp;
-  sp.bytes = s * sp.stride * 4;
+  sp.bytes = sp.splits * sp.stride * 4;
   return sp;
+}
+double split_us(const GemmArgs& g, const SplitPlan& sp) {
+  return rounds_us(g, tile_count(g) * sp.splits, sp.len) + 2 * kPartUs * static_cast<double>(sp.bytes);
 }
 
 // ------------------------------------------------------- small fp32 products
@@ -2345,12 +2371,12 @@ GemmArgs sub_product(const GemmArgs& g, int64_t r0, int64_t r1, int64_t c0, int6
 // round of fewer than 192 workgroups (for 256 CUs) runs its whole rounds as
 // one launch and the rest as a second product, which then splits K over the
 // CUs (plan_split): the tail costs a fraction of a round instead of a whole
-// one. The whole rounds must end on a tile boundary: in the columns (256 x
-// rounds divisible by the M-tiles, e.g. grad_W computed transposed with its
-// 16 M-tiles at H = 4096), else in the rows of every problem (by the
-// N-tiles x problems, e.g. grad_hidden at H = 4096 and BT = 5000); and the
-// tail must split. Returns the split point (a multiple of 256) as a column
-// (cols = true) or a row, or 0 when the product runs as one launch.
+// one. The whole rounds take the column tiles (e.g. grad_W computed
+// transposed), else, where they end on a tile boundary, the rows of every
+// problem (by the N-tiles x problems, e.g. grad_hidden at H = 4096 and BT =
+// 5000) that fit them; the tail must split, and cost less than the product in
+// one launch, split or not. Returns the split point (a multiple of 256) as a
+// column (cols = true) or a row, or 0 when the product runs as one launch.
 struct TailSplit {
   int64_t at;
   bool cols;
@@ -2362,13 +2388,18 @@ TailSplit plan_tail(const GemmArgs& g) {
   const int64_t Mv = Mt * g.nprob;
   const int64_t T = Mv * Nt, q = T / 256, r = T % 256;
   if (q < 1 || r == 0 || r >= 192) return none;
-  if ((256 * q) % Mv == 0) {
-    const int64_t n0 = 256 * q / Mv * kTile;
-    if (n0 < g.N && plan_split(sub_product(g, 0, g.M, n0, g.N)).splits > 1) return {n0, true};
-  }
+  const SplitPlan whole = plan_split(g);
+  const double one = whole.splits > 1 ? split_us(g, whole) : rounds_us(g, T, g.K);
+  const double rounds = q * (rounds_us(g, 1, g.K));
+  auto pays = [&](const GemmArgs& tail) {
+    const SplitPlan sp = plan_split(tail);
+    return sp.splits > 1 && rounds + split_us(tail, sp) < one;
+  };
+  const int64_t n0 = 256 * q / Mv * kTile;
+  if (n0 > 0 && n0 < g.N && pays(sub_product(g, 0, g.M, n0, g.N))) return {n0, true};
   if ((256 * q) % (Nt * g.nprob) == 0) {
     const int64_t m0 = 256 * q / (Nt * g.nprob) * kTile;
-    if (m0 < g.M && plan_split(sub_product(g, m0, g.M, 0, g.N)).splits > 1) return {m0, false};
+    if (m0 < g.M && pays(sub_product(g, m0, g.M, 0, g.N))) return {m0, false};
   }
   return none;
 }
