@@ -291,6 +291,22 @@ int32_t orda_quant_rows_int8(orda_ctx *ctx, const orda_tensor *m, const int64_t 
                              orda_tensor *out, orda_tensor *codes, orda_tensor *scales, char *err,
                              size_t err_len);
 
+/* ---- gradients of a scaled loss ------------------------------------------- */
+/* dst = scale * src, src float32, dst float32 (may be src) or bfloat16, both n
+ * contiguous elements on the device; scale one float32 on the device. The
+ * backward of a loss whose gradients orda_distillation_loss has returned: one
+ * launch for up to 4 of them, queued on hip_stream (NULL: the null stream) of
+ * `device` without waiting for it. No counterpart in the reference. */
+typedef struct {
+    const float *src;
+    void *dst;
+    int64_t n;
+    int32_t dst_dtype;   /* ORDA_F32 or ORDA_BF16 */
+} orda_scaled_gradient;
+int32_t orda_scale_gradients(int32_t device, void *hip_stream, const float *scale,
+                             const orda_scaled_gradient *gradients, int32_t count, char *err,
+                             size_t err_len);
+
 #ifdef __cplusplus
 }
 #endif

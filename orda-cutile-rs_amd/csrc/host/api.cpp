@@ -1845,4 +1845,27 @@ int32_t orda_quant_rows_int8(orda_ctx* ctx, const orda_tensor* m, const int64_t*
   }
 }
 
+int32_t orda_scale_gradients(int32_t device, void* hip_stream, const float* scale,
+                             const orda_scaled_gradient* gradients, int32_t count, char* err,
+                             size_t err_len) {
+  try {
+    if (count < 0 || count > 4) fail(ORDA_ERR_INVALID, "between 0 and 4 gradients, got %d", count);
+    if (count > 0 && (!gradients || !scale)) fail(ORDA_ERR_INVALID, "null argument");
+    orda::ScaleArgs a{};
+    a.count = count;
+    a.scale = scale;
+    for (int i = 0; i < count; ++i) {
+      const orda_scaled_gradient& g = gradients[i];
+      if (g.n < 0 || (g.n > 0 && (!g.src || !g.dst))) fail(ORDA_ERR_INVALID, "gradient %d has no data", i);
+      a.part[i] = {g.src, g.dst, g.n, to_dtype(g.dst_dtype, "a scaled gradient") == DType::BF16, 0};
+    }
+    hip_check(hipSetDevice(device), "hipSetDevice");
+    hip_check(orda::launch_scale(a, static_cast<hipStream_t>(hip_stream)), "scale gradients");
+    return ORDA_OK;
+  } catch (const Error& e) {
+    copy_err(e, err, err_len);
+    return e.status;
+  }
+}
+
 }  // extern "C"

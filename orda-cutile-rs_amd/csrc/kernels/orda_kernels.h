@@ -322,6 +322,20 @@ struct QuantArgs {
 };
 hipError_t launch_quant(const QuantArgs& a, hipStream_t stream);
 
+// dst = *scale * src for up to 4 contiguous arrays in one launch.
+struct ScaleArgs {
+  struct Part {
+    const float* src;
+    void* dst;
+    int64_t n;
+    bool bf16;              // dst's type: bf16, else fp32
+    int64_t block0;         // set by launch_scale: the part's first block
+  } part[4];
+  int count;
+  const float* scale;
+};
+hipError_t launch_scale(ScaleArgs a, hipStream_t stream);
+
 // Label validation on the device (src/api.rs:125-133) and the deferred-mean
 // scale (src/api.rs:225-230): n_valid counts labels != ignore_index; the
 // first label (lowest index) that is neither ignore_index nor in [0, v) is

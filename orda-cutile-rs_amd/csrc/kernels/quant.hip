@@ -310,6 +310,48 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* src, int6
   for (int q = 0; q < 3; ++q) *reinterpret_cast<u4*>(d + q * plane) = w[q];
 }
 
+// Gradients scaled by a device value into their inputs' type: 8 elements a
+// thread, 16-byte accesses where the arrays start on 16 bytes. Bound by HBM:
+// fp32 to bf16, 38.6e6 elements 43 us (5.4 TB/s) against 52 + 45 us for a
+// multiplication and a conversion by themselves.
+constexpr int kScaleBlock = 256 * 8;
+__global__ __launch_bounds__(256) void scale_kernel(ScaleArgs a) {
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (i < a.count && static_cast<int64_t>(blockIdx.x) >= a.part[i].block0) p = i;
+  const ScaleArgs::Part& q = a.part[p];
+  const int64_t j = (blockIdx.x - q.block0) * kScaleBlock + threadIdx.x * 8;
+  if (j >= q.n) return;
+  const float k = *a.scale;
+  const bool vec = j + 8 <= q.n && (reinterpret_cast<uintptr_t>(q.src) & 15) == 0 &&
+                   (reinterpret_cast<uintptr_t>(q.dst) & 15) == 0;
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  if (vec) {
+    const f32x4* s = reinterpret_cast<const f32x4*>(q.src + j);
+    const f32x4 x = k * s[0], y = k * s[1];
+    if (q.bf16) {
+      bf16x8 w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        w[i] = static_cast<__bf16>(x[i]);
+        w[4 + i] = static_cast<__bf16>(y[i]);
+      }
+      *reinterpret_cast<bf16x8*>(static_cast<__bf16*>(q.dst) + j) = w;
+    } else {
+      f32x4* d = reinterpret_cast<f32x4*>(static_cast<float*>(q.dst) + j);
+      d[0] = x;
+      d[1] = y;
+    }
+    return;
+  }
+  for (int64_t i = j; i < j + 8 && i < q.n; ++i) {
+    const float x = k * q.src[i];
+    if (q.bf16) static_cast<__bf16*>(q.dst)[i] = static_cast<__bf16>(x);
+    else static_cast<float*>(q.dst)[i] = x;
+  }
+}
+
 unsigned grid_for(int64_t total) {
   int64_t b = (total + 255) / 256;
   if (b > 65536) b = 65536;
@@ -331,6 +373,19 @@ hipError_t launch_quant(const QuantArgs& a, hipStream_t s) {
   else if (vec && a.cols <= 4 * per) hipLaunchKernelGGL(quant_vec_kernel<4>, grid, block, 0, s, a);
   else if (vec && a.cols <= 8 * per) hipLaunchKernelGGL(quant_vec_kernel<8>, grid, block, 0, s, a);
   else hipLaunchKernelGGL(quant_kernel, grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_scale(ScaleArgs a, hipStream_t s) {
+  if (a.count < 0 || a.count > 4) return hipErrorInvalidValue;
+  int64_t blocks = 0;
+  for (int i = 0; i < a.count; ++i) {
+    a.part[i].block0 = blocks;
+    blocks += (a.part[i].n + kScaleBlock - 1) / kScaleBlock;
+  }
+  if (blocks == 0) return hipSuccess;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(scale_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

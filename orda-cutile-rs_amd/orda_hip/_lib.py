@@ -71,6 +71,11 @@ class LossOutputC(C.Structure):
                 ("quant_codes", Tensor), ("quant_scales", Tensor)]
 
 
+class ScaledGradient(C.Structure):
+    _fields_ = [("src", C.c_void_p), ("dst", C.c_void_p), ("n", C.c_int64),
+                ("dst_dtype", C.c_int32)]
+
+
 # (name, restype, argtypes) for every entry point of include/orda/orda.h.
 SIGNATURES = [
     ("orda_abi_version", C.c_int32, []),
@@ -115,6 +120,9 @@ SIGNATURES = [
      [C.c_void_p, C.POINTER(Tensor), C.c_void_p, C.c_int64, C.c_int32, C.c_int64, C.c_int32,
       C.c_uint64, C.c_float, C.POINTER(Tensor), C.POINTER(Tensor), C.POINTER(Tensor),
       C.c_char_p, C.c_size_t]),
+    ("orda_scale_gradients", C.c_int32,
+     [C.c_int32, C.c_void_p, C.c_void_p, C.POINTER(ScaledGradient), C.c_int32, C.c_char_p,
+      C.c_size_t]),
 ]
 
 _lib = None

@@ -15,12 +15,43 @@ returned in its input's dtype.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Optional, Tuple
 
 import torch
 
 from . import Context, distillation_loss
-from .types import LossOptions, Teacher, TeacherMode
+from . import _lib as L
+from .types import LossOptions, OrdaError, Teacher, TeacherMode
+
+
+def _plain(t):
+    """A CUDA tensor with memory of its own (not one batched by vmap, as
+    torch.autograd.grad's is_grads_batched makes, nor another wrapper)."""
+    try:
+        return t.is_cuda and type(t) is torch.Tensor and (t.data_ptr() != 0 or t.numel() == 0)
+    except RuntimeError:
+        return False
+
+
+def _scaled(grads, dtypes, g_loss):
+    """[g_loss * g as dtype] on the current stream, in one launch
+    (orda_scale_gradients); a float32 gradient is scaled in place."""
+    dev = grads[0].device
+    out, parts = [], (L.ScaledGradient * len(grads))()
+    scale = g_loss.to(torch.float32)
+    p = scale.data_ptr()
+    for part, g, dt in zip(parts, grads, dtypes):
+        d = g if dt == torch.float32 else torch.empty_like(g, dtype=dt)
+        part.src, part.dst, part.n = g.data_ptr(), d.data_ptr(), g.numel()
+        part.dst_dtype = L.F32 if dt == torch.float32 else L.BF16
+        out.append(d)
+    err = ctypes.create_string_buffer(512)
+    rc = L.load().orda_scale_gradients(dev.index or 0, torch.cuda.current_stream(dev).cuda_stream, p,
+                                       parts, len(grads), err, 512)
+    if rc != L.ORDA_OK:
+        raise OrdaError(err.value.decode(), rc)
+    return out
 
 
 class DistillCEFunction(torch.autograd.Function):
@@ -42,21 +73,27 @@ class DistillCEFunction(torch.autograd.Function):
                             for t in (student_hidden, weight, teacher_hidden, teacher_weight))
         fctx.chunk_plan = out.chunk_plan
         dev = student_hidden.device
-        loss = torch.tensor(out.loss, dtype=torch.float32, device=dev)
+        # neither waits for the device: a fill, and a copy from pinned memory
+        loss = torch.full((), out.loss, dtype=torch.float32, device=dev)
         comps = torch.tensor([out.student_ce, out.teacher_ce, out.kl], dtype=torch.float32,
-                             device=dev)
+                             pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
         fctx.mark_non_differentiable(comps)
         return loss, comps
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(fctx, g_loss, g_comps):
-        res = []
-        for i, (g, dt) in enumerate(zip(fctx.grads, fctx.dtypes)):
-            if g is None or dt is None or not fctx.needs_input_grad[i]:
-                res.append(None)
+        res = [None] * 4
+        want = [i for i, (g, dt) in enumerate(zip(fctx.grads, fctx.dtypes))
+                if g is not None and dt is not None and fctx.needs_input_grad[i]]
+        if want:
+            grads, dtypes = [fctx.grads[i] for i in want], [fctx.dtypes[i] for i in want]
+            if _plain(g_loss) and all(_plain(g) and g.is_contiguous() for g in grads):
+                scaled = _scaled(grads, dtypes, g_loss)
             else:
-                res.append((g * g_loss.to(g.dtype)).to(dt))
+                scaled = [(g * g_loss.to(g.dtype)).to(dt) for g, dt in zip(grads, dtypes)]
+            for i, g in zip(want, scaled):
+                res[i] = g
         fctx.grads = None
         return (*res, None, None, None, None, None)
 
