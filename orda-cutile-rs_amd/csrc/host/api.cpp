@@ -548,7 +548,7 @@ bool teacher_logits_direct(const LossPlan& P, const Inputs& in) {
 
 // Whether an fp32 call runs its products over three-plane operands
 // (GemmArgs::plane_a) instead of the fp32 MFMA: six bf16 products take the
-// place of one fp32 product, at 240 against 133 TFLOP/s of fp32 work, and the
+// place of one fp32 product, at 265 against 133 TFLOP/s of fp32 work, and the
 // gradients come out nearer to a float64 result (2.2e-6 against 3.2e-6 for
 // the hidden rows, 6.1e-7 against 9.8e-7 for the weights at BT=2048, H=4096,
 // V=32000). The planes are made by a pass over the weights and one over the
@@ -558,8 +558,8 @@ bool teacher_logits_direct(const LossPlan& P, const Inputs& in) {
 // 155 / 183, 1.3e10 (Tied 256 x 512 x 8192) 223 / 226, 2.5e10 (Precomputed
 // 64 x 2048 x 32000) 740 / 614; as the products now go, 2.6e10 (Tied 2048 x
 // 256 x 4096) 353 / 316, 2.5e10 (Tied 16 x 4096 x 32000) 1955 / 1935, 3.2e12
-// (Tied 2048 x 4096 x 32000) 24.2 / 18.2 ms, 4.8e12 (Separate 4096 x (2048,
-// 4096) x 32000) 36.3 / 20.4 ms.
+// (Tied 2048 x 4096 x 32000) 24.2 / 16.5 ms, 4.8e12 (Separate 4096 x (2048,
+// 4096) x 32000) 36.3 / 18.3 ms.
 bool use_planes3(const LossPlan& P) {
   if (P.dt != orda::DType::F32 || P.h < 64 || P.v < 64) return false;
   const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;

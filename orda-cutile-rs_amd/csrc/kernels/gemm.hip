@@ -336,6 +336,7 @@ struct PairLoader {
       goff[t] = static_cast<uint32_t>((rr - b0) * ldb + q * 16);
     }
   }
+  __device__ __forceinline__ const unsigned char* src(int pair) const { return base + pair * step; }
 };
 
 // ---------------------------------------------------------------- fragments
@@ -519,26 +520,40 @@ __device__ __forceinline__ void mfma_step(f32x4 (&acc)[kFrag][kFrag], const u32x
 
 // fp32 products on the bf16 matrix units (GemmArgs::plane_a): each operand is
 // stored as three bf16 planes h + m + l (split3.h), which hold every bit of
-// an fp32 value, and a product of two such operands is the sum of the six
-// plane products hl, hm, hh, mm, mh, lh; the three left out (ml, lm, ll) lie
-// below 2^-26 of |a·b| each, under half an ulp of one fp32 product. The bf16
-// loops walk K in pairs of stages (64 elements): pair p is plane product p % 6
-// of K block p / 6.
-constexpr uint32_t kPlanesA = 0 << 0 | 0 << 2 | 0 << 4 | 1 << 6 | 1 << 8 | 2 << 10;
-constexpr uint32_t kPlanesB = 2 << 0 | 1 << 2 | 0 << 4 | 1 << 6 | 0 << 8 | 0 << 10;
-constexpr int kPlaneProducts = 6;
-
-// Source of stage pair `pair` of an operand whose pairs lie `step` bytes apart:
-// with three planes, plane (planes >> 2q) & 3 (`plane` elements apart) of K
-// block pair / 6, q = pair % 6.
-template <bool P3, uint32_t PLANES>
-__device__ __forceinline__ const unsigned char* pair_src(const unsigned char* base, int pair, int64_t step,
-                                                         int64_t plane) {
-  if constexpr (!P3) return base + pair * step;
-  const uint32_t kb = static_cast<uint32_t>(pair) / kPlaneProducts;
-  const uint32_t q = static_cast<uint32_t>(pair) - kb * kPlaneProducts;
-  return base + kb * step + static_cast<int64_t>((PLANES >> (2 * q)) & 3) * (2 * plane);
+// an fp32 value, and a product of two such operands is the sum of six plane
+// products; the three left out (ml, lm, ll) lie below 2^-26 of |a·b| each,
+// under half an ulp of one fp32 product. A K block is 64 elements, 12 stages of
+// MFMAs: the products in the order hl, hm, mm, mh, hh, lh (A's plane first), each
+// of which changes one operand, and the two 32-element halves of a product in
+// an order that ends on the half the next one starts with. So each plane is
+// moved into LDS once a block (six moves of 32 KB where a product at a time
+// takes twelve), and a stage reads only the fragments that changed. Bound by
+// the matrix units under the chip's power limit: 265 TFLOP/s of fp32 work
+// (1.59 PFLOP/s in bf16) at Precomputed 4096 x 4096 x 65536, against 240 with
+// a move for every product; where in an iteration the moves and reads sit
+// changes it by under 1 %.
+struct PlaneStage {
+  int pa, pb;       // planes: 0 h, 1 m, 2 l
+  int half;
+  bool ra, rb;      // fragments of A / B differ from the previous stage's
+};
+constexpr int kPlaneStages = 12;
+constexpr PlaneStage kPlaneSeq[kPlaneStages] = {
+    {0, 2, 0, true, true},  {0, 2, 1, true, true},   // hl
+    {0, 1, 1, false, true}, {0, 1, 0, true, true},   // hm
+    {1, 1, 0, true, false}, {1, 1, 1, true, true},   // mm
+    {1, 0, 1, false, true}, {1, 0, 0, true, true},   // mh
+    {0, 0, 0, true, false}, {0, 0, 1, true, true},   // hh
+    {2, 0, 1, true, true},  {2, 0, 0, true, true},   // lh (B again: an even number of reads)
+};
+// Fragment register set (0 or 1) that holds stage i's operand, the sets taking
+// turns with every read; both operands are read an even number of times.
+constexpr int plane_set(int i, bool a) {
+  int n = 0;
+  for (int k = 1; k <= i; ++k) n += (a ? kPlaneSeq[k].ra : kPlaneSeq[k].rb) ? 1 : 0;
+  return n & 1;
 }
+static_assert(plane_set(11, true) == 1 && plane_set(11, false) == 1, "stage 12 is stage 0's set again");
 
 struct TileCoord {
   int p, m0, n0, ntile;
@@ -612,7 +627,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
   constexpr bool kLogitsEpi = EPI == GemmEpilogue::Logits || kTeacherEpi;
   // Ring layout: A tiles of slots 0-3, then B tiles of slots 0-3 (16 KB
   // each), so every slot offset fits a DS instruction's immediate.
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kRing * kStageBytes + kEpiLds];
+  // (Three-plane operands: two slots of 32 KB for B's planes, then three for
+  // A's, all of the CU's LDS; the epilogue scratch lies in them.)
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[P3 ? 5 * 2 * kOpBytes : kRing * kStageBytes + kEpiLds];
   unsigned char* const epi = smem + kRing * kStageBytes;
   auto tileA = [&](int s) -> unsigned char* { return smem + s * kOpBytes; };
   auto tileB = [&](int s) -> unsigned char* { return smem + (kRing + s) * kOpBytes; };
@@ -711,7 +728,173 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
     __builtin_amdgcn_sched_barrier(0);
     mfma_prime();
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (kPaired) {
+    if constexpr (P3) {
+      // Iteration i computes stage i from registers and reads stage i+1's
+      // fragments. A plane whose last stage is L was last read in iteration
+      // L-1, so its slot is free from the barrier that opens iteration L (or
+      // a later one) on; one whose first stage is F must have landed by the
+      // barrier that opens F-1. With slots S0-S2 of A (h, m, l of block b in
+      // b, b+1, b+2 mod 3) and T0, T1 of B (l, m, h in t, 1-t, t, t = b mod 2):
+      //   iteration   moves (8 transfers a thread)   waits at its barrier for
+      //   0           A m                            -
+      //   1           -                              B m   (A m in flight)
+      //   2           B h                            -
+      //   3           -                              A m   (B h in flight)
+      //   5           A l                            B h
+      //   7           B l of the next block          -
+      //   8           A h of the next block          - (barrier: A m was read)
+      //   9           -                              A l   (both in flight)
+      //   11          B m of the next block          A h, B l
+      // Past the last block the moves re-read it, into slots nobody reads.
+      PairLoader<AK> pa;
+      PairLoader<BK> pb;
+      pa.init(pr.a, g.lda, g.M, tc.m0, wave, lane);
+      pb.init(pr.b, g.ldb, g.N, tc.n0, wave, lane);
+      const int nkb = static_cast<int>(Kl / 64);
+      FragReader<AK, AK> f3a;
+      FragReader<BK, BK> f3b;
+      f3a.init(lds0 + 4 * kOpBytes, wm * 128, lane);
+      f3b.init(lds0, wn * 128, lane);
+      constexpr uint32_t kSlot = 2 * kOpBytes;
+      uint32_t sh = 0, sm = kSlot, sl = 2 * kSlot;   // slot offsets of A's planes
+      uint32_t tb = 0;                               // slot offset of B's h and l
+      auto move = [&](auto a_c, int x, uint64_t src, uint32_t slot) {
+        constexpr bool kA = decltype(a_c)::value != 0;
+        const uint32_t m0 = m0wave + (kA ? 4 * kOpBytes : 0) + slot;
+        const auto& l = [&]() -> const auto& { if constexpr (kA) return pa; else return pb; }();
+        switch (x) {
+          case 0: dma16_at<0 * 4096>(src, l.goff[0], m0); break;
+          case 1: dma16_at<1 * 4096>(src, l.goff[1], m0); break;
+          case 2: dma16_at<2 * 4096>(src, l.goff[2], m0); break;
+          case 3: dma16_at<3 * 4096>(src, l.goff[3], m0); break;
+          case 4: dma16_at<4 * 4096>(src, l.goff[4], m0); break;
+          case 5: dma16_at<5 * 4096>(src, l.goff[5], m0); break;
+          case 6: dma16_at<6 * 4096>(src, l.goff[6], m0); break;
+          default: dma16_at<7 * 4096>(src, l.goff[7], m0); break;
+        }
+      };
+      auto src_a = [&](int kb, int plane) {
+        return uniform64(pa.base + kb * pa.step + static_cast<int64_t>(plane) * 2 * g.plane_a);
+      };
+      auto src_b = [&](int kb, int plane) {
+        return uniform64(pb.base + kb * pb.step + static_cast<int64_t>(plane) * 2 * g.plane_b);
+      };
+      constexpr int kOpsA = FragReader<AK, AK>::kOps, kOpsB = FragReader<BK, BK>::kOps;
+      // Operation o of reading half HALF of the plane in A's slot `slot`, or of
+      // the B plane f3b points to.
+      auto read_a = [&](auto half_c, int o, uint32_t addr, u32x4 (&r)[kFrag]) {
+        r[o] = *(const lds_u32x4*)(static_cast<uintptr_t>(addr + o * 2048));
+      };
+      auto read_b = [&](auto half_c, int o, u32x4 (&r)[kFrag]) {
+        constexpr int kHalf = decltype(half_c)::value;
+        if constexpr (BK) {
+          r[o] = *(const lds_u32x4*)(static_cast<uintptr_t>(f3b.addr[kHalf] + o * 2048));
+        } else {
+          f3b.template read_op<kHalf>(o, r);
+        }
+      };
+      auto iter = [&](auto i_c, int kb) {
+        constexpr int I = decltype(i_c)::value;
+        constexpr int N = (I + 1) % kPlaneStages;
+        constexpr PlaneStage nx = kPlaneSeq[N];
+        constexpr int kSetA = plane_set(I, true), kSetB = plane_set(I, false);
+        constexpr int kNextA = nx.ra ? 1 - kSetA : kSetA, kNextB = nx.rb ? 1 - kSetB : kSetB;
+        constexpr bool kBarrier = I == 1 || I == 3 || I == 5 || I == 8 || I == 9 || I == 11;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kBarrier) {
+          // transfers that may still be in flight
+          constexpr int kFly = I == 1 || I == 3 || I == 8 ? 8 : I == 9 ? 16 : 0;
+          if constexpr (I == 8) __builtin_amdgcn_s_waitcnt(kWaitLds);
+          else __builtin_amdgcn_s_waitcnt(vm_wait(kFly));
+          __builtin_amdgcn_s_barrier();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int nxt = kb + 1 < nkb ? kb + 1 : kb;
+        constexpr bool kMoveA = I == 0 || I == 5 || I == 8, kMoveB = I == 2 || I == 7 || I == 11;
+        uint64_t src = 0;
+        uint32_t slot = 0;
+        if constexpr (I == 0) src = src_a(kb, 1), slot = sm;
+        if constexpr (I == 5) src = src_a(kb, 2), slot = sl;
+        if constexpr (I == 8) src = src_a(nxt, 0), slot = sm;
+        if constexpr (I == 2) src = src_b(kb, 0), slot = tb;
+        if constexpr (I == 7) src = src_b(nxt, 2), slot = kSlot - tb;
+        if constexpr (I == 11) src = src_b(nxt, 1), slot = tb;
+        // stage I+1's addresses (the next block's h is where m was)
+        uint32_t aslot = nx.pa == 0 ? sh : nx.pa == 1 ? sm : sl;
+        if constexpr (N == 0) aslot = sm;
+        const uint32_t aaddr = f3a.addr[nx.half] + aslot;
+        if constexpr (N == 2 || N == 6 || N == 0) {   // B's other slot
+          const uint32_t d = N == 2 ? kSlot - 2 * tb : 2 * tb - kSlot;
+          const uint32_t dd = N == 0 ? kSlot - 2 * tb : d;
+#pragma unroll
+          for (int o = 0; o < (BK ? 2 : 2 * kFrag); ++o) f3b.addr[o] += dd;
+        }
+        constexpr int kReadA = nx.ra ? kOpsA : 0, kReadB = nx.rb ? kOpsB : 0;
+        constexpr int kReads = kReadA + kReadB;
+#pragma unroll
+        for (int pr = 0; pr < 32; ++pr) {
+          if constexpr (kMoveA) {
+            if (pr >= 2 && pr < 26 && (pr - 2) % 3 == 0) move(SlotC<1>{}, (pr - 2) / 3, src, slot);
+          }
+          if constexpr (kMoveB) {
+            if (pr >= 2 && pr < 26 && (pr - 2) % 3 == 0) move(SlotC<0>{}, (pr - 2) / 3, src, slot);
+          }
+#pragma unroll
+          for (int o = 0; o < kReads; ++o) {
+            if ((o * 28) / kReads != pr) continue;
+            if (o < kReadA) read_a(SlotC<nx.half>{}, o, aaddr, ra[kNextA]);
+            else read_b(SlotC<nx.half>{}, o - kReadA, rb[kNextB]);
+          }
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const int mm = 2 * pr + q;
+            if constexpr (kSwapAB)
+              mfma_bf16(acc[mm & 7][mm >> 3], rb[kSetB][mm >> 3], ra[kSetA][mm & 7]);
+            else
+              mfma_bf16(acc[mm >> 3][mm & 7], ra[kSetA][mm >> 3], rb[kSetB][mm & 7]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if (nkb > 0) {
+        uint64_t src = src_b(0, 2);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) move(SlotC<0>{}, x, src, tb);
+        src = src_a(0, 0);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) move(SlotC<1>{}, x, src, sh);
+        src = src_b(0, 1);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) move(SlotC<0>{}, x, src, kSlot - tb);
+        __builtin_amdgcn_s_waitcnt(vm_wait(8));
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int o = 0; o < kOpsA; ++o) read_a(SlotC<0>{}, o, f3a.addr[0] + sh, ra[0]);
+#pragma unroll
+        for (int o = 0; o < kOpsB; ++o) read_b(SlotC<0>{}, o, rb[0]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      for (int kb = 0; kb < nkb; ++kb) {
+        iter(SlotC<0>{}, kb);
+        iter(SlotC<1>{}, kb);
+        iter(SlotC<2>{}, kb);
+        iter(SlotC<3>{}, kb);
+        iter(SlotC<4>{}, kb);
+        iter(SlotC<5>{}, kb);
+        iter(SlotC<6>{}, kb);
+        iter(SlotC<7>{}, kb);
+        iter(SlotC<8>{}, kb);
+        iter(SlotC<9>{}, kb);
+        iter(SlotC<10>{}, kb);
+        iter(SlotC<11>{}, kb);
+        const uint32_t f = sh;   // next: h where m was, m where l was, l where h was
+        sh = sm;
+        sm = sl;
+        sl = f;
+        tb = kSlot - tb;
+        mfma_prime();   // also for accumulators the compiler copies out at the loop's exit
+      }
+    } else if constexpr (kPaired) {
       // The ring holds two stage pairs (64 elements of K each): pair p sits in
       // double slot p%2, stage s in half s%2 of double slot (s/2)%2.
       //
@@ -737,9 +920,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       else
         pa.init(pr.a, g.lda, g.M, tc.m0, wave, lane);
       pb.init(pr.b, g.ldb, g.N, tc.n0, wave, lane);
-      const int np = P3 ? static_cast<int>(Kl / 64) * kPlaneProducts : nkf / 2;
-      auto src_a = [&](int pair) { return pair_src<P3, kPlanesA>(pa.base, pair, pa.step, g.plane_a); };
-      auto src_b = [&](int pair) { return pair_src<P3, kPlanesB>(pb.base, pair, pb.step, g.plane_b); };
+      const int np = nkf / 2;
       // Transfer x (0-7 A, 8-15 B) of a pair's DMA into double slot D, from
       // the pair's sources sa, sb.
       auto dma_op = [&](auto d_c, int x, uint64_t sa, uint64_t sb) {
@@ -766,12 +947,12 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       };
       if (np > 0) {
         {
-          const uint64_t sa = uniform64(src_a(0)), sb = uniform64(src_b(0));
+          const uint64_t sa = uniform64(pa.src(0)), sb = uniform64(pb.src(0));
   #pragma unroll
           for (int x = 0; x < 16; ++x) dma_op(SlotC<0>{}, x, sa, sb);
         }
         if (np > 1) {
-          const uint64_t sa = uniform64(src_a(1)), sb = uniform64(src_b(1));
+          const uint64_t sa = uniform64(pa.src(1)), sb = uniform64(pb.src(1));
   #pragma unroll
           for (int x = 0; x < 16; ++x) dma_op(SlotC<1>{}, x, sa, sb);
           __builtin_amdgcn_s_waitcnt(vm_wait(16));   // pair 0 landed
@@ -817,8 +998,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
             // overlaps MFMAs.
             const int p = (st >> 1) + 2;
             const int nxt = p < np ? p : np - 1;
-            sa = uniform64(src_a(nxt));
-            sb = uniform64(src_b(nxt));
+            sa = uniform64(pa.src(nxt));
+            sb = uniform64(pb.src(nxt));
           }
           if (!kOdd && pr == kMid) {
             __builtin_amdgcn_sched_barrier(0);
@@ -878,20 +1059,12 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       // followed by exactly 16 (s even) or 4 (s odd) younger ones. Past the
       // last pair the DMAs re-read stage 0 (B) or the last pair (A) into
       // slots nobody reads again.
-      const int np = P3 ? static_cast<int>(Kl / 64) * kPlaneProducts : nkf / 2;
+      const int np = nkf / 2;
       const int ns = 2 * np;
       PairLoader<AK> pa;
       pa.init(pr.a, g.lda, g.M, tc.m0, wave, lane);
       LoaderB lb;
       init_b(lb);
-      auto src_a = [&](int pair) { return pair_src<P3, kPlanesA>(pa.base, pair, pa.step, g.plane_a); };
-      // B stage st: half st % 2 of pair st / 2's 64 K rows
-      auto src_b = [&](int st) {
-        if constexpr (!P3) return lb.stage_src(st);
-        else
-          return pair_src<true, kPlanesB>(lb.base, st >> 1, 64 * lb.ld_bytes, g.plane_b) +
-                 (st & 1) * 32 * lb.ld_bytes;
-      };
       // Transfer x (0-7) of an A pair into double slot D.
       auto dma_a = [&](auto d_c, int x, uint64_t sa) {
         constexpr int MA = decltype(d_c)::value * 2 * kOpBytes;
@@ -919,22 +1092,22 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
       if (np > 0) {
         // A pair 0, B stages 0-3, A pair 1; then stage 0 is followed by 20
         // younger transfers.
-        uint64_t sa = uniform64(src_a(0));
+        uint64_t sa = uniform64(pa.src(0));
 #pragma unroll
         for (int x = 0; x < 8; ++x) dma_a(SlotC<0>{}, x, sa);
-        uint64_t sb = uniform64(src_b(0));
+        uint64_t sb = uniform64(lb.stage_src(0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<0>{}, x, sb);
-        sb = uniform64(src_b(1 < ns ? 1 : 0));
+        sb = uniform64(lb.stage_src(1 < ns ? 1 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<1>{}, x, sb);
-        sb = uniform64(src_b(2 < ns ? 2 : 0));
+        sb = uniform64(lb.stage_src(2 < ns ? 2 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<2>{}, x, sb);
-        sb = uniform64(src_b(3 < ns ? 3 : 0));
+        sb = uniform64(lb.stage_src(3 < ns ? 3 : 0));
 #pragma unroll
         for (int x = 0; x < 4; ++x) dma_b(SlotC<3>{}, x, sb);
-        sa = uniform64(src_a(np > 1 ? 1 : 0));
+        sa = uniform64(pa.src(np > 1 ? 1 : 0));
 #pragma unroll
         for (int x = 0; x < 8; ++x) dma_a(SlotC<1>{}, x, sa);
         __builtin_amdgcn_s_waitcnt(vm_wait(20));
@@ -993,10 +1166,10 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
             // DMA sources (B stage s+4, A pair s/2 + 2), computed behind the
             // first MFMAs.
             const int nb = st + kRing < ns ? st + kRing : 0;
-            sb = uniform64(src_b(nb));
+            sb = uniform64(lb.stage_src(nb));
             if constexpr (kOdd) {
               const int p = (st >> 1) + 2;
-              sa = uniform64(src_a(p < np ? p : np - 1));
+              sa = uniform64(pa.src(p < np ? p : np - 1));
             }
           }
           __builtin_amdgcn_sched_barrier(0);
