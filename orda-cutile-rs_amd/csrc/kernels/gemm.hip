@@ -2197,28 +2197,41 @@ bool small_f32(const GemmArgs& g) {
   return tiles <= 64;
 }
 
-// The small kernel's split of K: as plan_split, over its 128 x 128 tiles,
-// each split at least 256 elements of K.
+// The small kernel's split of K, over its 128 x 128 tiles: the split of least
+// cost as in plan_split (2.4 us for every 32 elements of K, 6 us a round),
+// each part at least 128 elements. (Parts of at least 256, and as many as fill
+// 256 workgroups: Tied 64 x 256 x 2048 134 us a call against 117, Precomputed
+// 300 x 300 x 5000 193 against 167, Tied 300 x 768 x 3000 284 against 260, 256 x
+// 512 x 8192 the same; two workgroups a CU, 512 in all, were slower there, 253
+// against 223.)
 SplitPlan plan_split_small(const GemmArgs& g) {
   SplitPlan sp{1, g.K, 0, 0, 0};
   if (g.K <= 0) return sp;
   const int64_t tiles = small_tiles(g);
   if (tiles >= 192) return sp;
-  int64_t s = (256 + tiles - 1) / tiles;
-  const int64_t by_k = g.K / 256;
-  if (s > by_k) s = by_k;
-  if (s > 64) s = 64;
   const int64_t per_split = g.nprob * (g.c_trans ? g.N * ((g.M + 3) / 4 * 4) : g.M * ((g.N + 3) / 4 * 4)) * 4;
-  if (s > (int64_t{256} << 20) / per_split) s = (int64_t{256} << 20) / per_split;
-  if (s <= 1) return sp;
-  const int64_t len = ((g.K + s - 1) / s + 63) / 64 * 64;
-  s = (g.K + len - 1) / len;
-  if (s <= 1) return sp;
-  sp.splits = static_cast<int>(s);
-  sp.len = len;
+  int64_t most = (256 + tiles - 1) / tiles;
+  const int64_t by_k = g.K / 128, by_ws = (int64_t{256} << 20) / per_split;
+  if (most > by_k) most = by_k;
+  if (most > 64) most = 64;
+  if (most > by_ws) most = by_ws;
+  auto cost = [&](int64_t n, int64_t len) {
+    return static_cast<double>((tiles * n + 255) / 256) * (static_cast<double>(len) / 32 * 2.4 + 6.0) +
+           (n > 1 ? 2 * kPartUs * static_cast<double>(n * per_split) : 0.0);
+  };
+  double best = cost(1, g.K);
+  for (int64_t i = 2; i <= most; ++i) {
+    const int64_t len = ((g.K + i - 1) / i + 63) / 64 * 64, n = (g.K + len - 1) / len;
+    if (n <= 1) break;
+    if (cost(n, len) >= best) continue;
+    best = cost(n, len);
+    sp.splits = static_cast<int>(n);
+    sp.len = len;
+  }
+  if (sp.splits <= 1) return sp;
   sp.ldp = ((g.c_trans ? g.M : g.N) + 3) / 4 * 4;
   sp.stride = g.nprob * (g.c_trans ? g.N : g.M) * sp.ldp;
-  sp.bytes = s * sp.stride * 4;
+  sp.bytes = sp.splits * sp.stride * 4;
   return sp;
 }
 
