@@ -168,7 +168,7 @@ __device__ __forceinline__ uint64_t uniform64(const void* p) {
 //         columns [origin, origin+256).
 // Rows/columns past the operand's edge are clamped to the last one that
 // exists: they only feed output rows/columns that are never stored.
-template <typename T, bool KMAJOR>
+template <typename T, bool KMAJOR, int NX = kXfers>
 struct Loader {
   static constexpr int ES = Elem<T>::kSize;
   static constexpr int EPC = 16 / ES;       // elements per 16-byte chunk
@@ -178,8 +178,8 @@ struct Loader {
   const unsigned char* base;   // operand origin: KMAJOR row origin, else column origin
   int64_t ld_bytes;
   int64_t K;
-  uint32_t goff[kXfers];       // byte offset of each transfer within a stage
-  int kidx[kXfers];            // K coordinate of each transfer within the stage
+  uint32_t goff[NX];       // byte offset of each transfer within a stage
+  int kidx[NX];            // K coordinate of each transfer within the stage
 
   __device__ __forceinline__ void init(const void* p, int64_t ld, int64_t ext, int64_t k,
                                        int origin, int wave, int lane) {
@@ -189,7 +189,7 @@ struct Loader {
       base = static_cast<const unsigned char*>(p) + static_cast<int64_t>(origin) * ld_bytes;
       const int rmax = static_cast<int>(ext - 1 - origin);
 #pragma unroll
-      for (int i = 0; i < kXfers; ++i) {
+      for (int i = 0; i < NX; ++i) {
         const int P = (i * 4 + wave) * 64 + lane;
         const int r = P / CPR;
         const int c = (P % CPR) ^ kmaj_swz(r);
@@ -201,7 +201,7 @@ struct Loader {
       base = static_cast<const unsigned char*>(p) + static_cast<int64_t>(origin) * ES;
       const int cmax = static_cast<int>((ext - 1 - origin) / EPC);
 #pragma unroll
-      for (int i = 0; i < kXfers; ++i) {
+      for (int i = 0; i < NX; ++i) {
         const int P = (i * 4 + wave) * 64 + lane;
         const int r = P / CPR;
         const int pc = P % CPR;
@@ -227,7 +227,7 @@ struct Loader {
     const int64_t b0 = origin < last ? origin : last;
     base = static_cast<const unsigned char*>((wave & 1) ? pt : ps) + b0 * ld_bytes;
 #pragma unroll
-    for (int i = 0; i < kXfers; ++i) {
+    for (int i = 0; i < NX; ++i) {
       const int P = (i * 4 + wave) * 64 + lane;
       const int r = P / CPR;
       const int c = (P % CPR) ^ kmaj_swz(r);
@@ -252,11 +252,11 @@ struct Loader {
     const int64_t krem = K - k0;
     if (krem >= SK) {
 #pragma unroll
-      for (int i = 0; i < kXfers; ++i)
+      for (int i = 0; i < NX; ++i)
         dma16(s, goff[i], tile + (i * 4 + wave) * 1024);
     } else {
 #pragma unroll
-      for (int i = 0; i < kXfers; ++i) {
+      for (int i = 0; i < NX; ++i) {
         unsigned char* l = tile + (i * 4 + wave) * 1024;
         if (kidx[i] < krem) {
           dma16(s, goff[i], l);
@@ -559,17 +559,19 @@ struct TileCoord {
   int p, m0, n0, ntile;
 };
 
+template <int TM>
 __device__ __forceinline__ TileCoord tile_at(int64_t pm, int64_t pn, int64_t Mt) {
   TileCoord c;
   c.p = static_cast<int>(pm / Mt);
-  c.m0 = static_cast<int>((pm % Mt) * kTile);
+  c.m0 = static_cast<int>((pm % Mt) * TM);
   c.n0 = static_cast<int>(pn * kTile);
   c.ntile = static_cast<int>(pn);
   return c;
 }
 
+template <int TM = kTile>
 __device__ __forceinline__ TileCoord map_tile(const GemmArgs& g, int64_t t) {
-  const int64_t Mt = (g.M + kTile - 1) / kTile;
+  const int64_t Mt = (g.M + TM - 1) / TM;
   const int64_t Nt = (g.N + kTile - 1) / kTile;
   int64_t Mv = Mt * g.nprob;
   int64_t T = Mv * Nt;
@@ -590,7 +592,7 @@ __device__ __forceinline__ TileCoord map_tile(const GemmArgs& g, int64_t t) {
     const int64_t full = Mv / bm * bm * Nt;   // 8 * per tiles per band
     if (t < full) {
       const int64_t x = t % 8, l = t / 8, k = l / per, j = l % per;
-      return tile_at(k * bm + (x / xn) * a + j % a, (x % xn) * b + j / a, Mt);
+      return tile_at<TM>(k * bm + (x / xn) * a + j % a, (x % xn) * b + j / a, Mt);
     }
     t -= full;
     T -= full;
@@ -607,7 +609,7 @@ __device__ __forceinline__ TileCoord map_tile(const GemmArgs& g, int64_t t) {
   const int64_t first = gid * gm;
   const int64_t gsize = (Mv - first) < gm ? (Mv - first) : gm;
   const int64_t r = t % in_group;
-  return tile_at(mfirst + first + r % gsize, r / gsize, Mt);
+  return tile_at<TM>(mfirst + first + r % gsize, r / gsize, Mt);
 }
 
 // Two floats as packed bf16 (round to nearest even), low half first.
@@ -615,6 +617,581 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
   return __builtin_bit_cast(uint32_t, v);
+}
+
+// The epilogue of a workgroup tile of 32*MF rows x 256 columns, 4 waves of
+// 16*MF x 128 as MF x 8 fragments in acc. epi: scratch of 112 bytes a tile row
+// (MF = 8: 16 KB beside the ring; else in the ring), ring: the operand ring,
+// idle by now.
+template <int ES, GemmEpilogue EPI, typename LT, bool CT, int MF>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const GemmProblem& pr, const TileCoord& tc,
+                                              f32x4 (&acc)[MF][kFrag], unsigned char* epi,
+                                              unsigned char* ring, int64_t lab_pre) {
+  constexpr bool kTeacherEpi = EPI == GemmEpilogue::LogitsTeacher || EPI == GemmEpilogue::LogitsTeacher16;
+  constexpr int TM = 32 * MF;   // tile rows
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  // ------------------------------------------------------------ epilogue
+  const int lrow = lane & 15;
+  const int lgrp = lane >> 4;
+  if constexpr (EPI == GemmEpilogue::StoreF32 || EPI == GemmEpilogue::AccumF32) {
+    float* C = static_cast<float*>(pr.c);
+    const float alpha = g.alpha_ptr != nullptr ? g.alpha * *g.alpha_ptr : g.alpha;
+    // acc[i][j][e] is row wm*16*MF + 16i + 4*lgrp + e, column wn*128 + 16j + lrow.
+    const int row_w = tc.m0 + wm * (TM / 2);
+    const int col_l = tc.n0 + wn * 128 + lrow;
+    if constexpr (CT) {
+      // C[n][m]: each lane holds 4 consecutive m of one n, one 16-byte
+      // store where the pitch and base allow (lanes lrow + 16g write 64
+      // contiguous bytes of row n).
+      const bool vec = (g.ldc % 4) == 0 && (reinterpret_cast<uintptr_t>(C) % 16) == 0;
+#pragma unroll
+      for (int j = 0; j < kFrag; ++j) {
+        const int64_t n = col_l + j * 16;
+        if (n >= g.N) continue;
+        float* cn = C + n * g.ldc;
+#pragma unroll
+        for (int i = 0; i < MF; ++i) {
+          const int64_t m = row_w + i * 16 + lgrp * 4;
+          f32x4 v = acc[i][j];
+          if (vec && m + 4 <= g.M) {
+            f32x4* dst = reinterpret_cast<f32x4*>(cn + m);
+            if constexpr (EPI == GemmEpilogue::AccumF32) v = alpha * (*dst + v);
+            else v = alpha * v;
+            *dst = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (m + e < g.M) {
+                float x = v[e];
+                if constexpr (EPI == GemmEpilogue::AccumF32) x = alpha * (cn[m + e] + x);
+                else x = alpha * x;
+                cn[m + e] = x;
+              }
+            }
+          }
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t row = row_w + i * 16 + lgrp * 4 + e;
+        if (row >= g.M) continue;
+        float* crow = C + row * g.ldc;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+          const int64_t col = col_l + j * 16;
+          if (col < g.N) {
+            float v = acc[i][j][e];
+            if constexpr (EPI == GemmEpilogue::AccumF32) v = alpha * (crow[col] + v);
+            else v = alpha * v;
+            crow[col] = v;
+          }
+        }
+      }
+    }
+  } else {
+    // Logits: per-row partial softmax statistics of this 256-column tile, the
+    // label logit, and the logits themselves. The accumulators hold
+    // transposed blocks (kSwapAB): acc[i][j][e] is row wm*128 + 16i + lrow,
+    // column wn*128 + 16j + 4*lgrp + e, so a lane owns 8 rows x 32 columns
+    // and each row's 128 columns of this wave sit in the 4 lanes lrow + 16g.
+    // With paired rows (pair_rows > 0) fragments 2q and 2q+1 hold a block of
+    // student rows and the same teacher rows, so a lane also holds both
+    // logits of every (row, column) it owns and forms the KL cross term.
+    LT* C = static_cast<LT*>(pr.c);
+    int64_t* lab = reinterpret_cast<int64_t*>(epi);                      // [TM]
+    float4* part = reinterpret_cast<float4*>(epi + 8 * TM);              // [2][TM]
+    float2* xpart = reinterpret_cast<float2*>(epi + 40 * TM);            // [2][TM]
+    const int64_t prs = g.lg.pair_rows;
+    // Tile row rl as (output row, teacher?, valid): stats / xy / C row index.
+    auto out_row = [&](int rl, bool& teacher, bool& valid) -> int64_t {
+      if (prs > 0) {
+        const int64_t R = static_cast<int64_t>(tc.m0) + rl;
+        const int64_t r = ((R >> 5) << 4) + (R & 15);
+        teacher = ((R >> 4) & 1) != 0;
+        valid = r < prs;
+        return teacher ? prs + r : r;
+      }
+      teacher = false;
+      valid = tc.m0 + rl < g.M;
+      return static_cast<int64_t>(tc.p) * g.M + tc.m0 + rl;
+    };
+    if (TM == kThreads || tid < TM) lab[tid] = lab_pre;
+    __syncthreads();
+    const float it2 = g.lg.inv_t * kLog2e;
+    const int64_t colw = static_cast<int64_t>(tc.n0) + wn * 128 + 4 * lgrp;   // (j, e) = (0, 0)
+    const int64_t ncol64 = g.N - colw;                    // (j, e) valid iff 16j + e < ncol
+    const int ncol = static_cast<int>(ncol64 < 128 ? (ncol64 < 0 ? 0 : ncol64) : 128);
+    // This lane's 32 logits of one row, from column colw on.
+    auto store_row = [&](auto full_c, LT* crow, const f32x4 (&v)[kFrag]) {
+      constexpr bool kFull = decltype(full_c)::value;
+#pragma unroll
+      for (int j = 0; j < kFrag; ++j) {
+        if (kFull || j * 16 + 4 <= ncol) {
+          if constexpr (Elem<LT>::kSize == 2) {
+            u32x2 w;
+            w[0] = pack_bf16(v[j][0], v[j][1]);
+            w[1] = pack_bf16(v[j][2], v[j][3]);
+            *reinterpret_cast<u32x2*>(crow + j * 16) = w;
+          } else {
+            *reinterpret_cast<f32x4*>(crow + j * 16) = v[j];
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (j * 16 + e < ncol) crow[j * 16 + e] = static_cast<LT>(v[j][e]);
+        }
+      }
+    };
+    // bf16 rows of full tiles leave as 16-byte stores: for each fragment pair
+    // (j, j+1), one v_permlane16_swap per dword gives the lanes of 16-lane
+    // row g (g = lane/16) eight consecutive columns, 16*(j + g%2) + 8*(g/2)
+    // onward, so a store instruction writes 64 contiguous bytes of each of 16
+    // rows instead of 32. Done by every lane (the swap pairs lanes 16 apart,
+    // which hold the same row); the stores follow under the row's test.
+    auto swap_rows = [&](const f32x4 (&v)[kFrag], u32x4 (&w)[kFrag / 2]) {
+#pragma unroll
+      for (int jp = 0; jp < kFrag; jp += 2) {
+        const auto a = __builtin_amdgcn_permlane16_swap(pack_bf16(v[jp][0], v[jp][1]),
+                                                        pack_bf16(v[jp + 1][0], v[jp + 1][1]),
+                                                        false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(pack_bf16(v[jp][2], v[jp][3]),
+                                                        pack_bf16(v[jp + 1][2], v[jp + 1][3]),
+                                                        false, false);
+        w[jp / 2] = u32x4{a[0], b[0], a[1], b[1]};
+      }
+    };
+    // rowbase: the row's element at column tc.n0 + wn*128. Non-temporal
+    // stores: the logits are read again only by the row pass, after gigabytes
+    // of other traffic, and as ordinary stores they displace operand strips
+    // from L2 (measured 0.04-0.1 ms faster on the logits GEMM; the same for
+    // grad_W's fp32 stores measured 0.27 ms slower).
+    auto store_swapped = [&](LT* rowbase, const u32x4 (&w)[kFrag / 2]) {
+      const int c0 = 16 * (lgrp & 1) + 8 * (lgrp >> 1);
+#pragma unroll
+      for (int jp = 0; jp < kFrag; jp += 2)
+        __builtin_nontemporal_store(w[jp / 2], reinterpret_cast<u32x4*>(rowbase + 16 * jp + c0));
+    };
+    constexpr bool kSwapStore = Elem<LT>::kSize == 2;
+    // bf16 logits are stored as t = (x - m)·log2(e), m the row's maximum over
+    // this wave's 128 columns (written to hmax after the merge below): the
+    // first exponent's argument, so e^((x-m)/T) = 2^(t/T) costs no more.
+    constexpr bool kRel = Elem<LT>::kSize == 2;
+    const float inv_t = g.lg.inv_t;
+    // The label's logit, if this lane holds its column (16j + e == yl):
+    // select e, then j.
+    auto pick = [&](const f32x4 (&v)[kFrag], int yl) {
+      const int jy = yl >> 4, ey = yl & 3;
+      float xy = 0.f;
+#pragma unroll
+      for (int j = 0; j < kFrag; ++j) {
+        float t = v[j][0];
+        t = ey == 1 ? v[j][1] : t;
+        t = ey == 2 ? v[j][2] : t;
+        t = ey == 3 ? v[j][3] : t;
+        xy = jy == j ? t : xy;
+      }
+      return xy;
+    };
+    auto quad_max = [](float x) {
+      x = fmaxf(x, __shfl_xor(x, 16));
+      return fmaxf(x, __shfl_xor(x, 32));
+    };
+    auto quad_sum = [](float x) {
+      x += __shfl_xor(x, 16);
+      return x + __shfl_xor(x, 32);
+    };
+    // Full tiles (all but the last column tile when N % 256 != 0) take a
+    // path without per-column checks.
+    auto rows = [&](auto full_c) {
+      constexpr bool kFull = decltype(full_c)::value;
+#pragma unroll
+      for (int i = 0; i < MF; ++i) {
+        f32x4 av[kFrag];
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) av[j] = from_acc(acc[i][j]);
+        const int rl = wm * (TM / 2) + i * 16 + lrow;           // row within tile
+        const int64_t row = tc.m0 + rl;
+        const int64_t yl64 = lab[rl] - colw;
+        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
+        float mx = -INFINITY;
+        if constexpr (kFull) {
+          mx = row_max32(av);
+        } else {
+#pragma unroll
+          for (int j = 0; j < kFrag; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (j * 16 + e < ncol) mx = fmaxf(mx, av[j][e]);
+        }
+        mx = quad_max(mx);
+        // exp((x - mx)) and exp((x - mx)/T) as exp2 of one fma each.
+        const float o1 = -mx * kLog2e, oT = -mx * it2;
+        const bool hit = yl >= 0 && (yl & 12) == 0;
+        float xyv = 0.f;   // the label's fp32 logit, before av holds t
+        if constexpr (kRel) {
+          if (hit) xyv = pick(av, yl);
+        }
+        float d1 = 0.f, dT = 0.f, sx = 0.f;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float x = av[j][e];
+            float a1, aT;
+            if constexpr (kRel) {
+              const float t = fmaf(x, kLog2e, o1);
+              a1 = __builtin_amdgcn_exp2f(t);
+              aT = __builtin_amdgcn_exp2f(t * inv_t);
+              av[j][e] = t;
+            } else {
+              a1 = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, o1));
+              aT = __builtin_amdgcn_exp2f(fmaf(x, it2, oT));
+            }
+            if (kFull || j * 16 + e < ncol) {
+              d1 += a1;
+              dT += aT;
+              sx += x;
+            }
+          }
+        }
+        d1 = quad_sum(d1);
+        dT = quad_sum(dT);
+        sx = quad_sum(sx);
+        if (lgrp == 0) part[wn * TM + rl] = make_float4(mx, d1, dT, sx);
+        u32x4 aw[kFrag / 2];
+        if constexpr (kSwapStore && kFull) swap_rows(av, aw);
+        if (row < g.M) {
+          if (hit) g.lg.xy[tc.p * g.M + row] = kRel ? xyv : pick(av, yl);
+          if constexpr (kSwapStore && kFull)
+            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), aw);
+          else
+            store_row(full_c, C + row * g.ldc + colw, av);
+        }
+      }
+    };
+    auto rows_pair = [&](auto full_c) {
+      constexpr bool kFull = decltype(full_c)::value;
+#pragma unroll
+      for (int q = 0; q < MF / 2; ++q) {
+        f32x4 as[kFrag], at[kFrag];
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) as[j] = from_acc(acc[2 * q][j]);
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) at[j] = from_acc(acc[2 * q + 1][j]);
+        const int rs = wm * (TM / 2) + q * 32 + lrow;                         // tile rows
+        const int rt = rs + 16;
+        const int64_t row = (tc.m0 >> 1) + wm * (TM / 4) + q * 16 + lrow;      // student row
+        const int64_t yl64 = lab[rs] - colw;
+        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
+        float ms = -INFINITY, mt = -INFINITY;
+        if constexpr (kFull) {
+          ms = row_max32(as);
+          mt = row_max32(at);
+        } else {
+#pragma unroll
+          for (int j = 0; j < kFrag; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (j * 16 + e < ncol) {
+                ms = fmaxf(ms, as[j][e]);
+                mt = fmaxf(mt, at[j][e]);
+              }
+        }
+        ms = quad_max(ms);
+        mt = quad_max(mt);
+        const float o1s = -ms * kLog2e, o1t = -mt * kLog2e;
+        const bool hit = yl >= 0 && (yl & 12) == 0;
+        float xys = 0.f, xyt = 0.f;   // the label's fp32 logits, before as/at hold t
+        if constexpr (kRel) {
+          if (hit) {
+            xys = pick(as, yl);
+            xyt = pick(at, yl);
+          }
+        }
+        // Per element pair, in log2 units relative to the rows' own half
+        // maxima: ts, tt (the stored values), e^((x-m)/T) = 2^(t/T). The KL
+        // sums take (tt - ts) and (aTs - aTt), so a constant offset between
+        // the two rows cancels in each element; Σ aTs = dd + Σ aTt.
+        float d1s = 0.f, sxs = 0.f, d1t = 0.f, dTt = 0.f, sxt = 0.f, cx = 0.f, dd = 0.f;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float xs = as[j][e], xt = at[j][e];
+            const float ts = fmaf(xs, kLog2e, o1s), tt = fmaf(xt, kLog2e, o1t);
+            const float a1s = __builtin_amdgcn_exp2f(ts);
+            const float aTs = __builtin_amdgcn_exp2f(ts * inv_t);
+            const float a1t = __builtin_amdgcn_exp2f(tt);
+            const float aTt = __builtin_amdgcn_exp2f(tt * inv_t);
+            if constexpr (kRel) {
+              as[j][e] = ts;
+              at[j][e] = tt;
+            }
+            if (kFull || j * 16 + e < ncol) {
+              d1s += a1s;
+              dd += aTs - aTt;
+              sxs += xs;
+              d1t += a1t;
+              dTt += aTt;
+              sxt += xt;
+              cx = fmaf(aTt, tt - ts, cx);
+            }
+          }
+        }
+        d1s = quad_sum(d1s);
+        dd = quad_sum(dd);
+        sxs = quad_sum(sxs);
+        d1t = quad_sum(d1t);
+        dTt = quad_sum(dTt);
+        sxt = quad_sum(sxt);
+        cx = quad_sum(cx);
+        const float dTs = dd + dTt;
+        if (lgrp == 0) {
+          part[wn * TM + rs] = make_float4(ms, d1s, dTs, sxs);
+          part[wn * TM + rt] = make_float4(mt, d1t, dTt, sxt);
+          xpart[wn * TM + rt] = make_float2(cx, dd);
+        }
+        u32x4 sw[kFrag / 2], tw[kFrag / 2];
+        if constexpr (kSwapStore && kFull) {
+          swap_rows(as, sw);
+          swap_rows(at, tw);
+        }
+        if (row < prs) {
+          if (hit) {   // one lane of a row at most, for one column tile
+            g.lg.xy[row] = kRel ? xys : pick(as, yl);
+            g.lg.xy[prs + row] = kRel ? xyt : pick(at, yl);
+          }
+          if constexpr (kSwapStore && kFull) {
+            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), sw);
+            store_swapped(C + (prs + row) * g.ldc + (colw - 4 * lgrp), tw);
+          } else {
+            store_row(full_c, C + row * g.ldc + colw, as);
+            store_row(full_c, C + (prs + row) * g.ldc + colw, at);
+          }
+        }
+      }
+    };
+    // Teacher logits beside the student rows (LogitsTeacher, LogitsTeacher16):
+    // per row block the lane's 32 teacher logits of its row are loaded
+    // (16-byte vectors of fp32 or 8-byte vectors of bf16, one block ahead,
+    // so that they are in flight while the previous block computes) and take
+    // the place of the paired GEMM's teacher accumulators: the teacher's
+    // half-tile statistics and label logit and the two KL sums come out as
+    // with paired rows. Only the student rows are stored. The teacher's half
+    // statistics go to partT, in the ring (idle once the main loop has
+    // drained). Non-temporal loads: the logits are read again only by the row
+    // pass, and the L2 holds the operand strips.
+    float4* partT = reinterpret_cast<float4*>(ring + (epi == ring ? 56 * TM : 0));   // [2][TM]
+    auto load_t = [&](auto full_c, int i, f32x4 (&tv)[kFrag]) {
+      constexpr bool kFull = decltype(full_c)::value;
+      const int64_t row = static_cast<int64_t>(tc.m0) + wm * (TM / 2) + i * 16 + lrow;
+      const int64_t off = (row < g.M ? row : g.M - 1) * g.lg.teacher_ld + colw;
+      if constexpr (EPI == GemmEpilogue::LogitsTeacher16) {
+        const __bf16* trow = static_cast<const __bf16*>(g.lg.teacher_logits) + off;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+          if (kFull || j * 16 + 4 <= ncol) {
+            const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(trow + j * 16));
+            tv[j][0] = __uint_as_float(w[0] << 16);
+            tv[j][1] = __uint_as_float(w[0] & 0xffff0000u);
+            tv[j][2] = __uint_as_float(w[1] << 16);
+            tv[j][3] = __uint_as_float(w[1] & 0xffff0000u);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              tv[j][e] = j * 16 + e < ncol ? static_cast<float>(trow[j * 16 + e]) : 0.f;
+          }
+        }
+      } else {
+        const float* trow = static_cast<const float*>(g.lg.teacher_logits) + off;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+          if (kFull || j * 16 + 4 <= ncol) {
+            tv[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(trow + j * 16));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tv[j][e] = j * 16 + e < ncol ? trow[j * 16 + e] : 0.f;
+          }
+        }
+      }
+    };
+    auto rows_teacher = [&](auto full_c) {
+      constexpr bool kFull = decltype(full_c)::value;
+      f32x4 tbuf[2][kFrag];
+      load_t(full_c, 0, tbuf[0]);
+#pragma unroll
+      for (int i = 0; i < MF; ++i) {
+        if (i + 1 < MF) load_t(full_c, i + 1, tbuf[(i + 1) & 1]);
+        f32x4 as[kFrag];
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) as[j] = from_acc(acc[i][j]);
+        const f32x4(&at)[kFrag] = tbuf[i & 1];
+        const int rl = wm * (TM / 2) + i * 16 + lrow;            // row within tile
+        const int64_t row = tc.m0 + rl;
+        const int64_t yl64 = lab[rl] - colw;
+        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
+        float ms = -INFINITY, mt = -INFINITY;
+        if constexpr (kFull) {
+          ms = row_max32(as);
+          mt = row_max32(at);
+        } else {
+#pragma unroll
+          for (int j = 0; j < kFrag; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (j * 16 + e < ncol) {
+                ms = fmaxf(ms, as[j][e]);
+                mt = fmaxf(mt, at[j][e]);
+              }
+        }
+        ms = quad_max(ms);
+        mt = quad_max(mt);
+        const float o1s = -ms * kLog2e, o1t = -mt * kLog2e;
+        const bool hit = yl >= 0 && (yl & 12) == 0;
+        float xys = 0.f, xyt = 0.f;   // the label's fp32 logits, before as holds t
+        if (hit) {
+          xys = pick(as, yl);
+          xyt = pick(at, yl);
+        }
+        // as in rows_pair: log2 units relative to the half maxima, the KL sums
+        // over (tt - ts) and (aTs - aTt), Σ aTs = dd + Σ aTt
+        float d1s = 0.f, sxs = 0.f, d1t = 0.f, dTt = 0.f, sxt = 0.f, cx = 0.f, dd = 0.f;
+#pragma unroll
+        for (int j = 0; j < kFrag; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float xs = as[j][e], xt = at[j][e];
+            const float ts = fmaf(xs, kLog2e, o1s), tt = fmaf(xt, kLog2e, o1t);
+            const float a1s = __builtin_amdgcn_exp2f(ts);
+            const float aTs = __builtin_amdgcn_exp2f(ts * inv_t);
+            const float a1t = __builtin_amdgcn_exp2f(tt);
+            const float aTt = __builtin_amdgcn_exp2f(tt * inv_t);
+            if constexpr (kRel) as[j][e] = ts;
+            if (kFull || j * 16 + e < ncol) {
+              d1s += a1s;
+              dd += aTs - aTt;
+              sxs += xs;
+              d1t += a1t;
+              dTt += aTt;
+              sxt += xt;
+              cx = fmaf(aTt, tt - ts, cx);
+            }
+          }
+        }
+        d1s = quad_sum(d1s);
+        dd = quad_sum(dd);
+        sxs = quad_sum(sxs);
+        d1t = quad_sum(d1t);
+        dTt = quad_sum(dTt);
+        sxt = quad_sum(sxt);
+        cx = quad_sum(cx);
+        const float dTs = dd + dTt;
+        if (lgrp == 0) {
+          part[wn * TM + rl] = make_float4(ms, d1s, dTs, sxs);
+          partT[wn * TM + rl] = make_float4(mt, d1t, dTt, sxt);
+          xpart[wn * TM + rl] = make_float2(cx, dd);
+        }
+        u32x4 aw[kFrag / 2];
+        if constexpr (kSwapStore && kFull) swap_rows(as, aw);
+        if (row < g.M) {
+          if (hit) {   // one lane of a row at most, for one column tile
+            g.lg.xy[row] = xys;
+            g.lg.xy[g.M + row] = xyt;
+          }
+          if constexpr (kSwapStore && kFull)
+            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), aw);
+          else
+            store_row(full_c, C + row * g.ldc + colw, as);
+        }
+      }
+    };
+    const bool full = tc.n0 + kTile <= g.N;
+    if constexpr (kTeacherEpi) {
+      static_assert(kRel, "the student rows beside Precomputed teacher logits are bf16");
+      if (full) rows_teacher(SlotC<1>{});
+      else rows_teacher(SlotC<0>{});
+    } else if (prs > 0) {
+      if (full) rows_pair(SlotC<1>{});
+      else rows_pair(SlotC<0>{});
+    } else {
+      if (full) rows(SlotC<1>{});
+      else rows(SlotC<0>{});
+    }
+    __syncthreads();
+    if (TM == kThreads || tid < TM) {
+      bool teacher, ok;
+      const int64_t orow = out_row(tid, teacher, ok);
+      if (ok) {
+        const float4 a = part[tid], b = part[TM + tid];
+        const float m = fmaxf(a.x, b.x);
+        float4 s;
+        s.x = m;
+        s.w = a.w + b.w;
+        float2 cx = make_float2(0.f, 0.f);
+        if (m == -INFINITY) {
+          s.y = 0.f;
+          s.z = 0.f;
+        } else if (teacher) {
+          // the KL sums of the two halves relative to the tile's maxima; the
+          // student row of this pair is tile row tid - 16
+          const float4 sa = part[tid - 16], sb = part[TM + tid - 16];
+          const float ms = fmaxf(sa.x, sb.x);
+          const float2 xa = kl_rebase(xpart[tid], sa.x, a.x, sa.z, a.z, ms, m, g.lg.inv_t);
+          const float2 xb = kl_rebase(xpart[TM + tid], sb.x, b.x, sb.z, b.z, ms, m, g.lg.inv_t);
+          cx = make_float2(xa.x + xb.x, xa.y + xb.y);
+        }
+        if (m != -INFINITY) {
+          const float ea = __builtin_amdgcn_exp2f((a.x - m) * kLog2e);
+          const float eb = __builtin_amdgcn_exp2f((b.x - m) * kLog2e);
+          const float fa = __builtin_amdgcn_exp2f((a.x - m) * it2);
+          const float fb = __builtin_amdgcn_exp2f((b.x - m) * it2);
+          s.y = a.y * ea + b.y * eb;
+          s.z = a.z * fa + b.z * fb;
+        }
+        g.lg.stats[orow * g.lg.stats_ld + tc.ntile] = s;
+        if constexpr (kRel) {   // the two halves' maxima, beside the other block's
+          const int64_t hrow = prs > 0 ? (teacher ? orow - prs : orow) : tc.m0 + tid;
+          const int side = prs > 0 ? (teacher ? 1 : 0) : tc.p;
+          float* hp = g.lg.hmax + hrow * g.lg.hmax_ld + 4 * tc.ntile + side;
+          hp[0] = a.x;
+          hp[2] = b.x;
+        }
+        if (teacher) g.lg.cross[(orow - prs) * g.lg.stats_ld + tc.ntile] = cx;
+        if constexpr (kTeacherEpi) {
+          // the teacher row beside this student row: its tile statistics,
+          // and the two KL sums relative to the two rows' tile maxima
+          const float4 ta = partT[tid], tb = partT[TM + tid];
+          const float mtt = fmaxf(ta.x, tb.x);
+          float4 st;
+          st.x = mtt;
+          st.w = ta.w + tb.w;
+          float2 kx = make_float2(0.f, 0.f);
+          if (mtt == -INFINITY) {
+            st.y = 0.f;
+            st.z = 0.f;
+          } else {
+            st.y = ta.y * __builtin_amdgcn_exp2f((ta.x - mtt) * kLog2e) +
+                   tb.y * __builtin_amdgcn_exp2f((tb.x - mtt) * kLog2e);
+            st.z = ta.z * __builtin_amdgcn_exp2f((ta.x - mtt) * it2) +
+                   tb.z * __builtin_amdgcn_exp2f((tb.x - mtt) * it2);
+            const float2 xa = kl_rebase(xpart[tid], a.x, ta.x, a.z, ta.z, m, mtt, g.lg.inv_t);
+            const float2 xb = kl_rebase(xpart[TM + tid], b.x, tb.x, b.z, tb.z, m, mtt, g.lg.inv_t);
+            kx = make_float2(xa.x + xb.x, xa.y + xb.y);
+          }
+          const int64_t r = orow - static_cast<int64_t>(tc.p) * g.M;
+          g.lg.stats[(g.M + r) * g.lg.stats_ld + tc.ntile] = st;
+          g.lg.cross[r * g.lg.stats_ld + tc.ntile] = kx;
+        }
+      }
+    }
+  }
 }
 
 template <typename T, bool AK, bool BK, GemmEpilogue EPI, typename LT, bool CT, bool P3 = false>
@@ -1262,568 +1839,135 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& g) {
   __builtin_amdgcn_s_waitcnt(kWaitAll);
   __builtin_amdgcn_s_barrier();
 
-  // ------------------------------------------------------------ epilogue
-  const int lrow = lane & 15;
-  const int lgrp = lane >> 4;
-  if constexpr (EPI == GemmEpilogue::StoreF32 || EPI == GemmEpilogue::AccumF32) {
-    float* C = static_cast<float*>(pr.c);
-    const float alpha = g.alpha_ptr != nullptr ? g.alpha * *g.alpha_ptr : g.alpha;
-    static_assert(!kSwapAB, "the store epilogues take unswapped operands");
-    // acc[i][j][e] is row wm*128 + 16i + 4*lgrp + e, column wn*128 + 16j + lrow.
-    const int row_w = tc.m0 + wm * 128;
-    const int col_l = tc.n0 + wn * 128 + lrow;
-    if constexpr (CT) {
-      // C[n][m]: each lane holds 4 consecutive m of one n, one 16-byte
-      // store where the pitch and base allow (lanes lrow + 16g write 64
-      // contiguous bytes of row n).
-      const bool vec = (g.ldc % 4) == 0 && (reinterpret_cast<uintptr_t>(C) % 16) == 0;
-#pragma unroll
-      for (int j = 0; j < kFrag; ++j) {
-        const int64_t n = col_l + j * 16;
-        if (n >= g.N) continue;
-        float* cn = C + n * g.ldc;
-#pragma unroll
-        for (int i = 0; i < kFrag; ++i) {
-          const int64_t m = row_w + i * 16 + lgrp * 4;
-          f32x4 v = acc[i][j];
-          if (vec && m + 4 <= g.M) {
-            f32x4* dst = reinterpret_cast<f32x4*>(cn + m);
-            if constexpr (EPI == GemmEpilogue::AccumF32) v = alpha * (*dst + v);
-            else v = alpha * v;
-            *dst = v;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (m + e < g.M) {
-                float x = v[e];
-                if constexpr (EPI == GemmEpilogue::AccumF32) x = alpha * (cn[m + e] + x);
-                else x = alpha * x;
-                cn[m + e] = x;
-              }
-            }
-          }
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < kFrag; ++i) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t row = row_w + i * 16 + lgrp * 4 + e;
-        if (row >= g.M) continue;
-        float* crow = C + row * g.ldc;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-          const int64_t col = col_l + j * 16;
-          if (col < g.N) {
-            float v = acc[i][j][e];
-            if constexpr (EPI == GemmEpilogue::AccumF32) v = alpha * (crow[col] + v);
-            else v = alpha * v;
-            crow[col] = v;
-          }
-        }
-      }
-    }
-  } else {
-    // Logits: per-row partial softmax statistics of this 256-column tile, the
-    // label logit, and the logits themselves. The accumulators hold
-    // transposed blocks (kSwapAB): acc[i][j][e] is row wm*128 + 16i + lrow,
-    // column wn*128 + 16j + 4*lgrp + e, so a lane owns 8 rows x 32 columns
-    // and each row's 128 columns of this wave sit in the 4 lanes lrow + 16g.
-    // With paired rows (pair_rows > 0) fragments 2q and 2q+1 hold a block of
-    // student rows and the same teacher rows, so a lane also holds both
-    // logits of every (row, column) it owns and forms the KL cross term.
-    LT* C = static_cast<LT*>(pr.c);
-    int64_t* lab = reinterpret_cast<int64_t*>(epi);                      // [256]
-    float4* part = reinterpret_cast<float4*>(epi + 2048);                // [2][256]
-    float2* xpart = reinterpret_cast<float2*>(epi + 10240);              // [2][256]
-    const int64_t prs = g.lg.pair_rows;
-    // Tile row rl as (output row, teacher?, valid): stats / xy / C row index.
-    auto out_row = [&](int rl, bool& teacher, bool& valid) -> int64_t {
-      if (prs > 0) {
-        const int64_t R = static_cast<int64_t>(tc.m0) + rl;
-        const int64_t r = ((R >> 5) << 4) + (R & 15);
-        teacher = ((R >> 4) & 1) != 0;
-        valid = r < prs;
-        return teacher ? prs + r : r;
-      }
-      teacher = false;
-      valid = tc.m0 + rl < g.M;
-      return static_cast<int64_t>(tc.p) * g.M + tc.m0 + rl;
-    };
-    lab[tid] = lab_pre;
-    __syncthreads();
-    const float it2 = g.lg.inv_t * kLog2e;
-    const int64_t colw = static_cast<int64_t>(tc.n0) + wn * 128 + 4 * lgrp;   // (j, e) = (0, 0)
-    const int64_t ncol64 = g.N - colw;                    // (j, e) valid iff 16j + e < ncol
-    const int ncol = static_cast<int>(ncol64 < 128 ? (ncol64 < 0 ? 0 : ncol64) : 128);
-    // This lane's 32 logits of one row, from column colw on.
-    auto store_row = [&](auto full_c, LT* crow, const f32x4 (&v)[kFrag]) {
-      constexpr bool kFull = decltype(full_c)::value;
-#pragma unroll
-      for (int j = 0; j < kFrag; ++j) {
-        if (kFull || j * 16 + 4 <= ncol) {
-          if constexpr (Elem<LT>::kSize == 2) {
-            u32x2 w;
-            w[0] = pack_bf16(v[j][0], v[j][1]);
-            w[1] = pack_bf16(v[j][2], v[j][3]);
-            *reinterpret_cast<u32x2*>(crow + j * 16) = w;
-          } else {
-            *reinterpret_cast<f32x4*>(crow + j * 16) = v[j];
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j * 16 + e < ncol) crow[j * 16 + e] = static_cast<LT>(v[j][e]);
-        }
-      }
-    };
-    // bf16 rows of full tiles leave as 16-byte stores: for each fragment pair
-    // (j, j+1), one v_permlane16_swap per dword gives the lanes of 16-lane
-    // row g (g = lane/16) eight consecutive columns, 16*(j + g%2) + 8*(g/2)
-    // onward, so a store instruction writes 64 contiguous bytes of each of 16
-    // rows instead of 32. Done by every lane (the swap pairs lanes 16 apart,
-    // which hold the same row); the stores follow under the row's test.
-    auto swap_rows = [&](const f32x4 (&v)[kFrag], u32x4 (&w)[kFrag / 2]) {
-#pragma unroll
-      for (int jp = 0; jp < kFrag; jp += 2) {
-        const auto a = __builtin_amdgcn_permlane16_swap(pack_bf16(v[jp][0], v[jp][1]),
-                                                        pack_bf16(v[jp + 1][0], v[jp + 1][1]),
-                                                        false, false);
-        const auto b = __builtin_amdgcn_permlane16_swap(pack_bf16(v[jp][2], v[jp][3]),
-                                                        pack_bf16(v[jp + 1][2], v[jp + 1][3]),
-                                                        false, false);
-        w[jp / 2] = u32x4{a[0], b[0], a[1], b[1]};
-      }
-    };
-    // rowbase: the row's element at column tc.n0 + wn*128. Non-temporal
-    // stores: the logits are read again only by the row pass, after gigabytes
-    // of other traffic, and as ordinary stores they displace operand strips
-    // from L2 (measured 0.04-0.1 ms faster on the logits GEMM; the same for
-    // grad_W's fp32 stores measured 0.27 ms slower).
-    auto store_swapped = [&](LT* rowbase, const u32x4 (&w)[kFrag / 2]) {
-      const int c0 = 16 * (lgrp & 1) + 8 * (lgrp >> 1);
-#pragma unroll
-      for (int jp = 0; jp < kFrag; jp += 2)
-        __builtin_nontemporal_store(w[jp / 2], reinterpret_cast<u32x4*>(rowbase + 16 * jp + c0));
-    };
-    constexpr bool kSwapStore = Elem<LT>::kSize == 2;
-    // bf16 logits are stored as t = (x - m)·log2(e), m the row's maximum over
-    // this wave's 128 columns (written to hmax after the merge below): the
-    // first exponent's argument, so e^((x-m)/T) = 2^(t/T) costs no more.
-    constexpr bool kRel = Elem<LT>::kSize == 2;
-    const float inv_t = g.lg.inv_t;
-    // The label's logit, if this lane holds its column (16j + e == yl):
-    // select e, then j.
-    auto pick = [&](const f32x4 (&v)[kFrag], int yl) {
-      const int jy = yl >> 4, ey = yl & 3;
-      float xy = 0.f;
-#pragma unroll
-      for (int j = 0; j < kFrag; ++j) {
-        float t = v[j][0];
-        t = ey == 1 ? v[j][1] : t;
-        t = ey == 2 ? v[j][2] : t;
-        t = ey == 3 ? v[j][3] : t;
-        xy = jy == j ? t : xy;
-      }
-      return xy;
-    };
-    auto quad_max = [](float x) {
-      x = fmaxf(x, __shfl_xor(x, 16));
-      return fmaxf(x, __shfl_xor(x, 32));
-    };
-    auto quad_sum = [](float x) {
-      x += __shfl_xor(x, 16);
-      return x + __shfl_xor(x, 32);
-    };
-    // Full tiles (all but the last column tile when N % 256 != 0) take a
-    // path without per-column checks.
-    auto rows = [&](auto full_c) {
-      constexpr bool kFull = decltype(full_c)::value;
-#pragma unroll
-      for (int i = 0; i < kFrag; ++i) {
-        f32x4 av[kFrag];
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) av[j] = from_acc(acc[i][j]);
-        const int rl = wm * 128 + i * 16 + lrow;           // row within tile
-        const int64_t row = tc.m0 + rl;
-        const int64_t yl64 = lab[rl] - colw;
-        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
-        float mx = -INFINITY;
-        if constexpr (kFull) {
-          mx = row_max32(av);
-        } else {
-#pragma unroll
-          for (int j = 0; j < kFrag; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (j * 16 + e < ncol) mx = fmaxf(mx, av[j][e]);
-        }
-        mx = quad_max(mx);
-        // exp((x - mx)) and exp((x - mx)/T) as exp2 of one fma each.
-        const float o1 = -mx * kLog2e, oT = -mx * it2;
-        const bool hit = yl >= 0 && (yl & 12) == 0;
-        float xyv = 0.f;   // the label's fp32 logit, before av holds t
-        if constexpr (kRel) {
-          if (hit) xyv = pick(av, yl);
-        }
-        float d1 = 0.f, dT = 0.f, sx = 0.f;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float x = av[j][e];
-            float a1, aT;
-            if constexpr (kRel) {
-              const float t = fmaf(x, kLog2e, o1);
-              a1 = __builtin_amdgcn_exp2f(t);
-              aT = __builtin_amdgcn_exp2f(t * inv_t);
-              av[j][e] = t;
-            } else {
-              a1 = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, o1));
-              aT = __builtin_amdgcn_exp2f(fmaf(x, it2, oT));
-            }
-            if (kFull || j * 16 + e < ncol) {
-              d1 += a1;
-              dT += aT;
-              sx += x;
-            }
-          }
-        }
-        d1 = quad_sum(d1);
-        dT = quad_sum(dT);
-        sx = quad_sum(sx);
-        if (lgrp == 0) part[wn * 256 + rl] = make_float4(mx, d1, dT, sx);
-        u32x4 aw[kFrag / 2];
-        if constexpr (kSwapStore && kFull) swap_rows(av, aw);
-        if (row < g.M) {
-          if (hit) g.lg.xy[tc.p * g.M + row] = kRel ? xyv : pick(av, yl);
-          if constexpr (kSwapStore && kFull)
-            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), aw);
-          else
-            store_row(full_c, C + row * g.ldc + colw, av);
-        }
-      }
-    };
-    auto rows_pair = [&](auto full_c) {
-      constexpr bool kFull = decltype(full_c)::value;
-#pragma unroll
-      for (int q = 0; q < kFrag / 2; ++q) {
-        f32x4 as[kFrag], at[kFrag];
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) as[j] = from_acc(acc[2 * q][j]);
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) at[j] = from_acc(acc[2 * q + 1][j]);
-        const int rs = wm * 128 + q * 32 + lrow;                         // tile rows
-        const int rt = rs + 16;
-        const int64_t row = (tc.m0 >> 1) + wm * 64 + q * 16 + lrow;      // student row
-        const int64_t yl64 = lab[rs] - colw;
-        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
-        float ms = -INFINITY, mt = -INFINITY;
-        if constexpr (kFull) {
-          ms = row_max32(as);
-          mt = row_max32(at);
-        } else {
-#pragma unroll
-          for (int j = 0; j < kFrag; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (j * 16 + e < ncol) {
-                ms = fmaxf(ms, as[j][e]);
-                mt = fmaxf(mt, at[j][e]);
-              }
-        }
-        ms = quad_max(ms);
-        mt = quad_max(mt);
-        const float o1s = -ms * kLog2e, o1t = -mt * kLog2e;
-        const bool hit = yl >= 0 && (yl & 12) == 0;
-        float xys = 0.f, xyt = 0.f;   // the label's fp32 logits, before as/at hold t
-        if constexpr (kRel) {
-          if (hit) {
-            xys = pick(as, yl);
-            xyt = pick(at, yl);
-          }
-        }
-        // Per element pair, in log2 units relative to the rows' own half
-        // maxima: ts, tt (the stored values), e^((x-m)/T) = 2^(t/T). The KL
-        // sums take (tt - ts) and (aTs - aTt), so a constant offset between
-        // the two rows cancels in each element; Σ aTs = dd + Σ aTt.
-        float d1s = 0.f, sxs = 0.f, d1t = 0.f, dTt = 0.f, sxt = 0.f, cx = 0.f, dd = 0.f;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float xs = as[j][e], xt = at[j][e];
-            const float ts = fmaf(xs, kLog2e, o1s), tt = fmaf(xt, kLog2e, o1t);
-            const float a1s = __builtin_amdgcn_exp2f(ts);
-            const float aTs = __builtin_amdgcn_exp2f(ts * inv_t);
-            const float a1t = __builtin_amdgcn_exp2f(tt);
-            const float aTt = __builtin_amdgcn_exp2f(tt * inv_t);
-            if constexpr (kRel) {
-              as[j][e] = ts;
-              at[j][e] = tt;
-            }
-            if (kFull || j * 16 + e < ncol) {
-              d1s += a1s;
-              dd += aTs - aTt;
-              sxs += xs;
-              d1t += a1t;
-              dTt += aTt;
-              sxt += xt;
-              cx = fmaf(aTt, tt - ts, cx);
-            }
-          }
-        }
-        d1s = quad_sum(d1s);
-        dd = quad_sum(dd);
-        sxs = quad_sum(sxs);
-        d1t = quad_sum(d1t);
-        dTt = quad_sum(dTt);
-        sxt = quad_sum(sxt);
-        cx = quad_sum(cx);
-        const float dTs = dd + dTt;
-        if (lgrp == 0) {
-          part[wn * 256 + rs] = make_float4(ms, d1s, dTs, sxs);
-          part[wn * 256 + rt] = make_float4(mt, d1t, dTt, sxt);
-          xpart[wn * 256 + rt] = make_float2(cx, dd);
-        }
-        u32x4 sw[kFrag / 2], tw[kFrag / 2];
-        if constexpr (kSwapStore && kFull) {
-          swap_rows(as, sw);
-          swap_rows(at, tw);
-        }
-        if (row < prs) {
-          if (hit) {   // one lane of a row at most, for one column tile
-            g.lg.xy[row] = kRel ? xys : pick(as, yl);
-            g.lg.xy[prs + row] = kRel ? xyt : pick(at, yl);
-          }
-          if constexpr (kSwapStore && kFull) {
-            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), sw);
-            store_swapped(C + (prs + row) * g.ldc + (colw - 4 * lgrp), tw);
-          } else {
-            store_row(full_c, C + row * g.ldc + colw, as);
-            store_row(full_c, C + (prs + row) * g.ldc + colw, at);
-          }
-        }
-      }
-    };
-    // Teacher logits beside the student rows (LogitsTeacher, LogitsTeacher16):
-    // per row block the lane's 32 teacher logits of its row are loaded
-    // (16-byte vectors of fp32 or 8-byte vectors of bf16, one block ahead,
-    // so that they are in flight while the previous block computes) and take
-    // the place of the paired GEMM's teacher accumulators: the teacher's
-    // half-tile statistics and label logit and the two KL sums come out as
-    // with paired rows. Only the student rows are stored. The teacher's half
-    // statistics go to partT, in the ring (idle once the main loop has
-    // drained). Non-temporal loads: the logits are read again only by the row
-    // pass, and the L2 holds the operand strips.
-    float4* partT = reinterpret_cast<float4*>(smem);   // [2][256]
-    auto load_t = [&](auto full_c, int i, f32x4 (&tv)[kFrag]) {
-      constexpr bool kFull = decltype(full_c)::value;
-      const int64_t row = static_cast<int64_t>(tc.m0) + wm * 128 + i * 16 + lrow;
-      const int64_t off = (row < g.M ? row : g.M - 1) * g.lg.teacher_ld + colw;
-      if constexpr (EPI == GemmEpilogue::LogitsTeacher16) {
-        const __bf16* trow = static_cast<const __bf16*>(g.lg.teacher_logits) + off;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-          if (kFull || j * 16 + 4 <= ncol) {
-            const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(trow + j * 16));
-            tv[j][0] = __uint_as_float(w[0] << 16);
-            tv[j][1] = __uint_as_float(w[0] & 0xffff0000u);
-            tv[j][2] = __uint_as_float(w[1] << 16);
-            tv[j][3] = __uint_as_float(w[1] & 0xffff0000u);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              tv[j][e] = j * 16 + e < ncol ? static_cast<float>(trow[j * 16 + e]) : 0.f;
-          }
-        }
-      } else {
-        const float* trow = static_cast<const float*>(g.lg.teacher_logits) + off;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-          if (kFull || j * 16 + 4 <= ncol) {
-            tv[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(trow + j * 16));
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) tv[j][e] = j * 16 + e < ncol ? trow[j * 16 + e] : 0.f;
-          }
-        }
-      }
-    };
-    auto rows_teacher = [&](auto full_c) {
-      constexpr bool kFull = decltype(full_c)::value;
-      f32x4 tbuf[2][kFrag];
-      load_t(full_c, 0, tbuf[0]);
-#pragma unroll
-      for (int i = 0; i < kFrag; ++i) {
-        if (i + 1 < kFrag) load_t(full_c, i + 1, tbuf[(i + 1) & 1]);
-        f32x4 as[kFrag];
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) as[j] = from_acc(acc[i][j]);
-        const f32x4(&at)[kFrag] = tbuf[i & 1];
-        const int rl = wm * 128 + i * 16 + lrow;            // row within tile
-        const int64_t row = tc.m0 + rl;
-        const int64_t yl64 = lab[rl] - colw;
-        const int yl = (yl64 >= 0 && yl64 < 128) ? static_cast<int>(yl64) : -1;
-        float ms = -INFINITY, mt = -INFINITY;
-        if constexpr (kFull) {
-          ms = row_max32(as);
-          mt = row_max32(at);
-        } else {
-#pragma unroll
-          for (int j = 0; j < kFrag; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (j * 16 + e < ncol) {
-                ms = fmaxf(ms, as[j][e]);
-                mt = fmaxf(mt, at[j][e]);
-              }
-        }
-        ms = quad_max(ms);
-        mt = quad_max(mt);
-        const float o1s = -ms * kLog2e, o1t = -mt * kLog2e;
-        const bool hit = yl >= 0 && (yl & 12) == 0;
-        float xys = 0.f, xyt = 0.f;   // the label's fp32 logits, before as holds t
-        if (hit) {
-          xys = pick(as, yl);
-          xyt = pick(at, yl);
-        }
-        // as in rows_pair: log2 units relative to the half maxima, the KL sums
-        // over (tt - ts) and (aTs - aTt), Σ aTs = dd + Σ aTt
-        float d1s = 0.f, sxs = 0.f, d1t = 0.f, dTt = 0.f, sxt = 0.f, cx = 0.f, dd = 0.f;
-#pragma unroll
-        for (int j = 0; j < kFrag; ++j) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float xs = as[j][e], xt = at[j][e];
-            const float ts = fmaf(xs, kLog2e, o1s), tt = fmaf(xt, kLog2e, o1t);
-            const float a1s = __builtin_amdgcn_exp2f(ts);
-            const float aTs = __builtin_amdgcn_exp2f(ts * inv_t);
-            const float a1t = __builtin_amdgcn_exp2f(tt);
-            const float aTt = __builtin_amdgcn_exp2f(tt * inv_t);
-            if constexpr (kRel) as[j][e] = ts;
-            if (kFull || j * 16 + e < ncol) {
-              d1s += a1s;
-              dd += aTs - aTt;
-              sxs += xs;
-              d1t += a1t;
-              dTt += aTt;
-              sxt += xt;
-              cx = fmaf(aTt, tt - ts, cx);
-            }
-          }
-        }
-        d1s = quad_sum(d1s);
-        dd = quad_sum(dd);
-        sxs = quad_sum(sxs);
-        d1t = quad_sum(d1t);
-        dTt = quad_sum(dTt);
-        sxt = quad_sum(sxt);
-        cx = quad_sum(cx);
-        const float dTs = dd + dTt;
-        if (lgrp == 0) {
-          part[wn * 256 + rl] = make_float4(ms, d1s, dTs, sxs);
-          partT[wn * 256 + rl] = make_float4(mt, d1t, dTt, sxt);
-          xpart[wn * 256 + rl] = make_float2(cx, dd);
-        }
-        u32x4 aw[kFrag / 2];
-        if constexpr (kSwapStore && kFull) swap_rows(as, aw);
-        if (row < g.M) {
-          if (hit) {   // one lane of a row at most, for one column tile
-            g.lg.xy[row] = xys;
-            g.lg.xy[g.M + row] = xyt;
-          }
-          if constexpr (kSwapStore && kFull)
-            store_swapped(C + row * g.ldc + (colw - 4 * lgrp), aw);
-          else
-            store_row(full_c, C + row * g.ldc + colw, as);
-        }
-      }
-    };
-    const bool full = tc.n0 + kTile <= g.N;
-    if constexpr (kTeacherEpi) {
-      static_assert(kRel, "the student rows beside Precomputed teacher logits are bf16");
-      if (full) rows_teacher(SlotC<1>{});
-      else rows_teacher(SlotC<0>{});
-    } else if (prs > 0) {
-      if (full) rows_pair(SlotC<1>{});
-      else rows_pair(SlotC<0>{});
-    } else {
-      if (full) rows(SlotC<1>{});
-      else rows(SlotC<0>{});
-    }
-    __syncthreads();
-    {
-      bool teacher, ok;
-      const int64_t orow = out_row(tid, teacher, ok);
-      if (ok) {
-        const float4 a = part[tid], b = part[256 + tid];
-        const float m = fmaxf(a.x, b.x);
-        float4 s;
-        s.x = m;
-        s.w = a.w + b.w;
-        float2 cx = make_float2(0.f, 0.f);
-        if (m == -INFINITY) {
-          s.y = 0.f;
-          s.z = 0.f;
-        } else if (teacher) {
-          // the KL sums of the two halves relative to the tile's maxima; the
-          // student row of this pair is tile row tid - 16
-          const float4 sa = part[tid - 16], sb = part[256 + tid - 16];
-          const float ms = fmaxf(sa.x, sb.x);
-          const float2 xa = kl_rebase(xpart[tid], sa.x, a.x, sa.z, a.z, ms, m, g.lg.inv_t);
-          const float2 xb = kl_rebase(xpart[256 + tid], sb.x, b.x, sb.z, b.z, ms, m, g.lg.inv_t);
-          cx = make_float2(xa.x + xb.x, xa.y + xb.y);
-        }
-        if (m != -INFINITY) {
-          const float ea = __builtin_amdgcn_exp2f((a.x - m) * kLog2e);
-          const float eb = __builtin_amdgcn_exp2f((b.x - m) * kLog2e);
-          const float fa = __builtin_amdgcn_exp2f((a.x - m) * it2);
-          const float fb = __builtin_amdgcn_exp2f((b.x - m) * it2);
-          s.y = a.y * ea + b.y * eb;
-          s.z = a.z * fa + b.z * fb;
-        }
-        g.lg.stats[orow * g.lg.stats_ld + tc.ntile] = s;
-        if constexpr (kRel) {   // the two halves' maxima, beside the other block's
-          const int64_t hrow = prs > 0 ? (teacher ? orow - prs : orow) : tc.m0 + tid;
-          const int side = prs > 0 ? (teacher ? 1 : 0) : tc.p;
-          float* hp = g.lg.hmax + hrow * g.lg.hmax_ld + 4 * tc.ntile + side;
-          hp[0] = a.x;
-          hp[2] = b.x;
-        }
-        if (teacher) g.lg.cross[(orow - prs) * g.lg.stats_ld + tc.ntile] = cx;
-        if constexpr (kTeacherEpi) {
-          // the teacher row beside this student row: its tile statistics,
-          // and the two KL sums relative to the two rows' tile maxima
-          const float4 ta = partT[tid], tb = partT[256 + tid];
-          const float mtt = fmaxf(ta.x, tb.x);
-          float4 st;
-          st.x = mtt;
-          st.w = ta.w + tb.w;
-          float2 kx = make_float2(0.f, 0.f);
-          if (mtt == -INFINITY) {
-            st.y = 0.f;
-            st.z = 0.f;
-          } else {
-            st.y = ta.y * __builtin_amdgcn_exp2f((ta.x - mtt) * kLog2e) +
-                   tb.y * __builtin_amdgcn_exp2f((tb.x - mtt) * kLog2e);
-            st.z = ta.z * __builtin_amdgcn_exp2f((ta.x - mtt) * it2) +
-                   tb.z * __builtin_amdgcn_exp2f((tb.x - mtt) * it2);
-            const float2 xa = kl_rebase(xpart[tid], a.x, ta.x, a.z, ta.z, m, mtt, g.lg.inv_t);
-            const float2 xb = kl_rebase(xpart[256 + tid], b.x, tb.x, b.z, tb.z, m, mtt, g.lg.inv_t);
-            kx = make_float2(xa.x + xb.x, xa.y + xb.y);
-          }
-          const int64_t r = orow - static_cast<int64_t>(tc.p) * g.M;
-          g.lg.stats[(g.M + r) * g.lg.stats_ld + tc.ntile] = st;
-          g.lg.cross[r * g.lg.stats_ld + tc.ntile] = kx;
-        }
-      }
-    }
-  }
+  gemm_epilogue<Elem<T>::kSize, EPI, LT, CT, kFrag>(g, pr, tc, acc, epi, smem, lab_pre);
 }
 
+
+// ------------------------------------------------- two workgroups on a CU
+// bf16 products on tiles of 128 x 256: 4 waves of 64 x 128, at most 256
+// registers a wave and 72 KB of LDS, so that two workgroups share a CU and one
+// computes while the other runs its epilogue, waits for its operands or fills
+// its ring. Half the tile rows also leave less work for padding and for a last
+// round. K advances one stage (32) at a time through a ring of three; an
+// iteration waits for its stage, starts the DMA of the stage two ahead into
+// the slot read one ago, reads its fragments and computes. Bound by LDS where
+// the CU is full: the two workgroups' 96 KB of fragment reads and 48 KB of DMA
+// a stage pair take 1150 cycles of the 1024 that their MFMAs do, so that long
+// products run at 0.7 to 0.8 of the larger tile's rate (mid_tiles).
+constexpr int kMidM = 128;
+constexpr int kMidFrag = 4;                     // fragments of A per wave
+constexpr int kMidA = kMidM * kSlab;            // bytes of A a stage
+constexpr int kMidRing = 3;
+constexpr int kMidX = kXfers + kXfers / 2;      // transfers per thread and stage
+
+template <bool BK, GemmEpilogue EPI, typename LT, bool CT>
+__device__ __forceinline__ void mid_body(const GemmArgs& g) {
+  constexpr bool kLogitsEpi = EPI == GemmEpilogue::Logits || EPI == GemmEpilogue::LogitsTeacher ||
+                              EPI == GemmEpilogue::LogitsTeacher16;
+  // A tiles of slots 0-2, then B tiles of slots 0-2.
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kMidRing * (kMidA + kOpBytes)];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int64_t Kl = g.K;
+  const TileCoord tc = map_tile<kMidM>(g, blockIdx.x);
+  const GemmProblem pr = g.prob[tc.p];
+  Loader<__bf16, true, kXfers / 2> la;
+  Loader<__bf16, BK> lb;
+  if (EPI == GemmEpilogue::Logits && g.lg.pair_rows > 0)
+    la.init_paired(pr.a, g.lg.pair_teacher, g.lda, g.lg.pair_rows, Kl, tc.m0 >> 1, wave, lane);
+  else
+    la.init(pr.a, g.lda, g.M, Kl, tc.m0, wave, lane);
+  lb.init(pr.b, g.ldb, g.N, Kl, tc.n0, wave, lane);
+  int64_t lab_pre = 0;   // as in gemm_body
+  if constexpr (kLogitsEpi) {
+    const int64_t R = static_cast<int64_t>(tc.m0) + tid;
+    const int64_t prs = g.lg.pair_rows;
+    const int64_t r = prs > 0 ? ((R >> 5) << 4) + (R & 15) : R;
+    const bool ok = tid < kMidM && (prs > 0 ? r < prs : R < g.M);
+    lab_pre = ok ? g.lg.labels[r] : g.lg.ignore_index;
+  }
+  f32x4 acc[kMidFrag][kFrag];
+#pragma unroll
+  for (int i = 0; i < kMidFrag; ++i)
+#pragma unroll
+    for (int j = 0; j < kFrag; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int SK = kSlab / 2;
+  const int nfull = static_cast<int>(Kl / SK);
+  const int nst = static_cast<int>((Kl + SK - 1) / SK);
+  auto tileA = [&](int sl) -> unsigned char* { return smem + sl * kMidA; };
+  auto tileB = [&](int sl) -> unsigned char* { return smem + kMidRing * kMidA + sl * kOpBytes; };
+  uint32_t lds0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)smem))));
+  asm volatile("" : "+s"(lds0));
+  const uint32_t m0wave = lds0 + static_cast<uint32_t>(wave) * 1024;
+  // The DMA of stage st into slot S (the partial last stage: issue() zeroes
+  // what lies past K).
+  auto dma = [&](auto slot_c, int st) {
+    constexpr int S = decltype(slot_c)::value;
+    if (st >= nst) return;
+    if (st >= nfull) {
+      la.issue(tileA(S), st, wave, lane);
+      lb.issue(tileB(S), st, wave, lane);
+      return;
+    }
+    const uint64_t sa = uniform64(la.stage_src(st)), sb = uniform64(lb.stage_src(st));
+    constexpr int MA = S * kMidA, MB = kMidRing * kMidA + S * kOpBytes;
+    dma16_at<MA>(sa, la.goff[0], m0wave);
+    dma16_at<MA + 4096>(sa, la.goff[1], m0wave);
+    dma16_at<MB>(sb, lb.goff[0], m0wave);
+    dma16_at<MB + 4096>(sb, lb.goff[1], m0wave);
+    dma16_at<MB + 2 * 4096>(sb, lb.goff[2], m0wave);
+    dma16_at<MB + 3 * 4096>(sb, lb.goff[3], m0wave);
+  };
+  FragReader<true, false> fa;
+  FragReader<BK, false> fb;
+  fa.init(lds0, wm * 64, lane);
+  fb.init(lds0 + kMidRing * kMidA, wn * 128, lane);
+  auto iter = [&](auto slot_c, int st) {
+    constexpr int S = decltype(slot_c)::value;
+    // Stage st has landed: of what this wave issued, only stage st+1's
+    // transfers may be in flight (kMidX of them when it is a full stage).
+    if (st + 1 < nfull) __builtin_amdgcn_s_waitcnt(vm_wait(kMidX));
+    else __builtin_amdgcn_s_waitcnt(kWaitAll);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    dma(SlotC<(S + 2) % kMidRing>{}, st + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 a[kMidFrag], b[kFrag];
+#pragma unroll
+    for (int i = 0; i < kMidFrag; ++i)
+      a[i] = *(const lds_u32x4*)(static_cast<uintptr_t>(fa.addr[0] + (i * 1024 + S * kMidA)));
+#pragma unroll
+    for (int o = 0; o < FragReader<BK, false>::kOps; ++o) fb.template read_op<S>(o, b);
+#pragma unroll
+    for (int j = 0; j < kFrag; ++j)
+#pragma unroll
+      for (int i = 0; i < kMidFrag; ++i) {
+        const bf16x8 x = __builtin_bit_cast(bf16x8, kLogitsEpi ? b[j] : a[i]);
+        const bf16x8 y = __builtin_bit_cast(bf16x8, kLogitsEpi ? a[i] : b[j]);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, acc[i][j], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  dma(SlotC<0>{}, 0);
+  dma(SlotC<1>{}, 1);
+  for (int st = 0; st < nst; st += 3) {
+    iter(SlotC<0>{}, st);
+    if (st + 1 < nst) iter(SlotC<1>{}, st + 1);
+    if (st + 2 < nst) iter(SlotC<2>{}, st + 2);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(kWaitAll);
+  __builtin_amdgcn_s_barrier();
+  mfma_drain();
+#pragma unroll
+  for (int i = 0; i < kMidFrag; ++i)
+#pragma unroll
+    for (int j = 0; j < kFrag; ++j) asm volatile("" : "+a"(acc[i][j]));
+  gemm_epilogue<2, EPI, LT, CT, kMidFrag>(g, pr, tc, acc, smem, smem, lab_pre);
+}
 
 // One named entry point per variant, so that profiles and the build's ISA
 // check can tell them apart: gemm_<A layout><B layout>[t]_<epilogue>_<input>
@@ -1861,11 +2005,24 @@ ORDA_GEMM3(gemm_kmt_store_bf16x3, false, GemmEpilogue::StoreF32, true)
 ORDA_GEMM3(gemm_kmt_accum_bf16x3, false, GemmEpilogue::AccumF32, true)
 #undef ORDA_GEMM3
 
+// The 128 x 256 tiles: gemm_<layouts>_mid_<epilogue>_bf16.
+#define ORDA_MID(NAME, BK, EPI, LT, CT) \
+  __global__ __launch_bounds__(kThreads, 2) void NAME(GemmArgs g) { mid_body<BK, EPI, LT, CT>(g); }
+ORDA_MID(gemm_kk_mid_logits_bf16_bf16, true, GemmEpilogue::Logits, __bf16, false)
+
+ORDA_MID(gemm_kk_mid_logits_bf16_f32, true, GemmEpilogue::Logits, float, false)
+ORDA_MID(gemm_kmt_mid_store_bf16, false, GemmEpilogue::StoreF32, float, true)
+ORDA_MID(gemm_kmt_mid_accum_bf16, false, GemmEpilogue::AccumF32, float, true)
+#undef ORDA_MID
 typedef void (*GemmKernel)(GemmArgs);
 
-GemmKernel select_kernel(const GemmArgs& g) {
+GemmKernel select_kernel(const GemmArgs& g, bool mid) {
   using E = GemmEpilogue;
   const bool bf = g.in_type == DType::BF16;
+  if (mid) {   // mid_tiles(g)
+    if (g.c_trans) return g.epi == E::StoreF32 ? gemm_kmt_mid_store_bf16 : gemm_kmt_mid_accum_bf16;
+    return g.logits_type == DType::BF16 ? gemm_kk_mid_logits_bf16_bf16 : gemm_kk_mid_logits_bf16_f32;
+  }
   if (g.plane_a > 0) {
     if (!bf || !g.a_kmajor) return nullptr;
     if (g.epi == E::Logits)
@@ -2621,6 +2778,34 @@ int64_t gemm_split_bytes(const GemmArgs& g) {
 bool gemm_small_tiles(const GemmArgs& g) { return small_f32(g); }
 
 namespace {
+// Whether launch_gemm runs g (a whole product) on the 128 x 256 tiles, two
+// workgroups a CU: bf16 logits without teacher logits beside them, and grad_W
+// computed transposed, where neither K nor the last round is split. The larger
+// tile is the better one per operation (the two workgroups' LDS traffic bounds
+// the smaller), the smaller one where the epilogue is long beside K or a round
+// is mostly empty. Both sides' cost in us, fitted to 140 shapes of 64 to 2000
+// rows, widths of 256 to 4096 and vocabularies of 8000 to 128256 (15 % off for
+// the logits, 9 % for grad_W): per round of 256 tiles, the last one of the
+// smaller with a CU to itself where 256 more do not follow. From nine tenths
+// on: at these sizes the logits then take 7 % less time and grad_W 3 %, none
+// over 5 % more; 64 x 512 x 128256 58 us against 41, 300 x 768 x 50257 (Tied) 99
+// against 84, 300 x 512 x 50257 80 against 60; at 2000 x 1536 x 128256, where
+// the rule keeps the larger tile, 737 against 957.
+bool mid_tiles(const GemmArgs& g) {
+  const bool logits = g.epi == GemmEpilogue::Logits;
+  if (g.in_type != DType::BF16 || g.plane_a > 0 || !g.a_kmajor || g.M <= 0 || g.N <= 0) return false;
+  if (logits ? (!g.b_kmajor || g.c_trans || g.lg.teacher_logits != nullptr) : (g.b_kmajor || !g.c_trans))
+    return false;
+  if (!logits && (plan_split(g).splits > 1 || plan_tail(g).at > 0)) return false;
+  const double s = static_cast<double>(g.K) / 32;
+  const int64_t rounds = (tile_count(g) + 255) / 256;
+  const int64_t halves =
+      (((g.M + kMidM - 1) / kMidM) * ((g.N + kTile - 1) / kTile) * g.nprob + 255) / 256;
+  const double large = logits ? rounds * (0.71 * s + 14.4) + 4.9 : rounds * (0.74 * s + 13.9) + 4.2;
+  const double small = logits ? halves / 2 * (1.08 * s + 9.2) + halves % 2 * (0.63 * s + 5.5) + 8.7
+                              : halves / 2 * (0.94 * s + 13.7) + halves % 2 * (0.53 * s + 4.3) + 0.7;
+  return small < 0.9 * large;
+}
 hipError_t launch_gemm_impl(const GemmArgs& g, hipStream_t stream, bool whole);
 }  // namespace
 
@@ -2661,10 +2846,17 @@ hipError_t launch_gemm_impl(const GemmArgs& g, hipStream_t stream, bool whole) {
       return launch_gemm_impl(tail_part(g, ts, true), stream, false);
     }
   }
-  const int64_t tiles = ((g.M + kTile - 1) / kTile) * ((g.N + kTile - 1) / kTile) * g.nprob;
+  const bool mid = whole && mid_tiles(g);
+  const int64_t tiles = mid ? ((g.M + kMidM - 1) / kMidM) * ((g.N + kTile - 1) / kTile) * g.nprob
+                            : tile_count(g);
   GemmArgs gr = g;
-  set_share_blocks(gr);
-  set_band_blocks(gr);
+  if (mid) {
+    gr.sh_a = 0;
+    gr.group_m *= 2;   // the rows of a raster group
+  } else {
+    set_share_blocks(gr);
+    set_band_blocks(gr);
+  }
   const SplitPlan sp = plan_split(g);
   if (sp.splits > 1 && g.split_ws != nullptr && g.split_ws_bytes >= sp.bytes) {
     // Partials of every split with the Store epilogue (alpha 1), in C's
@@ -2679,7 +2871,7 @@ hipError_t launch_gemm_impl(const GemmArgs& g, hipStream_t stream, bool whole) {
     s.split_stride = sp.stride;
     const int64_t rows = g.c_trans ? g.N : g.M, cols = g.c_trans ? g.M : g.N;
     for (int p = 0; p < g.nprob; ++p) s.prob[p].c = g.split_ws + p * rows * sp.ldp;
-    const GemmKernel k = select_kernel(s);
+    const GemmKernel k = select_kernel(s, false);
     if (k == nullptr) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(tiles * sp.splits)), dim3(kThreads), 0,
                        stream, s);
@@ -2695,7 +2887,7 @@ hipError_t launch_gemm_impl(const GemmArgs& g, hipStream_t stream, bool whole) {
   if (g.partials_only) return hipErrorInvalidValue;   // not split
   GemmArgs one = gr;
   one.split_k = 1;
-  const GemmKernel k = select_kernel(one);
+  const GemmKernel k = select_kernel(one, mid);
   if (k == nullptr) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, stream, one);
   return hipGetLastError();
