@@ -574,9 +574,8 @@ bool use_planes3(const LossPlan& P) {
 // to 1.2e-5 relative, and those are held to 1e-5 of an fp32 product's
 // (tests/test_gpu_full_size.py). Accumulated in the same order the two differ
 // by 5e-6; over planes, though nearer to float64, by 1.5e-5.
-bool planes3_logits(const LossPlan& P) {
-  return P.planes3 && !(P.need_teacher && P.mode == ORDA_TEACHER_TIED);
-}
+bool fp32_logits(const LossPlan& P) { return P.need_teacher && P.mode == ORDA_TEACHER_TIED; }
+bool planes3_logits(const LossPlan& P) { return P.planes3 && !fp32_logits(P); }
 
 // Device bytes of the three-plane buffers of a call whose groups hold `cap`
 // rows: the weights, and the rows' share (as run_loss sizes them).
@@ -812,6 +811,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       f.lg.cross = cross;
     }
     f.group_m = 8;
+    f.fp32_mfma = fp32_logits(P);
     if (p3_logits) {
       timed(c, ORDA_KERNEL_OTHER, [&] {
         const hipError_t e = launch_split3_rows(reinterpret_cast<const float*>(at(in.hs.p, gs * in.hs.ld, dt)),

@@ -2323,22 +2323,25 @@ double split_us(const GemmArgs& g, const SplitPlan& sp) {
 // ------------------------------------------------------- small fp32 products
 // fp32 Store/Accum products with at most 64 tiles of 256 x 256 (a quarter of
 // the CUs) run on 128 x 128 workgroup tiles instead: four times the
-// workgroups, so that K is split less finely or not at all. With 256-wide
-// tiles such a product splits K into slices of 128 (at BT=256, H=512,
-// V=8192: the logits into 4, grad_hidden into 64, grad_W into 4), and each
-// workgroup then spends about as long on its 256 KB of partials and on
-// filling its operand ring as on its 16.8 MFLOP. A kernel of its own: 4
-// waves of 64 x 64 (4 x 4 fragments of v_mfma_f32_16x16x4_f32), operands
-// read from global memory into registers one K stage (32) ahead and stored
-// to LDS transposed ([k][row], so that the 16 lanes of a fragment read 16
-// consecutive floats), two LDS stages (72 KB). A stage's fragments are all
-// read from LDS before its MFMAs (64 registers), so that only the first read
-// of a stage waits; left to the scheduler, every 4 K rows waited for their
-// reads between MFMAs.
+// workgroups, so that K is split less finely or not at all. A kernel of its
+// own: 4 waves of 64 x 64, K in stages of 32 through two LDS buffers; operands
+// are read from global memory into registers two stages ahead (a row's 128
+// bytes of a stage by 8 adjacent lanes, whole lines), and a stage is stored to
+// LDS beside the MFMAs of the one before. Bound by latency: one workgroup a CU,
+// a barrier a stage. (With a guard around each load every load waited for the
+// one before, 64-byte runs of a row a thread, one stage ahead, on the fp32
+// MFMA: Tied 256 x 512 x 8192 223 us a call against 208, 300 x 768 x 3000 259
+// against 224, Separate 128 x (512, 1024) x 16000 240 against 227.)
+//   X3: the values go to LDS as three bf16 planes (split3.h) and each product
+//   is the six plane products of the large three-plane kernels, on the bf16
+//   matrix units: 96 MFMAs of 16 cycles a wave and stage instead of 128 of 32.
+//   K-major planes are [row][64 B], N-major ones [k][256 B], swizzled and read
+//   as the large kernels' stages.
+//   else: fp32 values, [row][36 floats] (two b128 reads a fragment row without
+//   bank conflicts), v_mfma_f32_16x16x4_f32.
 constexpr int kSmTile = 128;
 constexpr int kSmK = 32;
-constexpr int kSmPer = kSmTile * kSmK / 256;   // floats of each operand per thread and stage
-constexpr int kSmPitch = kSmTile + 16;   // floats per LDS K row: the 4 K rows of a read in 4 bank groups
+constexpr int kSmPitch = kSmK + 4;
 
 int64_t small_tiles(const GemmArgs& g) {
   return ((g.M + kSmTile - 1) / kSmTile) * ((g.N + kSmTile - 1) / kSmTile) * g.nprob;
@@ -2360,7 +2363,7 @@ bool small_f32(const GemmArgs& g) {
 // 256 workgroups: Tied 64 x 256 x 2048 134 us a call against 117, Precomputed
 // 300 x 300 x 5000 193 against 167, Tied 300 x 768 x 3000 284 against 260, 256 x
 // 512 x 8192 the same; two workgroups a CU, 512 in all, were slower there, 253
-// against 223.)
+// against 223; all before the kernel's present loads.)
 SplitPlan plan_split_small(const GemmArgs& g) {
   SplitPlan sp{1, g.K, 0, 0, 0};
   if (g.K <= 0) return sp;
@@ -2397,10 +2400,12 @@ SplitPlan plan_split_small(const GemmArgs& g) {
 // before the scale, as the big kernel's AccumF32 does. Workgroup w < tiles
 // * split_k: split w / tiles over K range [s * split_len, +split_len),
 // partials at C + s * split_stride.
-template <bool BK, bool CT, bool ACC>
+template <bool BK, bool CT, bool ACC, bool X3>
 __device__ __forceinline__ void small_body(const GemmArgs& g) {
-  __shared__ __attribute__((aligned(16))) float sA[2][kSmK][kSmPitch];
-  __shared__ __attribute__((aligned(16))) float sB[2][kSmK][kSmPitch];
+  static_assert(X3 || BK, "the fp32 MFMA form takes K-major operands");
+  constexpr int kPlane = kSmTile * kSlab;                       // one plane of an operand's stage
+  constexpr int kOp = X3 ? 3 * kPlane : kSmTile * kSmPitch * 4;   // an operand's stage
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * kOp];   // buffer b: A, B at 2b, 2b+1
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int64_t mt = (g.M + kSmTile - 1) / kSmTile, nt = (g.N + kSmTile - 1) / kSmTile;
@@ -2420,64 +2425,70 @@ __device__ __forceinline__ void small_body(const GemmArgs& g) {
   const float* A = static_cast<const float*>(g.prob[p].a);
   const float* B = static_cast<const float*>(g.prob[p].b);
   float* C = static_cast<float*>(g.prob[p].c) + static_cast<int64_t>(split) * g.split_stride;
-  const bool avec = (reinterpret_cast<uintptr_t>(A) % 16) == 0 && (g.lda % 4) == 0;
-  const bool bvec = (reinterpret_cast<uintptr_t>(B) % 16) == 0 && (g.ldb % 4) == 0;
-
-  // Global loads of one stage: kSmPer consecutive floats of each operand
-  // per thread.
-  //   K-major operand: tile row tid % 128, K columns kSmPer * (tid / 128) + i;
-  //   N-major B: K row tid / kBRow, columns kSmPer * (tid % kBRow) + i, with
-  //   kBRow = 128 / kSmPer threads per K row.
-  constexpr int kBRow = kSmTile / kSmPer;
-  static_assert(2 * kSmPer == kSmK && 256 / kBRow == kSmK, "a stage is 256 threads x kSmPer floats");
-  const int kr = tid & 127, kq = (tid >> 7) * kSmPer;
-  const int br = tid / kBRow, bq = (tid % kBRow) * kSmPer;
-  float ra[kSmPer], rb[kSmPer];
-  auto load_run = [&](const float* src, bool whole, int64_t avail, float (&r)[kSmPer]) {
-    if (whole) {
+  // Global loads of one stage, four vectors of 4 floats of each operand per
+  // thread: a K-major operand's tile rows tid / 8 + 32v, K columns 4 (tid % 8);
+  // N-major B's K rows tid / 32 + 8v, columns 4 (tid % 32). Rows and columns
+  // past the operand's edge are clamped to its last ones (their outputs are
+  // not stored; pitches are multiples of 8, so that a vector that starts inside
+  // a row lies in it), so that a whole stage loads without a branch: a guard
+  // around each load made each wait for the one before. Only the last,
+  // partial stage takes single elements and zeros past K.
+  const int kr = tid >> 3, kc = 4 * (tid & 7);
+  const int br = tid >> 5, bc = 4 * (tid & 31);
+  const float *pa[4], *pb[4];
 #pragma unroll
-      for (int v = 0; v < kSmPer / 4; ++v) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(src + 4 * v);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[4 * v + i] = x[i];
-      }
+  for (int v = 0; v < 4; ++v) {
+    const int64_t ma = m0 + kr + 32 * v < g.M ? m0 + kr + 32 * v : g.M - 1;
+    pa[v] = A + ma * g.lda + kbeg + kc;
+    if constexpr (BK) {
+      const int64_t nb = n0 + kr + 32 * v < g.N ? n0 + kr + 32 * v : g.N - 1;
+      pb[v] = B + nb * g.ldb + kbeg + kc;
     } else {
+      const int64_t nb = n0 + bc < g.N ? n0 + bc : (g.N - 1) / 4 * 4;
+      pb[v] = B + (kbeg + br + 8 * v) * g.ldb + nb;
+    }
+  }
+  const int64_t kl = kend > kbeg ? kend - kbeg : 0;
+  const int64_t nfull = kl / kSmK;
+  auto load = [&](int64_t st, f32x4 (&ra)[4], f32x4 (&rb)[4]) {   // a whole stage
+    const int64_t k0 = st * kSmK;
 #pragma unroll
-      for (int i = 0; i < kSmPer; ++i) r[i] = i < avail ? src[i] : 0.f;
+    for (int v = 0; v < 4; ++v) ra[v] = *reinterpret_cast<const f32x4*>(pa[v] + k0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) rb[v] = *reinterpret_cast<const f32x4*>(pb[v] + (BK ? k0 : k0 * g.ldb));
+  };
+  auto load_part = [&](f32x4 (&ra)[4], f32x4 (&rb)[4]) {   // what is left of K, zeros past it
+    const int64_t k0 = nfull * kSmK;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ra[v][e] = k0 + kc + e < kl ? pa[v][k0 + e] : 0.f;
+        if constexpr (BK) rb[v][e] = k0 + kc + e < kl ? pb[v][k0 + e] : 0.f;
+      }
+      if constexpr (!BK) {
+        rb[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (k0 + br + 8 * v < kl) rb[v] = *reinterpret_cast<const f32x4*>(pb[v] + k0 * g.ldb);
+      }
     }
   };
-  // A run outside the operand (avail <= 0) loads nothing; its address is
-  // formed but never read (clamping it to row 0 made the kernels 10 %
-  // slower).
-  auto load_kmajor = [&](const float* X, int64_t ld, int64_t rows, int64_t r0, bool vec, int64_t k0,
-                         float (&r)[kSmPer]) {
-    const int64_t row = r0 + kr, k = k0 + kq;
-    const int64_t avail = row < rows ? kend - k : 0;   // elements of the run inside K
-    load_run(X + row * ld + k, vec && avail >= kSmPer, avail, r);
-  };
-  auto load_nmajor = [&](int64_t k0, float (&r)[kSmPer]) {
-    const int64_t k = k0 + br, n = n0 + bq;
-    const int64_t avail = k < kend ? g.N - n : 0;
-    load_run(B + k * g.ldb + n, bvec && avail >= kSmPer, avail, r);
-  };
-  auto load = [&](int64_t k0) {
-    load_kmajor(A, g.lda, g.M, m0, avec, k0, ra);
-    if constexpr (BK) load_kmajor(B, g.ldb, g.N, n0, bvec, k0, rb);
-    else load_nmajor(k0, rb);
-  };
-  auto store = [&](int buf) {
+  // The loaded stage into LDS operand `base`: vector v of a K-major operand
+  // (row kr + 32v) or of N-major B (K row br + 8v).
+  auto store = [&](unsigned char* base, const f32x4 (&r)[4], auto kmajor_c) {
+    constexpr bool kKmajor = decltype(kmajor_c)::value != 0;
 #pragma unroll
-    for (int i = 0; i < kSmPer; ++i) sA[buf][kq + i][kr] = ra[i];
-    if constexpr (BK) {
+    for (int v = 0; v < 4; ++v) {
+      if constexpr (X3) {
+        uint32_t lo[3], hi[3];
+        split3_pack(r[v][0], r[v][1], lo);
+        split3_pack(r[v][2], r[v][3], hi);
+        int off;
+        if constexpr (kKmajor) off = kmaj_off(kr + 32 * v, kc >> 3) + (kc & 4) * 2;
+        else off = (br + 8 * v) * 256 + (((bc >> 3) ^ mnb_swz(br + 8 * v)) << 4) + (bc & 4) * 2;
 #pragma unroll
-      for (int i = 0; i < kSmPer; ++i) sB[buf][kq + i][kr] = rb[i];
-    } else {
-#pragma unroll
-      for (int v = 0; v < kSmPer / 4; ++v) {
-        f32x4 x;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = rb[4 * v + i];
-        *reinterpret_cast<f32x4*>(&sB[buf][br][bq + 4 * v]) = x;
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x2*>(base + k * kPlane + off) = u32x2{lo[k], hi[k]};
+      } else {
+        *reinterpret_cast<f32x4*>(base + ((kr + 32 * v) * kSmPitch + kc) * 4) = r[v];
       }
     }
   };
@@ -2487,108 +2498,149 @@ __device__ __forceinline__ void small_body(const GemmArgs& g) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // MFMA ks of a stage takes K row 4 * ks + lane / 16 of the stage: lane
-  // (m, q) = (lane % 16, lane / 16) gives A[row m][k] and B[k][column m].
   const int lm = lane & 15, lq = lane >> 4;
-  const int64_t nst = kend > kbeg ? (kend - kbeg + kSmK - 1) / kSmK : 0;
   auto compute = [&](int buf) {
-    float fa[kSmK / 4][4], fb[kSmK / 4][4];
+    const unsigned char* const pa = smem + buf * 2 * kOp;
+    const unsigned char* const pb = pa + kOp;
+    if constexpr (X3) {
+      bf16x8 a[3][4], b[3][4];
 #pragma unroll
-    for (int ks = 0; ks < kSmK / 4; ++ks) {
+      for (int k = 0; k < 3; ++k) {
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        fa[ks][f] = sA[buf][4 * ks + lq][wm * 64 + f * 16 + lm];
-        fb[ks][f] = sB[buf][4 * ks + lq][wn * 64 + f * 16 + lm];
+        for (int f = 0; f < 4; ++f) {
+          a[k][f] = __builtin_bit_cast(
+              bf16x8, *reinterpret_cast<const u32x4*>(pa + k * kPlane + kmaj_off(wm * 64 + f * 16 + lm, lq)));
+          if constexpr (BK) {
+            b[k][f] = __builtin_bit_cast(
+                bf16x8, *reinterpret_cast<const u32x4*>(pb + k * kPlane + kmaj_off(wn * 64 + f * 16 + lm, lq)));
+          } else {
+            u32x4 w;
+            const int c = (wn * 64 + f * 16 + 4 * (lm & 3)) >> 3;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int row = 8 * lq + 4 * h + (lm >> 2);
+              const int off = k * kPlane + row * 256 + ((c ^ mnb_swz(row)) << 4) + (lm & 1) * 8;
+              const u32x2 v = __builtin_bit_cast(
+                  u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(pb + off)));
+              w[2 * h] = v[0];
+              w[2 * h + 1] = v[1];
+            }
+            b[k][f] = __builtin_bit_cast(bf16x8, w);
+          }
+        }
       }
+      constexpr int kA[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kA[q]][i], b[kB[q]][j], acc[i][j], 0, 0, 0);
+    } else {
+      // lane (lm, lq) holds K columns 8 lq .. 8 lq + 7 of its row; MFMA ks
+      // takes column 8 lq + ks of both operands
+      f32x4 a[4][2], b[4][2];
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = 8 * lq + 4 * h;
+          a[f][h] = *reinterpret_cast<const f32x4*>(pa + ((wm * 64 + f * 16 + lm) * kSmPitch + k) * 4);
+          b[f][h] = *reinterpret_cast<const f32x4*>(pb + ((wn * 64 + f * 16 + lm) * kSmPitch + k) * 4);
+        }
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][ks >> 2][ks & 3], b[j][ks >> 2][ks & 3],
+                                                             acc[i][j], 0, 0, 0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < kSmK / 4; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[ks][i], fb[ks][j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
   };
-  if (nst > 0) {
-    load(kbeg);
-    store(0);
-  }
-  __syncthreads();
-  for (int64_t st = 0; st < nst; ++st) {
-    const int buf = static_cast<int>(st & 1);
-    if (st + 1 < nst) load(kbeg + (st + 1) * kSmK);
-    compute(buf);
-    if (st + 1 < nst) store(buf ^ 1);
+  f32x4 la[2][4], lb[2][4];
+  auto put = [&](int buf, const f32x4 (&ra)[4], const f32x4 (&rb)[4]) {
+    unsigned char* const pa = smem + buf * 2 * kOp;
+    store(pa, ra, SlotC<1>{});
+    store(pa + kOp, rb, SlotC<(BK ? 1 : 0)>{});
+  };
+  // Stage st: in buffer st % 2; stage st + 1 in registers, st + 2 on its way.
+  // No branch but the loop's, so that the waits count single loads; past the
+  // last whole stage it is loaded and stored again, for nobody.
+  auto stage = [&](auto s_c, int64_t st) {
+    constexpr int S = decltype(s_c)::value;
+    load(st + 2 < nfull ? st + 2 : nfull - 1, la[S], lb[S]);
+    compute(S);
+    put(S ^ 1, la[S ^ 1], lb[S ^ 1]);
     __syncthreads();
+  };
+  if (nfull > 0) {
+    load(0, la[0], lb[0]);
+    load(nfull > 1 ? 1 : 0, la[1], lb[1]);
+    put(0, la[0], lb[0]);
+    __syncthreads();
+    int64_t st = 0;
+    for (; st + 1 < nfull; st += 2) {
+      stage(SlotC<0>{}, st);
+      stage(SlotC<1>{}, st + 1);
+    }
+    if (st < nfull) stage(SlotC<0>{}, st);
+  }
+  if (nfull * kSmK < kl) {
+    load_part(la[0], lb[0]);
+    put(0, la[0], lb[0]);
+    __syncthreads();
+    compute(0);
   }
 
-  // acc[i][j][e] is row wm*64 + 16i + 4*lq + e, column wn*64 + 16j + lm.
+  // acc[i][j][e] is row wm*64 + 16i + 4*lq + e, column wn*64 + 16j + lm. A tile
+  // inside C stores without a test for each element.
   const float alpha = g.alpha_ptr != nullptr ? g.alpha * *g.alpha_ptr : g.alpha;
+  const int64_t M = g.M, N = g.N, ldc = g.ldc;
   const int64_t row_w = m0 + wm * 64 + 4 * lq;
   const int64_t col_l = n0 + wn * 64 + lm;
-  if constexpr (CT) {
-    const bool vec = (g.ldc % 4) == 0 && (reinterpret_cast<uintptr_t>(C) % 16) == 0;
+  const bool inside = m0 + kSmTile <= M && n0 + kSmTile <= N &&
+                      (!CT || ((ldc % 4) == 0 && (reinterpret_cast<uintptr_t>(C) % 16) == 0));
+  if (inside) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t n = col_l + j * 16;
-      if (n >= g.N) continue;
-      float* cn = C + n * g.ldc;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t m = row_w + i * 16;
-        f32x4 v = acc[i][j];
-        if (vec && m + 4 <= g.M) {
-          f32x4* dst = reinterpret_cast<f32x4*>(cn + m);
-          if constexpr (ACC) v = alpha * (*dst + v);
-          else v = alpha * v;
-          *dst = v;
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (CT) {
+          f32x4* dst = reinterpret_cast<f32x4*>(C + (col_l + j * 16) * ldc + row_w + i * 16);
+          *dst = ACC ? alpha * (*dst + acc[i][j]) : alpha * acc[i][j];
         } else {
+          float* dst = C + (row_w + i * 16) * ldc + col_l + j * 16;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (m + e < g.M) {
-              float x = v[e];
-              if constexpr (ACC) x = alpha * (cn[m + e] + x);
-              else x = alpha * x;
-              cn[m + e] = x;
-            }
-          }
+          for (int e = 0; e < 4; ++e) dst[e * ldc] = ACC ? alpha * (dst[e * ldc] + acc[i][j][e]) : alpha * acc[i][j][e];
         }
       }
-    }
-  } else {
+    return;
+  }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t row = row_w + i * 16 + e;
-        if (row >= g.M) continue;
-        float* crow = C + row * g.ldc;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t col = col_l + j * 16;
-          if (col < g.N) {
-            float v = acc[i][j][e];
-            if constexpr (ACC) v = alpha * (crow[col] + v);
-            else v = alpha * v;
-            crow[col] = v;
-          }
-        }
+        const int64_t row = row_w + i * 16 + e, col = col_l + j * 16;
+        if (row >= M || col >= N) continue;
+        float* dst = CT ? C + col * ldc + row : C + row * ldc + col;
+        *dst = ACC ? alpha * (*dst + acc[i][j][e]) : alpha * acc[i][j][e];
       }
-    }
-  }
 }
 
 // One named entry point per variant, as for the 256-wide kernels:
-// gemm_<A layout><B layout>[t]_small[_accum]_f32.
-#define ORDA_SMALL(NAME, BK, CT, ACC) \
-  __global__ __launch_bounds__(256) void NAME(GemmArgs g) { small_body<BK, CT, ACC>(g); }
-ORDA_SMALL(gemm_kk_small_f32, true, false, false)
-ORDA_SMALL(gemm_km_small_f32, false, false, false)
-ORDA_SMALL(gemm_km_small_accum_f32, false, false, true)
-ORDA_SMALL(gemm_kmt_small_f32, false, true, false)
-ORDA_SMALL(gemm_kmt_small_accum_f32, false, true, true)
+// gemm_<A layout><B layout>[t]_small[_accum]_<f32: fp32 MFMA, x3: planes>.
+#define ORDA_SMALL(NAME, BK, CT, ACC, X3) \
+  __global__ __launch_bounds__(256, 1) void NAME(GemmArgs g) { small_body<BK, CT, ACC, X3>(g); }
+ORDA_SMALL(gemm_kk_small_f32, true, false, false, false)
+ORDA_SMALL(gemm_kk_small_x3, true, false, false, true)
+ORDA_SMALL(gemm_km_small_x3, false, false, false, true)
+ORDA_SMALL(gemm_km_small_accum_x3, false, false, true, true)
+ORDA_SMALL(gemm_kmt_small_x3, false, true, false, true)
+ORDA_SMALL(gemm_kmt_small_accum_x3, false, true, true, true)
 #undef ORDA_SMALL
 
 // g with small_f32(g): split K over the small tiles where plan_split_small
@@ -2596,10 +2648,10 @@ ORDA_SMALL(gemm_kmt_small_accum_f32, false, true, true)
 // reduction applying g's epilogue), else one launch.
 hipError_t launch_small(const GemmArgs& g, hipStream_t stream) {
   using K = void (*)(GemmArgs);
-  auto pick = [](bool bk, bool ct, bool acc) -> K {
-    if (bk) return acc ? nullptr : gemm_kk_small_f32;
-    if (ct) return acc ? gemm_kmt_small_accum_f32 : gemm_kmt_small_f32;
-    return acc ? gemm_km_small_accum_f32 : gemm_km_small_f32;
+  auto pick = [&](bool bk, bool ct, bool acc) -> K {
+    if (bk) return acc ? nullptr : g.fp32_mfma ? gemm_kk_small_f32 : gemm_kk_small_x3;
+    if (ct) return acc ? gemm_kmt_small_accum_x3 : gemm_kmt_small_x3;
+    return acc ? gemm_km_small_accum_x3 : gemm_km_small_x3;
   };
   const int64_t tiles = small_tiles(g);
   const SplitPlan sp = plan_split_small(g);

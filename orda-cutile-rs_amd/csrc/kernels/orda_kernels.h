@@ -126,6 +126,9 @@ struct GemmArgs {
   // reduction (the caller reduces them, e.g. launch_row_stats with
   // src_splits). Only for products gemm_split_plan splits whole.
   bool partials_only;
+  // fp32 operands: keep to the fp32 MFMA where launch_gemm would split the
+  // values into planes itself (small products).
+  bool fp32_mfma;
 };
 
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);

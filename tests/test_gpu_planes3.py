@@ -1,5 +1,6 @@
-"""fp32 products over three-plane operands (from 2^34 operations a call on),
-against a float64 restatement: widths, vocabularies and row counts that are
+"""fp32 products over three-plane operands (planes made beforehand from 2^34
+operations a call on, by the small products' own kernel below), against a
+float64 restatement: widths, vocabularies and row counts that are
 not multiples of the 64-element K blocks or the 256-wide tiles, every teacher
 mode, gradient rows from the fused and from the chunked row pass, two and more
 staging groups, and a memory limit that the planes do not fit.
@@ -36,6 +37,11 @@ CASES = {
     "precomputed-in-place": ("precomputed", 1000, 264, 0, 11000, 0.0, 1),
     "precomputed-copied": ("precomputed", 1000, 264, 0, 11003, 0.0, 1),
     "student-ce": ("none", 1000, 264, 0, 11003, 0.0, 1),
+    # few operations: the small kernel splits the values itself
+    "small-tied": ("tied", 90, 100, 100, 3001, 1.0, 1),
+    "small-separate": ("separate", 71, 33, 77, 2050, 1.0, 2),
+    "small-precomputed": ("precomputed", 129, 130, 0, 1027, 0.0, 1),
+    "small-student-ce": ("none", 5, 7, 0, 131, 0.0, 1),
 }
 
 
