@@ -362,6 +362,7 @@ def vendor_gemms(torch, wl, dev, s, w, t, reps):
 KERNEL_CLASSES = (
     # (substring of the kernel name, kernel kind)
     ("gemm_kk_logits_", "gemm_logits"),
+    ("gemm_kk_mid_", "gemm_logits"),        # 128 x 256 tiles
     ("gemm_kk_store_", "gemm_logits"),      # small fp32 problems: logits split over K
     ("gemm_kk_small_", "gemm_logits"),      # ... or on 128 x 128 tiles
     ("gemm_km_small_", "gemm_grad_hidden"),
@@ -370,6 +371,7 @@ KERNEL_CLASSES = (
     ("gemm_kmt_", "gemm_grad_weight"),
     ("splitk_reduce", "splitk_reduce"),   # split-K: ordered sum of the partials
     ("transpose_rows", "transpose_rows"),   # grad_W's A operand: hidden rows transposed
+    ("split3", "split3_planes"),          # fp32 rows as three bf16 planes (transposed or not)
     ("row_pass_", "row_pass"),            # row_pass_fused_kernel, row_pass_kernel
     ("row_consts_", "row_consts"),        # the chunked row pass: per-row constants ...
     ("row_grad_", "row_grad"),            # ... and the elementwise gradient
