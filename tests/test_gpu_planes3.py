@@ -123,3 +123,28 @@ def test_planes3_give_way_to_a_memory_limit():
             d = getattr(got, k).double() - getattr(want, k).double()
             assert float(d.norm() / getattr(want, k).double().norm()) <= 1e-5, k
     ctx.close()
+
+
+# An infinite weight (a vocabulary entry masked out): with hidden rows of one
+# sign its logits are -inf, its probabilities 0, and loss and weight gradient
+# finite, as an fp32 product gives them; the hidden gradients are 0 times an
+# infinity. The smaller call runs on the small kernel. Bounds: fp32 loss terms
+# and gradients (1e-4, 1e-3), as against the oracle elsewhere.
+@pytest.mark.parametrize("bt,h,v", [(70, 130, 1030), (512, 520, 11008)])
+def test_infinite_weight_masks_its_column(bt, h, v):
+    import torch
+    s, w = np.abs(normal((bt, h), 1)) + np.float32(0.01), normal((v, h), 2, 1.0 / np.sqrt(h))
+    y = uniform_labels(bt, v - 2, 3)
+    w[v - 2] = -np.inf
+    opts = LossOptions(kd_weight=0.0, teacher_ce_weight=0.0, label_smoothing=0.0)
+    dev = lambda a: torch.from_numpy(a).to("cuda:0")
+    got = H.distillation_loss(dev(s), dev(w), dev(y), Teacher.Precomputed(dev(normal((bt, v), 4))), opts)
+    x = torch.from_numpy(s).double() @ torch.from_numpy(w).double().T
+    p = torch.softmax(x, dim=1)
+    yt = torch.from_numpy(y)
+    loss = -torch.log_softmax(x, dim=1)[torch.arange(bt), yt].mean().item()
+    p[torch.arange(bt), yt] -= 1.0
+    gw = (p.T @ torch.from_numpy(s).double() / bt).numpy()
+    assert abs(got.student_ce - loss) <= 1e-4 * abs(loss)
+    assert rel(got.grad_weight, gw) <= 1e-3
+    assert torch.isnan(got.grad_student_hidden).all()
