@@ -26,6 +26,17 @@ sys.path.insert(0, os.path.join(ROOT, "orda-cutile-rs_amd"))
 PEAK_HBM_GBS = 8000.0           # MI355X HBM3E, GB/s
 PEAK_MFMA_TFLOPS = {"bf16": 2500.0, "f32": 157.3}   # dense
 
+
+def mfma_peak(wl, kind):
+    """What the matrix units give the product `kind` at most, in TFLOP/s of
+    its own work: an fp32 product is six bf16 products of three-plane operands,
+    except a Tied teacher's logits, which run on the fp32 MFMA."""
+    dt = compute_dtype(wl)
+    if dt == "f32" and not (wl[0] == "tied" and kind == "gemm_logits"):
+        return round(PEAK_MFMA_TFLOPS["bf16"] / 6, 1)
+    return PEAK_MFMA_TFLOPS[dt]
+
+
 WORKLOADS = {
     # name: (teacher, BT, H, Ht, V, dtype, kd, T, alpha, w_t, quant[, profile])
     "tied-8192x4096x131072-bf16-int8": ("tied", 8192, 4096, 4096, 131072, "bf16", 0.4, 1.5, 0.1,
@@ -596,7 +607,7 @@ def main():
         per_step = amount
         if bound == "mfma":
             achieved = per_step * args.steps / (ms * 1e-3) / 1e12
-            peak = PEAK_MFMA_TFLOPS[dt]
+            peak = mfma_peak(wl, kind)
             unit = "TFLOP/s"
         else:
             achieved = per_step * args.steps / (ms * 1e-3) / 1e9
