@@ -69,9 +69,11 @@ __device__ __forceinline__ float2 rebase(float2 c, float4 s, float4 t, float Ms,
   return make_float2(c.x, s.z * __builtin_amdgcn_exp2f((s.x - Ms) * it2) -
                               t.z * __builtin_amdgcn_exp2f((t.x - Mt) * it2));
 }
-// A statistic's two exponential sums relative to a larger maximum.
+// A statistic's two exponential sums relative to a larger maximum. The maximum
+// skips NaN: a range without another value has -inf beside sums of NaN, which
+// times 0 stay NaN, while those of a range that is -inf throughout are 0.
 __device__ __forceinline__ float2 rescale(float4 v, float m, float it2) {
-  if (v.x == -INFINITY) return make_float2(0.f, 0.f);
+  if (v.x == -INFINITY) return make_float2(v.y * 0.f, v.z * 0.f);
   return make_float2(v.y * __builtin_amdgcn_exp2f((v.x - m) * kLog2e),
                      v.z * __builtin_amdgcn_exp2f((v.x - m) * it2));
 }

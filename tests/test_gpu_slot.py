@@ -114,3 +114,29 @@ def test_slot_masked_vocabulary():
     lg[n:, 4096:8192] = 0.0
     got = H.kl_ce_on_logits_chunk(lg, y, n, 1.0, 0.4, 1.0, 1.0, 1.0, 0.0, IGNORE, False, True)
     assert bool(torch.isposinf(got["kl_per_row"]).all())
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.1])
+@pytest.mark.parametrize("v,lo", [(4097, 4096), (8193, 8192), (64 * 4096 + 1, 64 * 4096), (3 * 4096, 4096)])
+def test_slot_keeps_nan(v, lo, alpha):
+    """A row pair with NaN throughout one segment of either row (a last segment
+    of one column, a whole one): the losses and gradients that read that row
+    are NaN in every column, the others what they are without it."""
+    import torch
+    n, hi = 3, min(lo + 4096, v)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(v)
+    lg = torch.empty((2 * n, v), device="cuda").normal_(0, 2.0, generator=g)
+    y = torch.full((n,), 9, device="cuda", dtype=torch.int32)
+    call = lambda x: H.kl_ce_on_logits_chunk(x, y, n, 1.0, 0.4, 1.0, 1.0, 1.0, alpha, IGNORE, False, True)
+    clean = call(lg)
+    lg[0, lo:hi] = float("nan")        # pair 0: the student's row
+    lg[n + 1, lo:hi] = float("nan")    # pair 1: the teacher's
+    got = call(lg)
+    lost = {"ce_loss": [0, n + 1], "grad_ce": [0, n + 1], "kl_per_row": [0, 1], "grad_kl_student": [0, 1]}
+    for k, rows in lost.items():
+        for r in range(got[k].shape[0]):
+            if r in rows:
+                assert bool(torch.isnan(got[k][r]).all()), (k, r)
+            else:
+                assert torch.equal(got[k][r], clean[k][r]), (k, r)
