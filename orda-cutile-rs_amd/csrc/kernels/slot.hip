@@ -152,9 +152,8 @@ __device__ __forceinline__ void slot_stats(const SlotArgs& a, int64_t r, int64_t
         v[4] += t;
         v[5] = fmaf(aTt, tt - ts, v[5]);
         v[6] += aTs - aTt;
-      } else {
-        v[7] += aTs;
       }
+      v[7] += aTs;   // by itself: out of v[6] + v[3] it would lose a sum small beside the teacher's
     }
   }
 #pragma unroll
@@ -172,7 +171,7 @@ __device__ __forceinline__ void slot_stats(const SlotArgs& a, int64_t r, int64_t
       for (int w = 1; w < kThreads / 64; ++w) v[k] += red[w][k];
     }
     SegStats* st = out + sg;
-    st->s = make_float4(ms, v[0], teacher ? v[6] + v[3] : v[7], v[1]);
+    st->s = make_float4(ms, v[0], v[7], v[1]);
     st->t = make_float4(mt, v[2], v[3], v[4]);
     st->c = make_float2(v[5], v[6]);
   }
@@ -323,7 +322,7 @@ __device__ __forceinline__ void slot_grad(const SlotArgs& a, int64_t r, int64_t 
     if (tg)
       a.ce_loss[a.n_rows + r] =
           ignored ? 0.f : static_cast<float>(row_nll(tt, static_cast<float>(trow[y]), alpha, v));
-    a.kl_row[r] = kl && !ignored ? kl_paired(xc, ss, tt, inv_t, false) * a.t_sq : 0.f;
+    a.kl_row[r] = kl && !ignored ? kl_paired(xc, ss, tt, inv_t, false, -0.5f) * a.t_sq : 0.f;
   }
 }
 

@@ -140,3 +140,25 @@ def test_slot_keeps_nan(v, lo, alpha):
                 assert bool(torch.isnan(got[k][r]).all()), (k, r)
             else:
                 assert torch.equal(got[k][r], clean[k][r]), (k, r)
+
+
+@pytest.mark.parametrize("v", [4096, 32768, 131072])
+def test_slot_peaked_student_flat_teacher(v):
+    """Student rows with one logit far above the rest beside nearly flat
+    teacher rows: the student's exponential sum is about 1 next to the
+    teacher's of up to V, so that it must not come from their difference."""
+    import torch
+    n = 4
+    g = torch.Generator(device="cuda")
+    g.manual_seed(v)
+    lg = torch.empty((2 * n, v), device="cuda").normal_(0, 1.0, generator=g)
+    lg[n:] *= 0.3
+    lg[:n, 7] = 20.0
+    y = torch.randint(0, v, (n,), device="cuda", generator=g).to(torch.int32)
+    T, kd = 1.5, 0.4
+    got = H.kl_ce_on_logits_chunk(lg, y, n, 1.0 / T, kd * T, T * T, 1.0, 1.0, 0.0, IGNORE, False, True)
+    ref = reference(lg, y, n, T, kd, 1.0, 1.0, 0.0, False, 1.0)
+    d = (got["grad_kl_student"].double() - ref["grad_kl_student"]).norm()
+    k, want = got["kl_per_row"].double(), ref["kl_per_row"]
+    assert float(d) <= 1e-5 * float(ref["grad_kl_student"].norm())
+    assert float((k - want).abs().max()) <= 1e-6 * float(want.abs().max()) + 1e-6
