@@ -1535,14 +1535,11 @@ void kl_ce_slot(orda_ctx* c, const orda_tensor* logits_chunk, const int32_t* tar
     tg = static_cast<const int32_t*>(d);
   }
   int64_t band = slot_band_rows(L.t, std::max<int64_t>(1, n_rows), v);
-  void* scratch;
-  if (sc) {
-    band = std::min(band, sc->bytes / slot_scratch_bytes(1, v));
-    if (band < 1) fail(ORDA_ERR_INVALID, "V=%lld exceeds the no-allocation scratch", static_cast<long long>(v));
-    scratch = sc->p;
-  } else {
-    scratch = ws(c, "slot.scratch", slot_scratch_bytes(band, v));
-  }
+  // The fixed scratch holds one row pair's segments at least: 4096 columns each
+  // up to V = 94e6, wider ones beyond.
+  const int64_t seg_cols = slot_seg_cols(v, sc ? sc->bytes : INT64_MAX);
+  if (sc) band = std::min(band, sc->bytes / slot_scratch_bytes(1, v, seg_cols));
+  void* scratch = sc ? sc->p : ws(c, "slot.scratch", slot_scratch_bytes(band, v, seg_cols));
   auto on_line = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 128 == 0; };
   SlotArgs a{};
   a.ltype = L.t;
@@ -1559,6 +1556,7 @@ void kl_ce_slot(orda_ctx* c, const orda_tensor* logits_chunk, const int32_t* tar
   a.teacher_ce = student_only == 0;
   a.n_rows = n_rows;
   a.out_lines = v % 32 == 0 && on_line(gk.p) && on_line(gc.p);
+  a.seg_cols = seg_cols;
   a.scratch = scratch;
   a.student = L.p;
   a.teacher = at(L.p, n_rows * L.ld, L.t);

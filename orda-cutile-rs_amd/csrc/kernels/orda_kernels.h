@@ -285,11 +285,14 @@ struct SlotArgs {
   float* grad_ce;            // student rows, then (teacher_ce) teacher rows
   float* ce_loss;            // likewise
   bool out_lines;            // every output row starts on a 128-byte line
-  void* scratch;             // slot_scratch_bytes(band, v), 16-byte aligned
+  int64_t seg_cols;          // slot_seg_cols
+  void* scratch;             // slot_scratch_bytes(band, v, seg_cols), 16-byte aligned
 };
-// Rows per band for logits of type t, and the scratch of a call in such bands.
+// Rows per band for logits of type t, the columns of a statistics segment that
+// `scratch` bytes hold a row's of, and the scratch of a call in such bands.
 int64_t slot_band_rows(DType t, int64_t n_rows, int64_t v);
-int64_t slot_scratch_bytes(int64_t band, int64_t v);
+int64_t slot_seg_cols(int64_t v, int64_t scratch);
+int64_t slot_scratch_bytes(int64_t band, int64_t v, int64_t seg_cols);
 hipError_t launch_slot(const SlotArgs& a, int64_t band, hipStream_t stream);
 
 // ---------------------------------------------------------------- reductions

@@ -6,7 +6,9 @@
 //   * statistics, one block per (row pair, 4096-column segment): both rows'
 //     segments are held in registers, so that the maxima, the exponential sums
 //     and the KL sums (kl_sums.h) take one read. 8192-column segments measured
-//     15 % slower on bf16 logits (fewer blocks in flight), 2048 10 %;
+//     15 % slower on bf16 logits (fewer blocks in flight), 2048 10 %. Where a
+//     fixed scratch does not hold a row's segments (1.75 MiB: V > 94e6) a block
+//     takes several times 4096 columns in turn (WIDE);
 //   * gradients, elementwise over (row pair, 2048-column block): each wave
 //     merges the row's segments while its logits are in flight, the block of
 //     column 0 also writes the row's losses.
@@ -61,28 +63,30 @@ struct SegStats {
   float2 c;
 };
 
+// An exponential sum relative to a larger maximum m than its own, k = log2(e) / T.
+// The maximum skips NaN: a range without another value has -inf beside sums of
+// NaN, which times 0 stay NaN, while those of a range that is -inf throughout
+// are 0.
+__device__ __forceinline__ float shrink(float sum, float own, float m, float k) {
+  return sum * (own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((own - m) * k));
+}
+// A statistic's two exponential sums relative to a larger maximum.
+__device__ __forceinline__ float2 rescale(float4 v, float m, float it2) {
+  return make_float2(shrink(v.y, v.x, m, kLog2e), shrink(v.z, v.x, m, it2));
+}
 // KL sums of a range relative to larger maxima (kl_rebase); a range in which
 // one row is -inf throughout keeps what its elements gave (inf or NaN).
 __device__ __forceinline__ float2 rebase(float2 c, float4 s, float4 t, float Ms, float Mt, float inv_t) {
   if (s.x != -INFINITY && t.x != -INFINITY) return kl_rebase(c, s.x, t.x, s.z, t.z, Ms, Mt, inv_t);
   const float it2 = inv_t * kLog2e;
-  return make_float2(c.x, s.z * __builtin_amdgcn_exp2f((s.x - Ms) * it2) -
-                              t.z * __builtin_amdgcn_exp2f((t.x - Mt) * it2));
-}
-// A statistic's two exponential sums relative to a larger maximum. The maximum
-// skips NaN: a range without another value has -inf beside sums of NaN, which
-// times 0 stay NaN, while those of a range that is -inf throughout are 0.
-__device__ __forceinline__ float2 rescale(float4 v, float m, float it2) {
-  if (v.x == -INFINITY) return make_float2(v.y * 0.f, v.z * 0.f);
-  return make_float2(v.y * __builtin_amdgcn_exp2f((v.x - m) * kLog2e),
-                     v.z * __builtin_amdgcn_exp2f((v.x - m) * it2));
+  return make_float2(c.x, shrink(s.z, s.x, Ms, it2) - shrink(t.z, t.x, Mt, it2));
 }
 
+// The statistics of the kSegCols columns of row pair r from c0 on, in thread 0.
 template <typename LT>
-__device__ __forceinline__ void slot_stats(const SlotArgs& a, int64_t r, int64_t sg, int64_t nseg, SegStats* out) {
+__device__ __forceinline__ SegStats col_stats(const SlotArgs& a, int64_t r, int64_t c0) {
   __shared__ float red[kThreads / 64][8];
   const int tid = threadIdx.x;
-  const int64_t c0 = sg * kSegCols;
   const bool teacher = a.kl || a.teacher_ce;
   const LT* srow = static_cast<const LT*>(a.student) + r * a.ld + c0;
   const LT* trow = static_cast<const LT*>(a.teacher) + r * a.ld + c0;
@@ -170,11 +174,33 @@ __device__ __forceinline__ void slot_stats(const SlotArgs& a, int64_t r, int64_t
 #pragma unroll
       for (int w = 1; w < kThreads / 64; ++w) v[k] += red[w][k];
     }
-    SegStats* st = out + sg;
-    st->s = make_float4(ms, v[0], v[7], v[1]);
-    st->t = make_float4(mt, v[2], v[3], v[4]);
-    st->c = make_float2(v[5], v[6]);
   }
+  return {make_float4(ms, v[0], v[7], v[1]), make_float4(mt, v[2], v[3], v[4]), make_float2(v[5], v[6])};
+}
+
+// Two ranges' statistics as one's.
+__device__ __forceinline__ SegStats join(const SegStats& a, const SegStats& b, float inv_t) {
+  const float it2 = inv_t * kLog2e, ms = fmaxf(a.s.x, b.s.x), mt = fmaxf(a.t.x, b.t.x);
+  const float2 sa = rescale(a.s, ms, it2), sb = rescale(b.s, ms, it2);
+  const float2 ta = rescale(a.t, mt, it2), tb = rescale(b.t, mt, it2);
+  const float2 ca = rebase(a.c, a.s, a.t, ms, mt, inv_t), cb = rebase(b.c, b.s, b.t, ms, mt, inv_t);
+  return {make_float4(ms, sa.x + sb.x, sa.y + sb.y, a.s.w + b.s.w),
+          make_float4(mt, ta.x + tb.x, ta.y + tb.y, a.t.w + b.t.w), make_float2(ca.x + cb.x, ca.y + cb.y)};
+}
+
+// Segment sg: kSegCols columns, or WIDE, a.seg_cols of them in turn.
+template <typename LT, bool WIDE>
+__device__ __forceinline__ void slot_stats(const SlotArgs& a, int64_t r, int64_t sg, SegStats* out) {
+  const int64_t c0 = sg * (WIDE ? a.seg_cols : kSegCols);
+  SegStats st = col_stats<LT>(a, r, c0);
+  if constexpr (WIDE) {
+    const int64_t end = c0 + a.seg_cols < a.v ? c0 + a.seg_cols : a.v;
+    for (int64_t c = c0 + kSegCols; c < end; c += kSegCols) {
+      __syncthreads();   // thread 0 has read the last columns' sums
+      st = join(st, col_stats<LT>(a, r, c), a.inv_t);
+    }
+  }
+  if (threadIdx.x == 0) out[sg] = st;
 }
 
 template <typename LT>
@@ -330,7 +356,7 @@ __device__ __forceinline__ void slot_grad(const SlotArgs& a, int64_t r, int64_t 
 // band k, row by row, so that reads and writes run together and a launch's
 // last blocks are of both kinds. Bands use the two halves of the scratch in
 // turn.
-template <typename LT>
+template <typename LT, bool WIDE>
 __global__ __launch_bounds__(kThreads) void slot_kernel(SlotArgs a, int64_t k, int64_t band, int64_t nseg,
                                                         int64_t chunks, int64_t per) {
   const int64_t row = blockIdx.x / per;
@@ -342,10 +368,10 @@ __global__ __launch_bounds__(kThreads) void slot_kernel(SlotArgs a, int64_t k, i
   if (row >= band || r >= a.n_rows) return;
   SegStats* half = static_cast<SegStats*>(a.scratch) + (((grads ? k - 1 : k) & 1) * band + row) * nseg;
   if (grads) slot_grad<LT>(a, r, i, nseg, half);
-  else slot_stats<LT>(a, r, i, nseg, half);
+  else slot_stats<LT, WIDE>(a, r, i, half);
 }
 
-int64_t segments(int64_t v) { return (v + kSegCols - 1) / kSegCols; }
+int64_t segments(int64_t v, int64_t cols) { return (v + cols - 1) / cols; }
 
 }  // namespace
 
@@ -354,24 +380,31 @@ int64_t slot_band_rows(DType t, int64_t n_rows, int64_t v) {
   return b < 1 ? 1 : b < n_rows ? b : n_rows;
 }
 
-int64_t slot_scratch_bytes(int64_t band, int64_t v) {
-  return 2 * band * segments(v) * static_cast<int64_t>(sizeof(SegStats));
+int64_t slot_seg_cols(int64_t v, int64_t scratch) {
+  const int64_t most = scratch / (2 * static_cast<int64_t>(sizeof(SegStats)));
+  return (segments(v, kSegCols) + most - 1) / most * kSegCols;
+}
+
+int64_t slot_scratch_bytes(int64_t band, int64_t v, int64_t seg_cols) {
+  return 2 * band * segments(v, seg_cols) * static_cast<int64_t>(sizeof(SegStats));
 }
 
 hipError_t launch_slot(const SlotArgs& a, int64_t band, hipStream_t s) {
   if (a.n_rows <= 0) return hipSuccess;
-  const int64_t nseg = segments(a.v);
+  const int64_t nseg = segments(a.v, a.seg_cols);
   const int64_t chunks = (a.v + kGradCols - 1) / kGradCols;
   const int64_t bands = (a.n_rows + band - 1) / band;
-  if (band < 1 || band * (nseg + chunks) > 0x7fffffff) return hipErrorInvalidValue;
+  if (band < 1 || band * (nseg + chunks) > 0x7fffffff || a.seg_cols < 1 || a.seg_cols % kSegCols)
+    return hipErrorInvalidValue;
+  using K = void (*)(SlotArgs, int64_t, int64_t, int64_t, int64_t, int64_t);
+  const bool wide = a.seg_cols > kSegCols, bf16 = a.ltype == DType::BF16;
+  const K kernel = bf16 ? (wide ? K(slot_kernel<__bf16, true>) : K(slot_kernel<__bf16, false>))
+                        : (wide ? K(slot_kernel<float, true>) : K(slot_kernel<float, false>));
   for (int64_t k = 0; k <= bands; ++k) {
     const int64_t per = (k > 0 ? chunks : 0) + (k < bands ? nseg : 0);
     const int64_t left = a.n_rows - (k > 0 ? k - 1 : 0) * band;
     const dim3 grid(static_cast<unsigned>((left < band ? left : band) * per));
-    if (a.ltype == DType::BF16)
-      hipLaunchKernelGGL(slot_kernel<__bf16>, grid, dim3(kThreads), 0, s, a, k, band, nseg, chunks, per);
-    else
-      hipLaunchKernelGGL(slot_kernel<float>, grid, dim3(kThreads), 0, s, a, k, band, nseg, chunks, per);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, a, k, band, nseg, chunks, per);
   }
   return hipGetLastError();
 }

@@ -143,3 +143,32 @@ def test_noalloc_slot_under_graph_capture():
     del graph
     ctx.close()
     ref_ctx.close()
+
+
+@pytest.mark.parametrize("v", [94_000_003, 200_000_000])
+def test_noalloc_slot_takes_any_vocabulary(v):
+    """A row's segments past what the fixed scratch holds at 4096 columns each
+    (94e6 columns): the call runs, on wider segments, as the allocating one
+    does. Gradients: the two statistics are the same sums in another order
+    (fp32, 2^-21 of a probability)."""
+    import torch
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    ctx, ref_ctx = H.Context(0), H.Context(0)
+    ctx.bind_stream()
+    ref_ctx.bind_stream()
+    lc = (torch.randn(2, v, generator=g, device=dev) * 2).to(torch.bfloat16)
+    y = torch.full((1,), v - 2, dtype=torch.int32, device=dev)
+    rc_a, msg_a, a = _call("orda_kl_ce_on_logits_chunk", ref_ctx, lc, y, 1, False)
+    assert rc_a == L.ORDA_OK, msg_a
+    rc_b, msg_b, b = _call("orda_kl_ce_on_logits_chunk_noalloc", ctx, lc, y, 1, False)
+    assert rc_b == L.ORDA_OK, msg_b
+    torch.cuda.synchronize()
+    assert ctx.workspace_bytes() == 0
+    for name, x, z in zip(("grad_kl_student", "kl_per_row", "grad_ce", "ce_loss"), a, b):
+        assert bool(torch.isfinite(z).all()), name
+        d, s = float((z - x).norm()), float(x.norm())
+        assert d <= 2e-6 * s, name
+    ctx.close()
+    ref_ctx.close()
