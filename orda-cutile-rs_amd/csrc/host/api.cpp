@@ -473,6 +473,7 @@ struct LossPlan {
   bool quant, stochastic;
   uint64_t seed;
   bool planes3;             // fp32 products over three-plane operands (use_planes3)
+  double retry_us;          // what an out-of-memory costs: loss_impl's next form of the call
   bool fast_math;           // approximate per-row logs and divisions
   bool online;              // one-pass row statistics (KernelConfig::online_softmax)
 };
@@ -546,6 +547,13 @@ bool teacher_logits_direct(const LossPlan& P, const Inputs& in) {
           in.tl.ld % 8 == 0 && in.tl.cols % 8 == 0 && reinterpret_cast<uintptr_t>(in.tl.p) % 16 == 0);
 }
 
+// Operations of a call's products.
+double loss_ops(const LossPlan& P) {
+  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
+  const double width = 3.0 * P.h + (t_rows ? (P.w_t > 0.f ? 3.0 : 1.0) * P.ht : 0.0);
+  return 2.0 * P.bt * P.v * width;
+}
+
 // Whether an fp32 call runs its products over three-plane operands
 // (GemmArgs::plane_a) instead of the fp32 MFMA: six bf16 products take the
 // place of one fp32 product, at 265 against 133 TFLOP/s of fp32 work, and the
@@ -562,10 +570,8 @@ bool teacher_logits_direct(const LossPlan& P, const Inputs& in) {
 // 4096) x 32000) 36.3 / 18.3 ms.
 bool use_planes3(const LossPlan& P) {
   if (P.dt != orda::DType::F32 || P.h < 64 || P.v < 64) return false;
-  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
-  if (t_rows && P.ht < 64) return false;
-  const double width = 3.0 * P.h + (t_rows ? (P.w_t > 0.f ? 3.0 : 1.0) * P.ht : 0.0);
-  return 2.0 * P.bt * P.v * width >= 17179869184.0;
+  if (P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED && P.ht < 64) return false;
+  return loss_ops(P) >= 17179869184.0;
 }
 
 // Whether the logits products take planes too. A Tied teacher's stay on the
@@ -619,19 +625,39 @@ int64_t staged_bytes_per_row(const LossPlan& P, const Inputs& in) {
 }
 
 // The split-K workspace a backward GEMM asks for, if any (one buffer shared
-// by the GEMMs of a call: they run in order on one stream) and if it fits.
-void attach_split_ws(orda_ctx* c, orda::GemmArgs& g) {
-  const int64_t b = orda::gemm_split_bytes(g);
-  if (b <= 0) return;
+// by the GEMMs of a call: they run in order on one stream). Where it does not
+// fit, the product takes the parts that do (unsplit: none), as long as that
+// costs less (gemm_us) than the call's other ways to make room (retry_us). At
+// 300 x 768 x 50257 bf16, 0.34 ms a call with grad_hidden in 21 parts: under a
+// limit 8 MB short of them 0.33 ms, 18 MB short 0.35 (unsplit 1.18 ms, in more
+// chunks 1.0).
+void attach_split_ws(orda_ctx* c, const LossPlan& P, orda::GemmArgs& g) {
+  g.split_ws = nullptr;
+  g.split_ws_bytes = g.split_cap = 0;
+  const orda::GemmArgs full = g;
   const orda_ctx::Buf& cur = c->bufs["splitk"];
-  // Growing the buffer frees the old one, which launches already queued on
-  // the stream may still use.
-  if (cur.p && cur.bytes < b) hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-  try {
-    g.split_ws = static_cast<float*>(ws(c, "splitk", b));
-    g.split_ws_bytes = b;
-  } catch (const Error& e) {
-    if (e.status != ORDA_ERR_OOM) throw;   // no room: the product runs unsplit
+  auto room = [&] { return c->mem_limit > 0 ? (c->mem_limit - c->held + cur.bytes) / 256 * 256 : INT64_MAX; };
+  for (;;) {
+    const int64_t b = orda::gemm_split_bytes(g);
+    if (b <= 0) return;
+    if (room() < b) (void)reclaim_planes3(c);
+    int64_t cap = room();
+    if (cap >= b) {
+      // Growing the buffer frees the old one, which launches already queued on
+      // the stream may still use.
+      if (cur.p && cur.bytes < b) hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+      try {
+        g.split_ws = static_cast<float*>(ws(c, "splitk", b));
+        g.split_ws_bytes = b;
+        return;
+      } catch (const Error& e) {
+        if (e.status != ORDA_ERR_OOM) throw;
+      }
+      cap = b / 2;
+    }
+    g.split_cap = std::max<int64_t>(std::min(cap, b - 1) / 256 * 256, 1);
+    if (orda::gemm_us(g) - orda::gemm_us(full) > P.retry_us)
+      fail(ORDA_ERR_OOM, "no room for %lld bytes of split-K partials", static_cast<long long>(b));
   }
 }
 
@@ -840,7 +866,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         timed(c, ORDA_KERNEL_GEMM_LOGITS, [&] { return launch_gemm(g, c->stream); });
         return false;
       }
-      attach_split_ws(c, sg);
+      attach_split_ws(c, P, sg);
       const GemmSplit sp = gemm_split_plan(sg);
       const bool contiguous =
           g.nprob == 1 || static_cast<float*>(g.prob[1].c) == static_cast<float*>(g.prob[0].c) + g.M * g.ldc;
@@ -1048,7 +1074,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
         planes(d, pv, ph, v);
         d.prob[0].b = d.prob[1].b = W3;
       }
-      attach_split_ws(c, d);
+      attach_split_ws(c, P, d);
       timed(c, ORDA_KERNEL_GEMM_GRAD_HIDDEN, [&] { return launch_gemm(d, c->stream); });
       if (P.has_ght && !fuse) {
         GemmArgs t = d;
@@ -1061,7 +1087,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
           planes(t, pv, pt, v);
           t.prob[0].b = TW3;
         }
-        attach_split_ws(c, t);
+        attach_split_ws(c, P, t);
         timed(c, ORDA_KERNEL_GEMM_GRAD_HIDDEN, [&] { return launch_gemm(t, c->stream); });
       }
     }
@@ -1100,7 +1126,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
       w.nprob = 1;
       w.prob[0] = {hcat, D, C};
       if (p3) planes(w, round64(k), pv, k);
-      attach_split_ws(c, w);
+      attach_split_ws(c, P, w);
       timed(c, ORDA_KERNEL_GEMM_GRAD_WEIGHT, [&] { return launch_gemm(w, c->stream); });
     };
     grad_weight(at(in.hs.p, gs * in.hs.ld, dt), in.hs.ld,
@@ -1305,8 +1331,18 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
     P.planes3 = false;
     G = group_of();
   }
+  // The next entry of the doubling schedule, or -1.
+  auto more_chunks = [&] {
+    for (int64_t s : chunk_doubling_schedule(bt, plan.num_chunks, limit))
+      if (s > plan.num_chunks) return s;
+    return int64_t{-1};
+  };
   for (;;) {
     try {
+      // Releasing the buffers and beginning again takes 0.6 ms, without planes
+      // the products twice as long; with nothing left to try the call fails.
+      P.retry_us = P.planes3 ? 600.0 + loss_ops(P) / 267e6
+                   : G > 1 || more_chunks() > 0 ? 600.0 : INFINITY;
       run_loss(c, P, in, plan, G, row3, scal, &lstat->mean_scale);
       break;
     } catch (const Error& e) {
@@ -1336,13 +1372,7 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
         G /= 2;
         continue;
       }
-      const std::vector<int64_t> sched = chunk_doubling_schedule(bt, plan.num_chunks, limit);
-      int64_t next = -1;
-      for (int64_t s : sched)
-        if (s > plan.num_chunks) {
-          next = s;
-          break;
-        }
+      const int64_t next = more_chunks();
       if (next < 0)
         fail(ORDA_ERR_OOM, "out of device memory at num_chunks=%lld (limit %lld): %s",
              static_cast<long long>(plan.num_chunks), static_cast<long long>(limit), e.msg.c_str());

@@ -2203,7 +2203,9 @@ __global__ __launch_bounds__(256) void transpose_split3_kernel(const float* a, i
 struct SplitPlan {
   int splits;
   int64_t len, ldp, stride, bytes;
+  double us;   // what the product takes by the measure it is chosen with
 };
+int64_t split_cap(const GemmArgs& g) { return g.split_cap > 0 ? g.split_cap : int64_t{256} << 20; }
 
 // Shared-round blocks (map_tile) for a product with share_rounds set: xn in
 // {1, 2, 4, 8} dividing the N-tiles, b = Nt/xn, a = 32/b; the most tiles per
@@ -2289,22 +2291,22 @@ int64_t tile_count(const GemmArgs& g) {
 // such counts: 300 x 768 x 50257 128 us against 91, 2000 x 1536 x 128256 929
 // against 594.)
 SplitPlan plan_split(const GemmArgs& g) {
-  SplitPlan sp{1, g.K, 0, 0, 0};
+  SplitPlan sp{1, g.K, 0, 0, 0, 0.0};
   if (g.epi == GemmEpilogue::Logits || g.M <= 0 || g.N <= 0 || g.K <= 0) return sp;
   const int64_t tiles = tile_count(g);
   const int64_t per_split = g.nprob * (g.c_trans ? g.N * ((g.M + 3) / 4 * 4) : g.M * ((g.N + 3) / 4 * 4)) * 4;
   int64_t most = tiles < 192 ? (256 + tiles - 1) / tiles : 8;
-  const int64_t by_k = g.K / 128, by_ws = (int64_t{256} << 20) / per_split;
+  const int64_t by_k = g.K / 128, by_ws = split_cap(g) / per_split;
   if (most > by_k) most = by_k;
   if (most > 128) most = 128;
   if (most > by_ws) most = by_ws;
-  double best = rounds_us(g, tiles, g.K);
+  sp.us = rounds_us(g, tiles, g.K);
   for (int64_t i = 2; i <= most; ++i) {
     const int64_t len = ((g.K + i - 1) / i + 63) / 64 * 64, n = (g.K + len - 1) / len;
     if (n <= 1) break;
     const double us = rounds_us(g, tiles * n, len) + 2 * kPartUs * static_cast<double>(n * per_split);
-    if (us < best) {
-      best = us;
+    if (us < sp.us) {
+      sp.us = us;
       sp.splits = static_cast<int>(n);
       sp.len = len;
     }
@@ -2315,9 +2317,6 @@ SplitPlan plan_split(const GemmArgs& g) {
   sp.stride = g.nprob * (g.c_trans ? g.N : g.M) * sp.ldp;
   sp.bytes = sp.splits * sp.stride * 4;
   return sp;
-}
-double split_us(const GemmArgs& g, const SplitPlan& sp) {
-  return rounds_us(g, tile_count(g) * sp.splits, sp.len) + 2 * kPartUs * static_cast<double>(sp.bytes);
 }
 
 // ------------------------------------------------------- small fp32 products
@@ -2365,13 +2364,13 @@ bool small_f32(const GemmArgs& g) {
 // 512 x 8192 the same; two workgroups a CU, 512 in all, were slower there, 253
 // against 223; all before the kernel's present loads.)
 SplitPlan plan_split_small(const GemmArgs& g) {
-  SplitPlan sp{1, g.K, 0, 0, 0};
+  SplitPlan sp{1, g.K, 0, 0, 0, 0.0};
   if (g.K <= 0) return sp;
   const int64_t tiles = small_tiles(g);
   if (tiles >= 192) return sp;
   const int64_t per_split = g.nprob * (g.c_trans ? g.N * ((g.M + 3) / 4 * 4) : g.M * ((g.N + 3) / 4 * 4)) * 4;
   int64_t most = (256 + tiles - 1) / tiles;
-  const int64_t by_k = g.K / 128, by_ws = (int64_t{256} << 20) / per_split;
+  const int64_t by_k = g.K / 128, by_ws = split_cap(g) / per_split;
   if (most > by_k) most = by_k;
   if (most > 64) most = 64;
   if (most > by_ws) most = by_ws;
@@ -2379,12 +2378,12 @@ SplitPlan plan_split_small(const GemmArgs& g) {
     return static_cast<double>((tiles * n + 255) / 256) * (static_cast<double>(len) / 32 * 2.4 + 6.0) +
            (n > 1 ? 2 * kPartUs * static_cast<double>(n * per_split) : 0.0);
   };
-  double best = cost(1, g.K);
+  sp.us = cost(1, g.K);
   for (int64_t i = 2; i <= most; ++i) {
     const int64_t len = ((g.K + i - 1) / i + 63) / 64 * 64, n = (g.K + len - 1) / len;
     if (n <= 1) break;
-    if (cost(n, len) >= best) continue;
-    best = cost(n, len);
+    if (cost(n, len) >= sp.us) continue;
+    sp.us = cost(n, len);
     sp.splits = static_cast<int>(n);
     sp.len = len;
   }
@@ -2783,12 +2782,11 @@ TailSplit plan_tail(const GemmArgs& g) {
   const int64_t Mv = Mt * g.nprob;
   const int64_t T = Mv * Nt, q = T / 256, r = T % 256;
   if (q < 1 || r == 0 || r >= 192) return none;
-  const SplitPlan whole = plan_split(g);
-  const double one = whole.splits > 1 ? split_us(g, whole) : rounds_us(g, T, g.K);
+  const double one = plan_split(g).us;
   const double rounds = q * (rounds_us(g, 1, g.K));
   auto pays = [&](const GemmArgs& tail) {
     const SplitPlan sp = plan_split(tail);
-    return sp.splits > 1 && rounds + split_us(tail, sp) < one;
+    return sp.splits > 1 && rounds + sp.us < one;
   };
   const int64_t n0 = 256 * q / Mv * kTile;
   if (n0 > 0 && n0 < g.N && pays(sub_product(g, 0, g.M, n0, g.N))) return {n0, true};
@@ -2825,6 +2823,13 @@ int64_t gemm_split_bytes(const GemmArgs& g) {
   const TailSplit ts = plan_tail(g);
   const SplitPlan sp = plan_split(ts.at > 0 ? tail_part(g, ts, true) : g);
   return sp.splits > 1 ? sp.bytes : 0;
+}
+
+double gemm_us(const GemmArgs& g) {
+  if (small_f32(g)) return plan_split_small(g).us;
+  const TailSplit ts = plan_tail(g);
+  if (ts.at <= 0) return plan_split(g).us;
+  return plan_split(tail_part(g, ts, false)).us + plan_split(tail_part(g, ts, true)).us;
 }
 
 bool gemm_small_tiles(const GemmArgs& g) { return small_f32(g); }

@@ -118,6 +118,7 @@ struct GemmArgs {
   // workgroups per tile and sums their fp32 partials in a fixed order.
   float* split_ws;
   int64_t split_ws_bytes;
+  int64_t split_cap;   // most bytes of partials to plan for; 0: 256 MB
   // Set by launch_gemm for the split launch: K range s*split_len.. of the
   // workgroups of split s, partials of split s at split_ws + s*split_stride.
   int split_k;
@@ -154,8 +155,11 @@ hipError_t launch_transpose_rows(const void* a, int64_t lda, const void* b, int6
 hipError_t launch_transpose_split3(const float* a, int64_t lda, const float* b, int64_t ldb,
                                    int64_t rows, int64_t cols, void* dst, int64_t plane,
                                    hipStream_t stream);
-// Workspace bytes launch_gemm uses to split K for this GEMM (0: no split).
+// Workspace bytes launch_gemm uses to split K for this GEMM (0: no split), at
+// most split_cap, and what the product then takes, in us, by the measure the
+// split is chosen with.
 int64_t gemm_split_bytes(const GemmArgs& g);
+double gemm_us(const GemmArgs& g);
 // Whether launch_gemm runs this Store/Accum GEMM on 128 x 128 tiles (fp32
 // inputs, at most 64 tiles of 256 x 256): splits and partials as given by
 // gemm_split_plan / gemm_split_bytes.

@@ -6,8 +6,9 @@ GPU (tests/torch_reference.py; tolerances as in tests/parity.py):
 * one tile split in more than 64 parts;
 * grad_W (3 M-tiles x 100 N-tiles) as 85 column tiles in one round and 15 more
   split over K; grad_hidden (13 x 20 tiles) as 19 column tiles and one more;
-* the same products under a memory limit that leaves no room for partials:
-  they run unsplit, at the same chunk plan.
+* the same products under a memory limit that leaves no room for all their
+  partials: they take fewer parts, at the same chunk plan, and grad_hidden of
+  few tiles is not left on a few CUs.
 """
 import pytest
 
@@ -61,3 +62,37 @@ def test_uneven_splits(name, dtype):
             check_scalar(k, getattr(out, k), ref[k])
         for k in ("grad_student_hidden", "grad_weight", "grad_teacher_hidden"):
             check_grad_device(k, getattr(out, k), ref[k], dtype)
+
+
+@pytest.mark.parametrize("short", [1 << 20, 12 << 20, 18 << 20])
+def test_partials_that_do_not_fit_cost_no_idle_chip(short):
+    """grad_hidden at 300 x 768 x 50257 is 6 to 12 tiles over a K of 50257: with
+    K split over the CUs some 0.1 ms, unsplit ten times that. Under a limit
+    that leaves too little room for its partials (18 MB) the product runs in
+    the parts that fit, or the call makes room as it does for any other buffer;
+    bound: three times the unbounded call's time of that product."""
+    import torch
+    s, w, y, _ = inputs(torch, 300, 768, 50257, torch.bfloat16)
+    opts = LossOptions()
+
+    def run(ctx):
+        got = None
+        for i in range(4):
+            if i == 1:
+                ctx.set_timing(True)
+                ctx.reset_timing()
+            got = H.distillation_loss(s, w, y, Teacher.Tied(s), opts, ctx=ctx)
+        return got, ctx.kernel_time("gemm_grad_hidden")[0] / 3
+
+    free = H.Context(0)
+    want, t_free = run(free)
+    limit = free.workspace_bytes() - short
+    free.close()
+    ctx = H.Context(0)
+    ctx.set_memory_limit(limit)
+    got, t = run(ctx)
+    assert ctx.workspace_bytes() <= limit
+    ctx.close()
+    check_grad_device("grad_student_hidden", got.grad_student_hidden, want.grad_student_hidden, "bf16")
+    check_grad_device("grad_weight", got.grad_weight, want.grad_weight, "bf16")
+    assert t <= 3 * t_free
