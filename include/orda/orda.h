@@ -197,7 +197,8 @@ int32_t orda_ctx_set_memory_limit(orda_ctx *ctx, int64_t bytes);
  * accumulating into grad_W. The split-K partials of backward GEMMs with
  * fewer output tiles than CUs (at most 256 MB) come on top of it, and so do
  * the weights of a large fp32 call as three bf16 planes (6 bytes an element;
- * such a call runs without them where they do not fit the memory limit). No
+ * such a call runs without them where its buffers with them do not fit the
+ * memory limit, or at that moment the device). No
  * counterpart in the reference, which runs one chunk at a time
  * (src/api.rs:263-378). */
 int32_t orda_ctx_set_staging_budget(orda_ctx *ctx, int64_t bytes);

@@ -52,9 +52,12 @@ struct orda_ctx {
   };
   std::map<std::string, Buf> bufs;
   bool planes_live = false;   // the three-plane buffers are in use by this call
-  // Fewest plane bytes a call ran out of memory with (0: none since the limit
-  // was set or the workspace trimmed): calls of as many do not try again.
-  int64_t planes_refused = 0;
+  // While set, ws() adds up what it is asked for instead of allocating it: the
+  // bytes in all, and those past what the buffers hold.
+  struct Sizing {
+    int64_t need = 0, grow = 0;
+  };
+  Sizing* sizing = nullptr;
   // Pinned host staging for small device-to-host reads (the labels, which
   // the host validates and counts): a copy into pageable memory costs
   // several times as long.
@@ -172,8 +175,25 @@ void ws_release(orda_ctx* c, const std::string& name);
 
 // The buffers of the three-plane form (use_planes3): a call that runs short of
 // memory does without them, so they are given up before any other.
+constexpr const char* kPlanes3Bufs[] = {"p3.w", "p3.tw", "p3.hs", "p3.th", "p3.grad"};
+// The other buffers a group of chunks runs in.
+constexpr const char* kGroupBufs[] = {"logits", "hcat",   "hmax",    "stats",   "xy",    "dlogits",
+                                      "cross",  "rconst", "klpart", "tlogits", "tgrad", "splitk"};
 void release_planes3(orda_ctx* c) {
-  for (const char* n : {"p3.w", "p3.tw", "p3.hs", "p3.th", "p3.grad"}) ws_release(c, n);
+  for (const char* n : kPlanes3Bufs) ws_release(c, n);
+}
+void release_group(orda_ctx* c) {
+  for (const char* n : kGroupBufs) ws_release(c, n);
+}
+int64_t loss_held(const orda_ctx* c) {   // of all of these
+  int64_t b = 0;
+  auto add = [&](const char* n) {
+    const auto it = c->bufs.find(n);
+    if (it != c->bufs.end()) b += it->second.bytes;
+  };
+  for (const char* n : kPlanes3Bufs) add(n);
+  for (const char* n : kGroupBufs) add(n);
+  return b;
 }
 bool reclaim_planes3(orda_ctx* c) {
   const int64_t before = c->held;
@@ -185,13 +205,18 @@ bool reclaim_planes3(orda_ctx* c) {
 void* ws(orda_ctx* c, const std::string& name, int64_t bytes) {
   orda_ctx::Buf& b = c->bufs[name];
   if (bytes <= 0) return b.p;
+  const int64_t rounded = (bytes + 255) / 256 * 256;
+  if (c->sizing) {
+    c->sizing->need += rounded;
+    c->sizing->grow += std::max<int64_t>(0, rounded - b.bytes);
+    return b.p;
+  }
   if (b.p && b.bytes >= bytes) return b.p;
   if (b.p) {
     hip_check(hipFree(b.p), "hipFree");
     c->held -= b.bytes;
     b = orda_ctx::Buf{};
   }
-  const int64_t rounded = (bytes + 255) / 256 * 256;
   if (c->mem_limit > 0 && c->held + rounded > c->mem_limit && !(reclaim_planes3(c) && c->held + rounded <= c->mem_limit))
     fail(ORDA_ERR_OOM, "workspace '%s' (%lld bytes) exceeds the context memory limit",
          name.c_str(), static_cast<long long>(rounded));
@@ -583,15 +608,6 @@ bool use_planes3(const LossPlan& P) {
 bool fp32_logits(const LossPlan& P) { return P.need_teacher && P.mode == ORDA_TEACHER_TIED; }
 bool planes3_logits(const LossPlan& P) { return P.planes3 && !fp32_logits(P); }
 
-// Device bytes of the three-plane buffers of a call whose groups hold `cap`
-// rows: the weights, and the rows' share (as run_loss sizes them).
-int64_t planes3_bytes(const LossPlan& P, int64_t cap) {
-  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
-  const int64_t ph = round64(P.h), pt = t_rows ? round64(P.ht) : 0, pv = round64(P.v);
-  return 6 * (pv * (ph + (P.mode == ORDA_TEACHER_SEPARATE ? pt : 0)) +
-              cap * ((planes3_logits(P) ? ph + pt : 0) + (P.need_teacher ? 2 : 1) * pv));
-}
-
 // Device bytes the loss stages per chunk row: the buffers run_loss sizes by
 // the group's rows. (The split-K partials of small backward GEMMs are sized
 // by the GEMM, at most 256 MB, and come on top.)
@@ -743,6 +759,7 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
   // staged with, so the logits are exactly 0; the backward products keep the
   // true width (no output columns, nothing launched).
   const int64_t kh = std::max<int64_t>(h, 1);
+  if (c->sizing) return;   // planes3_fit
 
   if (v == 0) {
     // An empty vocabulary: every label is ignore_index (validated), so every
@@ -1153,6 +1170,36 @@ void run_loss(orda_ctx* c, const LossPlan& P, const Inputs& in, orda::ChunkPlan 
   timed(c, ORDA_KERNEL_OTHER, [&] { return launch_finalize(fa, c->stream); });
 }
 
+// Whether the buffers of a three-plane call (of run, a run_loss) fit the memory
+// limit and the device, beside what else the context holds: asked before each
+// such call, so that it goes by the memory there is and not by how an earlier
+// call fared. What earlier calls left in its buffers past its own needs is
+// given up where that is in the way.
+template <class F>
+bool planes3_fit(orda_ctx* c, F&& run) {
+  orda_ctx::Sizing z;
+  c->sizing = &z;
+  try {
+    run();
+  } catch (...) {
+    c->sizing = nullptr;
+    throw;
+  }
+  c->sizing = nullptr;
+  if (z.grow == 0) return true;
+  const int64_t mine = loss_held(c);
+  if (c->mem_limit > 0 && c->held - mine + z.need > c->mem_limit) return false;
+  size_t free = 0, total = 0;
+  hip_check(hipMemGetInfo(&free, &total), "hipMemGetInfo");
+  const int64_t dev = static_cast<int64_t>(free) - (int64_t{64} << 20);   // the allocator's grain
+  if (z.need > dev + mine) return false;
+  if ((c->mem_limit > 0 && c->held + z.grow > c->mem_limit) || z.grow > dev) {
+    release_group(c);
+    release_planes3(c);
+  }
+  return true;
+}
+
 void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const int64_t* labels,
                int64_t n_labels, int32_t lab_loc, const orda_teacher* teacher,
                const orda_loss_options* o, orda_loss_output* out) {
@@ -1326,8 +1373,7 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
     return std::max<int64_t>(1, std::min<int64_t>(plan.num_chunks, c->staging_budget / std::max<int64_t>(chunk_bytes, 1)));
   };
   int64_t G = group_of();
-  const int64_t planes_need = P.planes3 ? planes3_bytes(P, std::min(bt, G * plan.chunk_size)) : 0;
-  if (P.planes3 && c->planes_refused > 0 && planes_need >= c->planes_refused) {
+  if (P.planes3 && !planes3_fit(c, [&] { run_loss(c, P, in, plan, G, row3, scal, &lstat->mean_scale); })) {
     P.planes3 = false;
     G = group_of();
   }
@@ -1349,21 +1395,9 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
       if (e.status != ORDA_ERR_OOM) throw;
       (void)hipStreamSynchronize(c->stream);
       (void)hipGetLastError();
-      ws_release(c, "logits");
-      ws_release(c, "hcat");
-      ws_release(c, "hmax");
-      ws_release(c, "stats");
-      ws_release(c, "xy");
-      ws_release(c, "dlogits");
-      ws_release(c, "cross");
-      ws_release(c, "rconst");
-      ws_release(c, "klpart");
-      ws_release(c, "tlogits");
-      ws_release(c, "tgrad");
-      ws_release(c, "splitk");
+      release_group(c);
       if (P.planes3) {   // plain fp32 operands need less: first without the planes
         release_planes3(c);
-        c->planes_refused = c->planes_refused > 0 ? std::min(c->planes_refused, planes_need) : planes_need;
         P.planes3 = false;
         G = group_of();
         continue;
@@ -1708,7 +1742,6 @@ int32_t orda_ctx_set_stream(orda_ctx* c, void* s) {
 int32_t orda_ctx_set_memory_limit(orda_ctx* c, int64_t bytes) {
   if (!c || bytes < 0) return ORDA_ERR_INVALID;
   c->mem_limit = bytes;
-  c->planes_refused = 0;
   return ORDA_OK;
 }
 
@@ -1729,7 +1762,6 @@ int32_t orda_ctx_trim(orda_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   ws_trim(c);
-  c->planes_refused = 0;
   return ORDA_OK;
 }
 

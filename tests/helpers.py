@@ -59,3 +59,13 @@ def bf16_round(a: np.ndarray) -> np.ndarray:
     out = r.astype(np.uint32).view(np.float32).copy()
     out[nan] = np.nan
     return out
+
+
+def kernels_of(fn):
+    """(fn's result, the names of the GPU kernels it launched)."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as p:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, {e.name for e in p.events()}

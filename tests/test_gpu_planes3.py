@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import torch_reference as R
-from helpers import normal, uniform_labels
+from helpers import kernels_of, normal, uniform_labels
 
 import orda_hip as H
 from orda_hip import ChunkSize, LossOptions, Teacher
@@ -148,3 +148,34 @@ def test_infinite_weight_masks_its_column(bt, h, v):
     assert abs(got.student_ce - loss) <= 1e-4 * abs(loss)
     assert rel(got.grad_weight, gw) <= 1e-3
     assert torch.isnan(got.grad_student_hidden).all()
+
+
+def test_planes3_do_not_depend_on_earlier_calls():
+    """Under one memory limit, a call whose planes fit gives the same bits in a
+    fresh context and after a call of fewer plane bytes but more memory in
+    all, whose planes did not fit."""
+    import torch
+    v, h = 9000, 360
+    w, y = normal((v, h), 2, 1.0 / np.sqrt(h)), uniform_labels(1000, v, 3)
+    s, tl = normal((1000, h), 1), normal((1000, v), 6, 1.5)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    opts = LossOptions(kd_weight=0.4, temperature=1.5, teacher_ce_weight=0.0)
+    tied = LossOptions(kd_weight=0.4, temperature=1.5, teacher_ce_weight=1.0)
+    sd, wd, yd, td = dev(s), dev(w), dev(y), dev(tl)
+    large = lambda ctx: H.distillation_loss(sd[:700], wd, yd[:700], Teacher.Tied(dev(s[::-1][:700])), tied, ctx=ctx)
+    small = lambda ctx: H.distillation_loss(sd, wd, yd, Teacher.Precomputed(td), opts, ctx=ctx)
+    limit = 145_000_000
+    fresh, used = H.Context(0), H.Context(0)
+    for c in (fresh, used):
+        c.set_memory_limit(limit)
+    planes = lambda f, c: any("bf16x3" in k for k in kernels_of(lambda: f(c))[1])
+    assert planes(small, fresh) and not planes(large, used)
+    assert planes(small, used)
+    want = small(fresh)
+    for _ in range(2):
+        got = small(used)
+        assert used.workspace_bytes() <= limit
+        assert torch.equal(got.grad_weight, want.grad_weight)
+        assert torch.equal(got.grad_student_hidden, want.grad_student_hidden)
+    fresh.close()
+    used.close()
