@@ -12,14 +12,15 @@ namespace orda {
 // Each remainder is exact in fp32 and 24 bits of significand are three times
 // eight, so h + m + l == x for every finite x whose last bit is at or above
 // the smallest bf16 denormal, 2^-133 (below it l rounds). h truncates where
-// rounding would overflow. An infinity or a NaN is l alone: of the six plane
-// products only one takes l, with the other value's h, so that the product is
-// the infinity of the right sign (as h it would also meet the other's m and l,
-// of either sign, or zero: a NaN).
+// rounding would overflow. An infinity or a NaN is l, beside an h of its sign
+// and size 1: of the six plane products only l times the other value's h meets
+// it, so that infinity times a value is the infinity of the right sign, and
+// times another infinity too (1 * inf twice and 1 * 1). As h, it would also meet
+// the other value's m and l, of either sign, or zero: a NaN.
 __device__ __forceinline__ void split3(float x, float& h, float& m, float& l) {
   const bool finite = fabsf(x) <= FLT_MAX;
   h = static_cast<float>(static_cast<__bf16>(x));
-  if (!(fabsf(h) <= FLT_MAX)) h = finite ? __uint_as_float(__float_as_uint(x) & 0xffff0000u) : 0.f;
+  if (!(fabsf(h) <= FLT_MAX)) h = finite ? __uint_as_float(__float_as_uint(x) & 0xffff0000u) : copysignf(1.f, x);
   const float r = finite ? x - h : 0.f;
   m = static_cast<float>(static_cast<__bf16>(r));
   l = finite ? r - m : x;   // stored rounded to bf16
