@@ -608,6 +608,18 @@ bool use_planes3(const LossPlan& P) {
 bool fp32_logits(const LossPlan& P) { return P.need_teacher && P.mode == ORDA_TEACHER_TIED; }
 bool planes3_logits(const LossPlan& P) { return P.planes3 && !fp32_logits(P); }
 
+// Whether the three-plane kernels reach every row of an operand's tile: its
+// rows lie 32 bits of bytes apart, 6 bytes an element (the fp32 MFMA's 4), in
+// groups of `rows`. 256 rows of one K each reach V = 2.8e6.
+bool planes3_reach(const LossPlan& P, int64_t rows) {
+  const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
+  const int64_t ht = t_rows ? P.ht : 0, k = P.mode == ORDA_TEACHER_TIED && P.w_t > 0.f ? 2 * rows : rows;
+  auto fits = [](int64_t ext, int64_t pitch) {   // ext rows of pitch elements, in tiles of 64 or 256
+    return (std::min<int64_t>(std::max<int64_t>(ext, 64), 256) - 1) * 6 * round64(pitch) + 512 <= UINT32_MAX;
+  };
+  return fits(rows, P.v) && fits(std::max(rows, P.v), std::max(P.h, ht)) && fits(std::max(P.h, ht), k);
+}
+
 // Device bytes the loss stages per chunk row: the buffers run_loss sizes by
 // the group's rows. (The split-K partials of small backward GEMMs are sized
 // by the GEMM, at most 256 MB, and come on top.)
@@ -1373,6 +1385,10 @@ void loss_impl(orda_ctx* c, const orda_tensor* sh, const orda_tensor* w, const i
     return std::max<int64_t>(1, std::min<int64_t>(plan.num_chunks, c->staging_budget / std::max<int64_t>(chunk_bytes, 1)));
   };
   int64_t G = group_of();
+  if (P.planes3 && !planes3_reach(P, std::min(bt, G * plan.chunk_size))) {
+    P.planes3 = false;
+    G = group_of();
+  }
   if (P.planes3 && !planes3_fit(c, [&] { run_loss(c, P, in, plan, G, row3, scal, &lstat->mean_scale); })) {
     P.planes3 = false;
     G = group_of();

@@ -179,3 +179,28 @@ def test_planes3_do_not_depend_on_earlier_calls():
         assert torch.equal(got.grad_student_hidden, want.grad_student_hidden)
     fresh.close()
     used.close()
+
+
+# Row pitches of six bytes an element up to the 32 bits a tile's offsets have
+# (256 rows: V or rows of 2.8e6), and past them, where the call keeps to the
+# fp32 MFMA. fp32 sums of K terms in order are off by 2^-24 sqrt(K / 2) in the
+# mean, 7e-5 for the 2.9e6 of the last case, and other rows by all of it.
+@pytest.mark.parametrize("bt,h,v,planes", [(300, 64, 2_700_000, True), (300, 64, 2_900_000, False),
+                                           (2_900_000, 256, 64, False)])
+def test_planes3_up_to_what_a_tile_reaches(bt, h, v, planes):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(v)
+    rand = lambda *n: torch.randn(n, device="cuda", generator=g)
+    s, w, y = rand(bt, h), rand(v, h) / h ** 0.5, torch.randint(0, v, (bt,), device="cuda", generator=g)
+    opts = LossOptions(kd_weight=0.0, teacher_ce_weight=0.0, label_smoothing=0.0)
+    ctx = H.Context(0)
+    got, names = kernels_of(lambda: H.distillation_loss(s, w, y, Teacher.Tied(s), opts, ctx=ctx))
+    ctx.close()
+    assert any("bf16x3" in n for n in names) == planes
+    p = torch.softmax(s.double() @ w.double().T, dim=1)
+    p[torch.arange(bt, device="cuda"), y] -= 1.0
+    p /= bt
+    for k, ref in (("grad_student_hidden", lambda: p @ w.double()), ("grad_weight", lambda: p.T @ s.double())):
+        r = ref()
+        assert float((getattr(got, k).double() - r).norm() / r.norm()) <= 3e-4, k
