@@ -73,10 +73,11 @@ class DistillCEFunction(torch.autograd.Function):
                             for t in (student_hidden, weight, teacher_hidden, teacher_weight))
         fctx.chunk_plan = out.chunk_plan
         dev = student_hidden.device
-        # neither waits for the device: a fill, and a copy from pinned memory
+        # neither waits for the device: a fill, and a copy from pinned memory (of
+        # the host, whatever torch's default device is)
         loss = torch.full((), out.loss, dtype=torch.float32, device=dev)
         comps = torch.tensor([out.student_ce, out.teacher_ce, out.kl], dtype=torch.float32,
-                             pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
+                             device="cpu", pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
         fctx.mark_non_differentiable(comps)
         return loss, comps
 

@@ -59,3 +59,18 @@ def test_batched_incoming_gradients():
     k = torch.tensor([1.0, 3.0], device="cuda")
     g, = torch.autograd.grad(loss, [t["s"]], grad_outputs=k, is_grads_batched=True)
     assert torch.equal(g, (ref * k[:, None, None]).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("default", ["meta", "cuda", "cpu"])
+def test_default_device_does_not_matter(default):
+    """The op's outputs are on its inputs' device under any default device."""
+    import torch
+    t, y = make(16, 24, 100, torch.float32, False)
+    want = H.distillation_loss(t["s"], t["w"], y, teacher(t), OPTS)
+    t["w"].requires_grad_(True)
+    with torch.device(default):
+        loss, terms = distillation_loss_autograd(t["s"], t["w"], y, teacher(t), OPTS)
+        g, = torch.autograd.grad(loss, [t["w"]])
+    assert loss.item() == want.loss
+    assert terms.tolist() == [want.student_ce, want.teacher_ce, want.kl]
+    assert torch.equal(g, want.grad_weight)
