@@ -1,9 +1,11 @@
 """Build-time check of the GEMM's gfx950 assembly.
 
-The bf16 GEMM kernels issue their MFMAs as inline asm (accumulators tied to
-AGPRs), so the compiler's hazard recognizer does not see them and the kernel
-inserts the required wait states itself. This script verifies, on every
-control-flow path of every bf16 GEMM variant, that
+The bf16 GEMM kernels on 256 x 256 tiles, plain and three-plane, issue their
+MFMAs as inline asm (accumulators tied to AGPRs), so the compiler's hazard
+recognizer does not see them and the kernel inserts the required wait states
+itself. (The 128 x 256 and the small fp32 tiles use the builtins, which the
+compiler spaces.) This script verifies, on every control-flow path of each of
+these variants, that
   * no non-MFMA instruction reads or writes an MFMA result register within
     MFMA_RESULT_WAIT wait states of the MFMA that wrote it, and no MFMA reads
     it as an operand that soon either;
@@ -158,8 +160,8 @@ def check(path):
                     entry[j] = merged
                     if j not in work:
                         work.append(j)
-    if checked < 13:
-        errors.add(f"expected the 13 bf16 GEMM variants, found {checked}")
+    if checked < 12:
+        errors.add(f"expected the 12 bf16 GEMM variants with inline MFMAs, found {checked}")
     return sorted(errors)
 
 

@@ -521,8 +521,9 @@ __device__ __forceinline__ void mfma_step(f32x4 (&acc)[kFrag][kFrag], const u32x
 // fp32 products on the bf16 matrix units (GemmArgs::plane_a): each operand is
 // stored as three bf16 planes h + m + l (split3.h), which hold every bit of
 // an fp32 value, and a product of two such operands is the sum of six plane
-// products; the three left out (ml, lm, ll) lie below 2^-26 of |a·b| each,
-// under half an ulp of one fp32 product. A K block is 64 elements, 12 stages of
+// products. Of the three left out ml and lm lie below 2^-25 of |a·b| each (|m| <=
+// 2^-8 |a|, |l| <= 2^-17 |a| but for the rounding of h), 2^-24 together, half an
+// ulp of the product at most, and ll below 2^-34. A K block is 64 elements, 12 stages of
 // MFMAs: the products in the order hl, hm, mm, mh, hh, lh (A's plane first), each
 // of which changes one operand, and the two 32-element halves of a product in
 // an order that ends on the half the next one starts with. So each plane is
@@ -1982,13 +1983,11 @@ ORDA_GEMM(gemm_kk_logits_pre_bf16_bf16, __bf16, true, true, GemmEpilogue::Logits
 ORDA_GEMM(gemm_kk_logits_pre16_bf16_bf16, __bf16, true, true, GemmEpilogue::LogitsTeacher16, __bf16, false)
 ORDA_GEMM(gemm_kk_logits_bf16_f32, __bf16, true, true, GemmEpilogue::Logits, float, false)
 ORDA_GEMM(gemm_km_store_bf16, __bf16, true, false, GemmEpilogue::StoreF32, float, false)
-ORDA_GEMM(gemm_km_accum_bf16, __bf16, true, false, GemmEpilogue::AccumF32, float, false)
 ORDA_GEMM(gemm_kmt_store_bf16, __bf16, true, false, GemmEpilogue::StoreF32, float, true)
 ORDA_GEMM(gemm_kmt_accum_bf16, __bf16, true, false, GemmEpilogue::AccumF32, float, true)
 ORDA_GEMM(gemm_kk_logits_f32_bf16, float, true, true, GemmEpilogue::Logits, __bf16, false)
 ORDA_GEMM(gemm_kk_logits_f32_f32, float, true, true, GemmEpilogue::Logits, float, false)
 ORDA_GEMM(gemm_km_store_f32, float, true, false, GemmEpilogue::StoreF32, float, false)
-ORDA_GEMM(gemm_km_accum_f32, float, true, false, GemmEpilogue::AccumF32, float, false)
 ORDA_GEMM(gemm_kmt_store_f32, float, true, false, GemmEpilogue::StoreF32, float, true)
 ORDA_GEMM(gemm_kmt_accum_f32, float, true, false, GemmEpilogue::AccumF32, float, true)
 // fp32 logits of small problems, stored plainly and split over K (the row
@@ -2009,11 +2008,11 @@ ORDA_GEMM3(gemm_kmt_accum_bf16x3, false, GemmEpilogue::AccumF32, true)
 #define ORDA_MID(NAME, BK, EPI, LT, CT) \
   __global__ __launch_bounds__(kThreads, 2) void NAME(GemmArgs g) { mid_body<BK, EPI, LT, CT>(g); }
 ORDA_MID(gemm_kk_mid_logits_bf16_bf16, true, GemmEpilogue::Logits, __bf16, false)
-
 ORDA_MID(gemm_kk_mid_logits_bf16_f32, true, GemmEpilogue::Logits, float, false)
 ORDA_MID(gemm_kmt_mid_store_bf16, false, GemmEpilogue::StoreF32, float, true)
 ORDA_MID(gemm_kmt_mid_accum_bf16, false, GemmEpilogue::AccumF32, float, true)
 #undef ORDA_MID
+
 typedef void (*GemmKernel)(GemmArgs);
 
 GemmKernel select_kernel(const GemmArgs& g, bool mid) {
@@ -2048,7 +2047,8 @@ GemmKernel select_kernel(const GemmArgs& g, bool mid) {
   if (!g.a_kmajor || g.b_kmajor) return nullptr;
   if (g.c_trans)
     return bf ? (st ? gemm_kmt_store_bf16 : gemm_kmt_accum_bf16) : (st ? gemm_kmt_store_f32 : gemm_kmt_accum_f32);
-  return bf ? (st ? gemm_km_store_bf16 : gemm_km_accum_bf16) : (st ? gemm_km_store_f32 : gemm_km_accum_f32);
+  if (!st) return nullptr;
+  return bf ? gemm_km_store_bf16 : gemm_km_store_f32;
 }
 
 // Split-K reduction: C = alpha * (Σ_s partial_s) (+ alpha * C when
@@ -2270,9 +2270,9 @@ void set_band_blocks(GemmArgs& g) {
 // round of them takes kRoundUs for filling the ring and storing a tile, and
 // stage_us for every 32 elements of K (measured over bf16 products of 64 to
 // 2000 rows, widths of 256 to 4096 and vocabularies of 8000 to 128256: 0.7 us a
-// stage, 9 % off; six plane products a stage; the fp32 MFMA a sixteenth of the
-// bf16 rate). Split over K, a product also writes and reads its partials
-// (kPartUs a byte, 4 TB/s).
+// stage, 9 % off; six plane products 4.2, and at their 265 TFLOP/s of large
+// calls 4.05; the fp32 MFMA 7.3, 147 TFLOP/s). Split over K, a product also
+// writes and reads its partials (kPartUs a byte, 4 TB/s).
 constexpr double kRoundUs = 8.0, kPartUs = 0.25e-6;
 double stage_us(const GemmArgs& g) { return g.plane_a > 0 ? 4.2 : g.in_type == DType::BF16 ? 0.7 : 7.3; }
 double rounds_us(const GemmArgs& g, int64_t tiles, int64_t len) {
@@ -2351,18 +2351,19 @@ int64_t small_tiles(const GemmArgs& g) {
 bool small_f32(const GemmArgs& g) {
   if (g.in_type != DType::F32 || !g.a_kmajor || g.split_k > 1 || g.M <= 0 || g.N <= 0) return false;
   if (g.epi != GemmEpilogue::StoreF32 && g.epi != GemmEpilogue::AccumF32) return false;
-  if (g.b_kmajor && (g.c_trans || g.epi == GemmEpilogue::AccumF32)) return false;
+  if (g.c_trans ? g.b_kmajor : g.epi == GemmEpilogue::AccumF32) return false;
   const int64_t tiles = ((g.M + kTile - 1) / kTile) * ((g.N + kTile - 1) / kTile) * g.nprob;
   return tiles <= 64;
 }
 
 // The small kernel's split of K, over its 128 x 128 tiles: the split of least
-// cost as in plan_split (2.4 us for every 32 elements of K, 6 us a round),
-// each part at least 128 elements. (Parts of at least 256, and as many as fill
-// 256 workgroups: Tied 64 x 256 x 2048 134 us a call against 117, Precomputed
-// 300 x 300 x 5000 193 against 167, Tied 300 x 768 x 3000 284 against 260, 256 x
-// 512 x 8192 the same; two workgroups a CU, 512 in all, were slower there, 253
-// against 223; all before the kernel's present loads.)
+// cost as in plan_split (2.4 us for every 32 elements of K, 6 us a round: 44 us
+// for the 16 stages that measure 47 at Tied 256 x 512 x 8192), each part at
+// least 128 elements. (Parts of at least 256, and as many as fill 256
+// workgroups: Tied 64 x 256 x 2048 128 us a call against 115, Precomputed
+// 300 x 300 x 5000 172 against 160, Tied 300 x 768 x 3000 254 against 223, 256 x
+// 512 x 8192 the same. Two workgroups a CU, 512 in all, were slower there with
+// the loads as they were before, 253 against 223.)
 SplitPlan plan_split_small(const GemmArgs& g) {
   SplitPlan sp{1, g.K, 0, 0, 0, 0.0};
   if (g.K <= 0) return sp;
@@ -2637,7 +2638,6 @@ __device__ __forceinline__ void small_body(const GemmArgs& g) {
 ORDA_SMALL(gemm_kk_small_f32, true, false, false, false)
 ORDA_SMALL(gemm_kk_small_x3, true, false, false, true)
 ORDA_SMALL(gemm_km_small_x3, false, false, false, true)
-ORDA_SMALL(gemm_km_small_accum_x3, false, false, true, true)
 ORDA_SMALL(gemm_kmt_small_x3, false, true, false, true)
 ORDA_SMALL(gemm_kmt_small_accum_x3, false, true, true, true)
 #undef ORDA_SMALL
@@ -2648,9 +2648,9 @@ ORDA_SMALL(gemm_kmt_small_accum_x3, false, true, true, true)
 hipError_t launch_small(const GemmArgs& g, hipStream_t stream) {
   using K = void (*)(GemmArgs);
   auto pick = [&](bool bk, bool ct, bool acc) -> K {
-    if (bk) return acc ? nullptr : g.fp32_mfma ? gemm_kk_small_f32 : gemm_kk_small_x3;
     if (ct) return acc ? gemm_kmt_small_accum_x3 : gemm_kmt_small_x3;
-    return acc ? gemm_km_small_accum_x3 : gemm_km_small_x3;
+    if (acc) return nullptr;
+    return !bk ? gemm_km_small_x3 : g.fp32_mfma ? gemm_kk_small_f32 : gemm_kk_small_x3;
   };
   const int64_t tiles = small_tiles(g);
   const SplitPlan sp = plan_split_small(g);
