@@ -604,7 +604,9 @@ bool use_planes3(const LossPlan& P) {
 // rms at H=4096), which the INT8 scales of grad_W's unlabelled rows show as up
 // to 1.2e-5 relative, and those are held to 1e-5 of an fp32 product's
 // (tests/test_gpu_full_size.py). Accumulated in the same order the two differ
-// by 5e-6; over planes, though nearer to float64, by 1.5e-5.
+// by 5e-6; over planes, though nearer to float64, by 1.5e-5. Calls without INT8
+// keep to it too: an INT8 call quantizes the very gradient, bit for bit, that
+// the same call gives without INT8 (check_quant_of_own_gradient, tests/parity.py).
 bool fp32_logits(const LossPlan& P) { return P.need_teacher && P.mode == ORDA_TEACHER_TIED; }
 bool planes3_logits(const LossPlan& P) { return P.planes3 && !fp32_logits(P); }
 
