@@ -610,9 +610,9 @@ bool use_planes3(const LossPlan& P) {
 bool fp32_logits(const LossPlan& P) { return P.need_teacher && P.mode == ORDA_TEACHER_TIED; }
 bool planes3_logits(const LossPlan& P) { return P.planes3 && !fp32_logits(P); }
 
-// Whether the three-plane kernels reach every row of an operand's tile: its
-// rows lie 32 bits of bytes apart, 6 bytes an element (the fp32 MFMA's 4), in
-// groups of `rows`. 256 rows of one K each reach V = 2.8e6.
+// Whether the three-plane kernels reach every row of an operand's tile, in
+// groups of `rows`: a row's offset from its tile's first is 32 bits of bytes, 6
+// bytes an element (on the fp32 MFMA 4), so that 256 rows reach V = 2.8e6.
 bool planes3_reach(const LossPlan& P, int64_t rows) {
   const bool t_rows = P.need_teacher && P.mode != ORDA_TEACHER_PRECOMPUTED;
   const int64_t ht = t_rows ? P.ht : 0, k = P.mode == ORDA_TEACHER_TIED && P.w_t > 0.f ? 2 * rows : rows;
